@@ -629,12 +629,14 @@ int launch_attention(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads
 int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, int n_kv, int max_seq,
                              const MixIn &mix, const float *q_norm, const float *k_norm, const float *inv_freq,
                              const uint32_t *pos, __half *k_cache, __half *v_cache, size_t cache_off, float *part,
-                             const Planes &xp) {
+                             float *out, const Planes &xp) {
     hipLaunchKernelGGL(attn_append_kernel, dim3(n_kv, rows), dim3(64), 0, stream, mix, k_norm, inv_freq, pos, k_cache,
                        v_cache, cache_off, max_seq, n_heads, n_kv);
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-    return attention_impl(ctx, stream, rows, n_heads, n_kv, max_seq, mix, q_norm, k_norm, inv_freq, pos, k_cache,
-                          v_cache, part, nullptr, xp, cache_off, 0, false);
+    if (int rc = attention_impl(ctx, stream, rows, n_heads, n_kv, max_seq, mix, q_norm, k_norm, inv_freq, pos, k_cache,
+                                v_cache, part, out, xp.uniform ? Planes{} : xp, cache_off, 0, false))
+        return rc;
+    return xp.uniform ? launch_split_rows(ctx, stream, out, (uint32_t)rows, (uint32_t)(n_heads * kHd), xp) : ANEHIP_OK;
 }
 
 }  // namespace anehip

@@ -265,6 +265,12 @@ struct Planes {
     float *rs = nullptr;
     int rs_parts = 0;
     float rs_eps = 0.0f;
+    // One exponent per row: writers give all of a row's groups the exponent
+    // of the row's largest |x|, as the chunk GEMM (gemm_chunk) needs.  (hi +
+    // lo then hold x to 2^-22 relative down to 2^-17 of the row's largest
+    // value, and to 2^-39 of that below -- what a GEMM that brings the
+    // groups of a row to one exponent is left with.)
+    bool uniform = false;
     // the planes of rows 32 g .. 32 g + 31 for an n-column input
     __host__ __device__ Planes group(int g, int n) const {
         Planes p;
@@ -274,6 +280,7 @@ struct Planes {
         p.rs = rs ? rs + (size_t)g * 32 * rs_parts : nullptr;
         p.rs_parts = rs_parts;
         p.rs_eps = rs_eps;
+        p.uniform = uniform;
         return p;
     }
     Planes without_scale() const {
@@ -418,13 +425,20 @@ int gemm_packed_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t b
 // split_stride: floats between the K splits' outputs (0: batch * m).
 int launch_gemm_packed(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *wp, uint32_t m,
                        uint32_t n, const Planes &xp, uint32_t batch, float *out, int ksplit, size_t split_stride = 0);
-// The same for up to 256 rows: above 32 (the prefill's chunks) one gemm_tall
-// launch over the 32-row groups of the planes (Planes::group), writing
-// out[ks][row][r] with a split stride of rows * m; ksplit from
-// gemm_rows_ksplit.
+// The same for any number of rows (gemm_chunk.hip): above 32 one gemm_chunk
+// launch over the 32-row groups of the planes (Planes::group, which must be
+// uniform), writing out[ks][row][r] with a split stride of rows * m; ksplit
+// from gemm_rows_ksplit.
 int gemm_rows_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t rows);
 int launch_gemm_rows(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *wp, uint32_t m, uint32_t n,
                      const Planes &xp, uint32_t rows, float *out, int ksplit);
+// The FFN's gate / up product of more than 32 rows in one K split
+// (interleaved [gate; up] panel matrix, m = 2 F) with the SiLU-mul in its
+// epilogue: h[row][f] as fp32 rows [rows][F].
+int launch_gemm_rows_silu(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *wp, uint32_t m,
+                          uint32_t n, const Planes &xp, uint32_t rows, float *h);
+// x [rows][n] fp32 -> uniform fragment-order planes.
+int launch_split_rows(anehip_ctx *ctx, hipStream_t stream, const float *x, uint32_t rows, uint32_t n, const Planes &xp);
 // Whether gemm_packed_ksplit's split of [m x n] at this batch runs on an
 // x-stationary kernel, which can also take x as fp32 rows [batch][n] (no
 // planes needed): launch_gemm_xs_rows writes out[ks][b][r] for its
@@ -536,11 +550,12 @@ int launch_attention(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads
 // Prefill of `rows` consecutive tokens of one sequence (row t at position
 // pos[t], q / k / v in mix row t): appends every row's k / v to the cache at
 // cache_off (halves; the sequence's [kv_head][max_seq][256] block), then
-// attends row t over positions [0, pos[t]] and writes fragment-order planes.
+// attends row t over positions [0, pos[t]] and writes fragment-order planes
+// (uniform ones by way of out, [rows][n_heads * 256] fp32).
 int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, int n_kv, int max_seq,
                              const MixIn &mix, const float *q_norm, const float *k_norm, const float *inv_freq,
                              const uint32_t *pos, __half *k_cache, __half *v_cache, size_t cache_off, float *part,
-                             const Planes &xp);
+                             float *out, const Planes &xp);
 
 // elementwise.hip
 int launch_rmsnorm(anehip_ctx *ctx, hipStream_t s, int rows, int n, const float *x, const float *w, float *out,

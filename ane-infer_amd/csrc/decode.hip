@@ -67,7 +67,7 @@ struct Layer {
 
 // Tokens per prefill chunk: the rows of the chunk's GEMMs (launched per
 // 32-row group) and of its element-wise, DeltaNet and attention kernels.
-constexpr uint32_t kPrefillRows = 256;
+constexpr uint32_t kPrefillRows = 960;
 constexpr uint32_t kPrefillGroups = kPrefillRows / 32;
 
 struct Model {
@@ -107,6 +107,7 @@ struct Model {
     // (allocated by the first anehip_prefill; rows = tokens)
     struct {
         float *x = nullptr, *xn = nullptr, *pmix = nullptr, *p0 = nullptr, *p1 = nullptr, *attn_part = nullptr;
+        float *attn_out = nullptr;
         float *logits = nullptr;
         _Float16 *xin = nullptr;  // planes: hi then lo, xin_len halves each, then xe_cnt exponents
         uint32_t *d_tokens = nullptr, *d_pos = nullptr;
@@ -170,7 +171,7 @@ void free_state(Model *M) {
                     M->p1,    M->heads,    M->attn_out,  M->logits, M->attn_part, M->argmax_ws, M->xin, M->dn_pend,
                     M->norm_ss};
     for (void *p : bufs) free_ptr(p);
-    void *pfb[] = {M->pf.x, M->pf.xn, M->pf.pmix, M->pf.p0, M->pf.p1, M->pf.attn_part, M->pf.logits, M->pf.xin,
+    void *pfb[] = {M->pf.x, M->pf.xn, M->pf.pmix, M->pf.p0, M->pf.p1, M->pf.attn_part, M->pf.attn_out, M->pf.logits, M->pf.xin,
                    M->pf.d_tokens, M->pf.d_pos};
     for (void *p : pfb) free_ptr(p);
     M->pf = {};
@@ -654,9 +655,7 @@ int pack_weights(anehip_ctx *ctx, Model *M) {
 
 
 // K-split partial floats of the prefill's GEMMs at up to kPrefillRows rows
-// (the split depends on the rows only through rows <= 16, <= 32, or the
-// number of 128-row blocks above 32), of the
-// batch-1 lm_head GEMV, and the DeltaNet scan's per-token inputs (q, k, v,
+// (below 16 rows the split is that of 16), of the batch-1 lm_head GEMV, and the DeltaNet scan's per-token inputs (q, k, v,
 // beta, decay; kept in the ffn partial buffer, which is free at that point).
 size_t prefill_part_floats(anehip_ctx *ctx, Model *M) {
     const anehip_model_desc &D = M->desc;
@@ -664,9 +663,10 @@ size_t prefill_part_floats(anehip_ctx *ctx, Model *M) {
     const uint32_t g[][2] = {{M->rows_dn, d}, {M->rows_attn, d}, {d, d}, {d, D.n_heads * D.head_dim}, {2 * F, d}, {d, F}};
     size_t mx = (size_t)gemv_packed_ksplit(ctx, D.vocab_size, d) * D.vocab_size;
     mx = std::max(mx, (size_t)kPrefillRows * (3 * d + 2 * D.ssm_group_count));
+    mx = std::max(mx, (size_t)kPrefillRows * F);  // SiLU(gate) * up as fp32 rows
     for (auto &e : g)
-        for (uint32_t rows : {16u, 32u, kPrefillRows})  // the split depends on rows <= 16, <= 32 or above
-            if (e[0]) mx = std::max(mx, (size_t)gemm_rows_ksplit(ctx, e[0], e[1], rows) * rows * e[0]);
+        for (uint32_t rows = 16; e[0] && rows <= kPrefillRows; rows++)
+            mx = std::max(mx, (size_t)gemm_rows_ksplit(ctx, e[0], e[1], rows) * rows * e[0]);
     return mx;
 }
 
@@ -686,7 +686,9 @@ int alloc_prefill(anehip_ctx *ctx, Model *M) {
         size_t bytes;
     } a[] = {{(void **)&M->pf.x, kPrefillRows * d * 4}, {(void **)&M->pf.xn, kPrefillRows * d * 4},
              {(void **)&M->pf.pmix, part * 4}, {(void **)&M->pf.p0, part * 4}, {(void **)&M->pf.p1, part * 4},
-             {(void **)&M->pf.attn_part, std::max<size_t>(attn, 1) * 4}, {(void **)&M->pf.logits, (size_t)D.vocab_size * 4},
+             {(void **)&M->pf.attn_part, std::max<size_t>(attn, 1) * 4},
+             {(void **)&M->pf.attn_out, std::max<size_t>((size_t)kPrefillRows * D.n_heads * D.head_dim, 1) * 4},
+             {(void **)&M->pf.logits, (size_t)D.vocab_size * 4},
              {(void **)&M->pf.xin, M->pf_planes_bytes()}, {(void **)&M->pf.d_tokens, kPrefillRows * 4},
              {(void **)&M->pf.d_pos, kPrefillRows * 4}};
     for (auto &e : a) {
@@ -709,7 +711,8 @@ int enqueue_prefill_chunk(anehip_ctx *ctx, Model *M, hipStream_t s, uint32_t seq
     const anehip_model_desc &D = M->desc;
     const uint32_t d = D.dim, F = D.hidden_dim, H = D.ssm_group_count, C = 3 * d;
     const float eps = D.rms_norm_eps;
-    const Planes xp = M->pf_planes();
+    Planes xp = M->pf_planes();
+    xp.uniform = T > 32;  // the chunk GEMM's input
     float *x = M->pf.x;
     TRY(launch_embed_rmsnorm(ctx, s, T, (int)d, M->pf.d_tokens, M->embedding, D.vocab_size, x,
                              M->layers[0].attn_norm, nullptr, eps, xp));
@@ -735,15 +738,23 @@ int enqueue_prefill_chunk(anehip_ctx *ctx, Model *M, hipStream_t s, uint32_t seq
             const size_t cache_off = (size_t)seq * D.n_kv_heads * M->max_seq * D.head_dim;
             TRY(launch_attention_prefill(ctx, s, T, (int)D.n_heads, (int)D.n_kv_heads, (int)M->max_seq, mix, L.q_norm,
                                          L.k_norm, M->inv_freq, M->pf.d_pos, L.kc, L.vc, cache_off, M->pf.attn_part,
-                                         xp));
+                                         M->pf.attn_out, xp));
             cols3 = D.n_heads * D.head_dim;
         }
         const int k3 = gemm_rows_ksplit(ctx, d, cols3, T);
         TRY(launch_gemm_rows(ctx, s, L.mix_out.type, L.mix_out.p, d, cols3, xp, T, M->pf.p0, k3));
         TRY(launch_residual_rmsnorm(ctx, s, T, (int)d, x, M->pf.p0, k3, L.post_attn_norm, nullptr, eps, xp));
         const int k4 = gemm_rows_ksplit(ctx, 2 * F, d, T);
-        TRY(launch_gemm_rows(ctx, s, L.ffn_gu.type, L.ffn_gu.p, 2 * F, d, xp, T, M->pf.p1, k4));
-        TRY(launch_silu_mul_stacked(ctx, s, T, (int)F, M->pf.p1, k4, nullptr, xp));
+        if (T > 32 && k4 == 1) {
+            // SiLU-mul in the product's epilogue, then the rows split for the down product
+            TRY(launch_gemm_rows_silu(ctx, s, L.ffn_gu.type, L.ffn_gu.p, 2 * F, d, xp, T, M->pf.p1));
+            TRY(launch_split_rows(ctx, s, M->pf.p1, T, F, xp));
+        } else {
+            TRY(launch_gemm_rows(ctx, s, L.ffn_gu.type, L.ffn_gu.p, 2 * F, d, xp, T, M->pf.p1, k4));
+            TRY(launch_silu_mul_stacked(ctx, s, T, (int)F, M->pf.p1, k4, xp.uniform ? M->pf.pmix : nullptr,
+                                        xp.uniform ? Planes{} : xp));
+            if (xp.uniform) TRY(launch_split_rows(ctx, s, M->pf.pmix, T, F, xp));
+        }
         const int k5 = gemm_rows_ksplit(ctx, d, F, T);
         TRY(launch_gemm_rows(ctx, s, L.ffn_down.type, L.ffn_down.p, d, F, xp, T, M->pf.p0, k5));
         if (l + 1 < D.n_layers)

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(kThreads) void dn_prep_kernel(MixIn mix, MixIn mbet
 // consecutive lanes.  Raw head outputs go to out[t][chunk].
 constexpr int kScanCols = 4;
 constexpr int kScanMaxT = 32;    // tokens staged in LDS at a time
-constexpr int kScanMaxRows = 256;  // tokens per launch
+constexpr int kScanMaxRows = 1024;  // tokens per launch
 constexpr int kDropOffset = 0x7ffffff0;  // buffer offset past any output: the store is dropped
 
 // sum over each 16-lane row: row_ror 8, 4, 2, 1
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(kWave) void deltanet_scan_kernel(const float *__res
 // kKsize values of (old window, the T inputs).  grid = (n_heads, T), 128 threads.
 template <int KP>
 __global__ __launch_bounds__(kDk) void dn_scan_finish_kernel(MixIn mix, float *__restrict__ conv_state,
-                                                             const float *__restrict__ heads, int gate_off,
+                                                             float *__restrict__ heads, int gate_off,
                                                              const float *__restrict__ norm_w, Planes xp,
                                                              int n_heads, float eps, int T) {
     __shared__ float red[2], mred[2];
@@ -640,7 +640,8 @@ __global__ __launch_bounds__(kDk) void dn_scan_finish_kernel(MixIn mix, float *_
     __syncthreads();
     const float inv_rms = 1.0f / sqrtf((red[0] + red[1]) / (float)kDk + eps);
     const float v = ((x * inv_rms) * norm_w[t]) * gs;
-    head_to_planes(v, b, h * kDk, chunk, group_exp(fmaxf(mred[0], mred[1]) * inv_rms), xp);
+    if (xp.uniform) heads[(size_t)b * chunk + h * kDk + t] = v;  // the row's exponent needs every head: split after
+    else head_to_planes(v, b, h * kDk, chunk, group_exp(fmaxf(mred[0], mred[1]) * inv_rms), xp);
 }
 
 }  // namespace
@@ -670,6 +671,7 @@ int launch_deltanet_scan(anehip_ctx *ctx, hipStream_t stream, int rows, int n_he
     }
 #undef DN_SCAN
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
+    if (xp.uniform) return launch_split_rows(ctx, stream, heads, (uint32_t)rows, (uint32_t)(n_heads * kDk), xp);
     return ANEHIP_OK;
 }
 

@@ -50,11 +50,11 @@ __device__ __forceinline__ void rmsnorm_row(const float *x, const float *__restr
         return;
     }
     for (int i = threadIdx.x; i < n; i += kThreads)
-        atomicMax(&gmax[i / kXeGroup], __float_as_int(fabsf((x[i] * inv_rms) * w[i])));
+        atomicMax(&gmax[xp.uniform ? 0 : i / kXeGroup], __float_as_int(fabsf((x[i] * inv_rms) * w[i])));
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += kThreads) {
         const float v = (x[i] * inv_rms) * w[i];
-        const int e = group_exp(__int_as_float(gmax[i / kXeGroup]));
+        const int e = group_exp(__int_as_float(gmax[xp.uniform ? 0 : i / kXeGroup]));
         split_scaled(v, e, xp.hi[xf_index(brow, i, n)], xp.lo[xf_index(brow, i, n)]);
         if (i % kXeGroup == 0) xp.xe[xe_index(brow, i, n)] = (int8_t)e;
     }
@@ -112,7 +112,7 @@ template <int KP>
 __global__ __launch_bounds__(512) void residual_rmsnorm_v4(float *__restrict__ x, const float *__restrict__ part,
                                                            int ksplit, int rows, const float *__restrict__ w,
                                                            float *__restrict__ xn, int n, float eps, Planes xp) {
-    __shared__ float red[8];
+    __shared__ float red[8], rmax[8];
     const int t = threadIdx.x;
     const size_t b = blockIdx.x;
     const int n4 = n >> 2, e4 = min(t, n4 - 1);
@@ -144,11 +144,19 @@ __global__ __launch_bounds__(512) void residual_rmsnorm_v4(float *__restrict__ x
     // threads of one wave, all inside the row or all outside: n % 128 == 0),
     // taken while the sum of squares crosses the barrier; times inv_rms it
     // gives the group's binade (to a few ulps)
-    const float gmax = xp.hi ? half_max32(mine ? fmaxf(fmaxf(fabsf(r.x * wv.x), fabsf(r.y * wv.y)),
-                                                      fmaxf(fabsf(r.z * wv.z), fabsf(r.w * wv.w)))
-                                               : 0.0f)
-                             : 0.0f;
+    float gmax = xp.hi ? half_max32(mine ? fmaxf(fmaxf(fabsf(r.x * wv.x), fabsf(r.y * wv.y)),
+                                                 fmaxf(fabsf(r.z * wv.z), fabsf(r.w * wv.w)))
+                                         : 0.0f)
+                       : 0.0f;
+    if (xp.uniform) {
+        gmax = lanes_max2(gmax);  // of the wave; the row's from the 8 waves' below
+        if ((t & 63) == 0) rmax[t >> 6] = gmax;
+    }
     __syncthreads();
+    if (xp.uniform) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) gmax = fmaxf(gmax, rmax[i]);
+    }
     float tot = red[0];
 #pragma unroll
     for (int i = 1; i < 8; i++) tot += red[i];

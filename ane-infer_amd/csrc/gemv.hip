@@ -20,14 +20,12 @@
 //     fill the chip, K is split across workgroups, which write partial sums
 //     to a workspace; a second pass adds them in fixed order, so results are
 //     deterministic and no device-wide fence is needed.
-#include "common.h"
+#include "panel.h"
 
 namespace anehip {
 
 namespace {
 
-constexpr int kWave = 64;
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <uint32_t T> struct QTraits;
 template <> struct QTraits<ANEHIP_GGML_Q8_0> {
@@ -589,16 +587,6 @@ __global__ __launch_bounds__(512) void gemv_fused_xs(const uint8_t *__restrict__
 // own row's 256 weights and scales, with no LDS transposition.  Panels of a
 // tile are consecutive; rows past m are zero.
 // ---------------------------------------------------------------------------
-
-template <uint32_t T> struct Panel;
-template <> struct Panel<ANEHIP_GGML_Q8_0> {
-    static constexpr int kChunks = 16;
-    static constexpr int kBytes = 17 * 1024;
-};
-template <> struct Panel<ANEHIP_GGML_Q4_0> {
-    static constexpr int kChunks = 8;
-    static constexpr int kBytes = 9 * 1024;
-};
 
 // The GGUF row behind panel row `row`: the identity, or (il = F > 0, a
 // stacked [gate (F rows); up (F rows)] matrix) gate rows 32 t .. 32 t + 31 in
@@ -1392,8 +1380,6 @@ __global__ __launch_bounds__(kWave *rows_waves(H)) void gemv_rows(const uint8_t 
 // acc += C * d (q8_gemv.rs:234-242 order within a block up to fp32 summation).
 // ---------------------------------------------------------------------------
 
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-
 // Range-safe planes on the GEMM side (see Planes): the largest exponent of
 // groups [g0, g0 + ng) of batch row b.
 // The row's exponents are read as dwords (a row starts 16-byte aligned, its
@@ -1459,13 +1445,10 @@ __device__ __forceinline__ void split8_scaled(const float (&v)[8], int E, h8v &h
 }
 
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kGemmWaves = 4;
 constexpr int kGemmRing = 2;  // panel GEMM: units in flight per wave
-// word 3 of a raw buffer resource on gfx9-family parts (data format 32 bit)
-constexpr int kBufferWord3 = 0x00020000;
 
 // Four signed int8 (one dword) -> four fp16, exact.
 __device__ __forceinline__ void i8x4_to_h(uint32_t d, _Float16 *o) {
@@ -1515,14 +1498,6 @@ __device__ __forceinline__ void swap_halves(uint32_t &a0, uint32_t &a1, uint32_t
     b0 = s0[1];
     a1 = s1[0];
     b1 = s1[1];
-}
-
-// Barrier for LDS traffic only: the fences order LDS accesses, so waves do
-// not wait for their outstanding global loads (the prefetched units) here.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // One wave's operands for one panel of its TV tiles: per tile the quant
@@ -1637,10 +1612,6 @@ constexpr int kBadOffset = 0x7ffffff0;  // buffer offset past any output: the st
 // kernel reads once, this measured 2 % faster over a batch-32 decode step
 // (non-temporal stores: 2 % slower).
 constexpr int kCpolDevice = 16;
-// Cache-policy bit nt for streamed weight loads through buffer resources (the
-// other kernels use __builtin_nontemporal_load): prefill of 2048 tokens
-// 48.6 -> 47.9-48.1 ms.
-constexpr int kCpolNtLoad = 2;
 
 template <int CPOL = 0>
 __device__ __forceinline__ void gemm_tile_epilogue(float (*red)[32][kWave], const float (&fEb)[2], const f32x16 &acc0,
@@ -2448,250 +2419,6 @@ __global__ __launch_bounds__(kWave *kGemmWaves *H) __attribute__((amdgpu_waves_p
             }
         }
     } while (ct < tiles);
-}
-
-// Prefill GEMM: up to 256 rows of x (compute wave w takes rows 32 w .. 32 w +
-// 31, that group's 32-row planes) against 64-row weight tiles.  Items are
-// (tile, K split); one workgroup per CU walks the panels ("units") of items
-// g, g + G, ... as one pipeline.  Per unit:
-//  * a ninth wave (the loader) loaded the panel's bytes into registers a unit
-//    ahead and turned them into MFMA B fragments of the quantised values q as
-//    fp16 (exact: |q| <= 127) in LDS, with each weight row's fp16 block
-//    scales d beside them (the compute waves then wait on nothing but their
-//    own x loads, which come from L2: a load waits for every load its wave
-//    issued before it, so panel loads of their own would hold up the next x
-//    wait for an HBM round trip);
-//  * each wave multiplies its rows' x fragments (hi + lo at x 2^-E, E the
-//    row's largest group exponent) with them on v_mfma_f32_32x32x16_f16,
-//    one 32-column block at a time: c = x_hi q + x_lo q over the block's two
-//    16-column steps, then sums += c d, the block's (sum q x) d of
-//    q8_gemv.rs:234-242 (x_lo q is exact in the MFMA's fp32 products; x_hi +
-//    x_lo holds x to 2^-22);
-//  * an item's sums go out, times 2^E, after its last unit.
-// out[ks * split_stride + row * m + r] (rows past `rows` or m: not stored).
-constexpr int kTallWaves = 8;
-constexpr int kTallMaxRows = 32 * kTallWaves;
-
-// 8 signed bytes q (Q8_0) as fp16 q, exactly: q + 128 placed in the
-// mantissa of 1024 (fp16 0x64xx is 1024 + xx), minus 1152
-__device__ __forceinline__ h8v q8_fragment(uint32_t w0, uint32_t w1) {
-    const uint32_t u0 = w0 ^ 0x80808080u, u1 = w1 ^ 0x80808080u;
-    const u32x4 p = {__builtin_amdgcn_perm(0x64646464u, u0, 0x04010400u),
-                     __builtin_amdgcn_perm(0x64646464u, u0, 0x04030402u),
-                     __builtin_amdgcn_perm(0x64646464u, u1, 0x04010400u),
-                     __builtin_amdgcn_perm(0x64646464u, u1, 0x04030402u)};
-    const h8v k = {1152, 1152, 1152, 1152, 1152, 1152, 1152, 1152};
-    return __builtin_bit_cast(h8v, p) - k;
-}
-// 8 nibbles (Q4_0: the low, shift 0, or high, shift 4, nibbles of 8 bytes)
-// as fp16 nibble - 8, exactly (1024 + nibble, minus 1032)
-__device__ __forceinline__ h8v q4_fragment(uint32_t w0, uint32_t w1, int shift) {
-    const uint32_t n0 = (w0 >> shift) & 0x0f0f0f0fu, n1 = (w1 >> shift) & 0x0f0f0f0fu;
-    const u32x4 p = {__builtin_amdgcn_perm(0x64646464u, n0, 0x04010400u),
-                     __builtin_amdgcn_perm(0x64646464u, n0, 0x04030402u),
-                     __builtin_amdgcn_perm(0x64646464u, n1, 0x04010400u),
-                     __builtin_amdgcn_perm(0x64646464u, n1, 0x04030402u)};
-    const h8v k = {1032, 1032, 1032, 1032, 1032, 1032, 1032, 1032};
-    return __builtin_bit_cast(h8v, p) - k;
-}
-
-template <uint32_t T>
-__global__ __launch_bounds__(kWave *(kTallWaves + 1)) __attribute__((amdgpu_waves_per_eu(3, 3))) void gemm_tall(
-    const uint8_t *__restrict__ Wp, Planes xp, float *__restrict__ out, int m, int n, int rows, int ksplit, int per,
-    size_t split_stride) {
-    constexpr int CH = Panel<T>::kChunks;  // quant chunks of a tile's panel
-    __shared__ h8v wf[2][16][2][kWave];    // B fragments [unit parity][16-column step][weight block][lane]
-    __shared__ u32x4 dsc[2][kWave];        // 8 fp16 block scales of each weight row [unit parity][row]
-    __shared__ uint16_t xes[2][kTallMaxRows];  // the panel's two group exponents of each x row [unit parity][row]
-    __shared__ int erow[kTallWaves][32];
-    const int nsb = n >> 8, ptiles = (m + kWave - 1) / kWave;
-    const int items = ptiles * ksplit, G = (int)gridDim.x;
-    // this workgroup's units: the panels of items g, g + G, ... in order
-    const int units = ((items - (int)blockIdx.x + G - 1) / G) * per;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    auto item_of = [&](int u) { return (int)blockIdx.x + G * (u / per); };
-    auto panel_of = [&](int u) { return (item_of(u) % ksplit) * per + u % per; };
-    if (units == 0) return;
-
-    if (wave == kTallWaves) {
-        // The loader wave: unit u's panel bytes (lane l: chunk c of weight row
-        // l for every c, row l's scale vector, and the two group exponents of
-        // x rows l, l + 64, l + 128, l + 192 (the last row past the rows); a
-        // tile past the matrix reads the last one again: its rows are never
-        // stored) into registers, then into the B fragments of q as fp16 of
-        // the unit's parity.  Its loads are the only ones it waits on, so
-        // each has a whole unit to arrive.  Buffer loads: the offset within a
-        // panel per lane, the panel's offset wave-uniform.
-        const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint8_t *>(Wp), 0, (int)((size_t)ptiles * nsb * Panel<T>::kBytes), kBufferWord3);
-        const __amdgpu_buffer_rsrc_t xersrc =
-            __builtin_amdgcn_make_buffer_rsrc(xp.xe, 0, rows * xe_stride(n), kBufferWord3);
-        u32x4 rq[CH], rs;
-        uint32_t rxe[kTallMaxRows / kWave];
-        auto load_raw = [&](int u) {
-            const int tile = min(item_of(u) / ksplit, ptiles - 1), p = panel_of(u);
-            const int base = (tile * nsb + p) * Panel<T>::kBytes;
-#pragma unroll
-            for (int c = 0; c < CH; c++)
-                rq[c] = __builtin_bit_cast(
-                    u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, 16 * (c * kWave + lane), base, kCpolNtLoad));
-            rs = __builtin_bit_cast(
-                u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, 16 * (CH * kWave + lane), base, kCpolNtLoad));
-#pragma unroll
-            for (int i = 0; i < kTallMaxRows / kWave; i++)
-                rxe[i] = __builtin_amdgcn_raw_buffer_load_b16(xersrc, min(lane + kWave * i, rows - 1) * xe_stride(n),
-                                                              2 * p, 0);
-        };
-        // Q8_0 chunk c holds a row's columns 16 c .. + 15 (step c); Q4_0
-        // chunk c its block c, byte i the columns 32 c + i (low nibble, step
-        // 2 c) and 32 c + 16 + i (high, step 2 c + 1).  Lane l of a step's
-        // fragment: weight row l % 32 of the block, columns 8 (l / 32) .. + 7
-        // of the step.
-        auto convert = [&](int b) {
-            const int cb = lane / 32, l = lane % 32;
-#pragma unroll
-            for (int c = 0; c < CH; c++) {
-                const u32x4 q = rq[c];
-                if constexpr (T == ANEHIP_GGML_Q8_0) {
-                    wf[b][c][cb][l] = q8_fragment(q.x, q.y);
-                    wf[b][c][cb][l + 32] = q8_fragment(q.z, q.w);
-                } else {
-                    wf[b][2 * c][cb][l] = q4_fragment(q.x, q.y, 0);
-                    wf[b][2 * c][cb][l + 32] = q4_fragment(q.z, q.w, 0);
-                    wf[b][2 * c + 1][cb][l] = q4_fragment(q.x, q.y, 4);
-                    wf[b][2 * c + 1][cb][l + 32] = q4_fragment(q.z, q.w, 4);
-                }
-                __builtin_amdgcn_sched_barrier(0);  // one chunk's fragments at a time
-            }
-            dsc[b][lane] = rs;
-#pragma unroll
-            for (int i = 0; i < kTallMaxRows / kWave; i++) xes[b][lane + kWave * i] = (uint16_t)rxe[i];
-        };
-        load_raw(0);
-        convert(0);
-        load_raw(1);
-        __syncthreads();  // unit 0's fragments ready
-        for (int u = 0; u < units; u++) {
-            // unit u + 1 into the parity unit u - 1 read (past the last unit:
-            // not read), then the loads of unit u + 2
-            convert((u + 1) & 1);
-            load_raw(u + 2);
-            __syncthreads();  // end of unit u
-        }
-        return;
-    }
-
-    // The compute waves: wave w takes x rows 32 w .. + 31
-    const int grows = rows - 32 * wave;  // rows of this wave's group (<= 0: products not stored)
-    const bool active = grows > 0;
-    const Planes gp = xp.group(active ? wave : 0, n);
-    const int brow = min(lane & 31, (active ? min(grows, 32) : 1) - 1);  // rows past the group repeat its last
-    const int8_t *xe_row = gp.xe + (size_t)brow * xe_stride(n);
-    // block j of panel p (steps 16 p + 2 j, + 1): hi and lo fragments
-    // (buffer loads: the lane's offset in a step's 1 KiB, the step's offset
-    // wave-uniform)
-    const int plane_bytes = (int)(2 * xf_plane_len((size_t)n));
-    const __amdgpu_buffer_rsrc_t hrsrc = __builtin_amdgcn_make_buffer_rsrc(gp.hi, 0, plane_bytes, kBufferWord3);
-    const __amdgpu_buffer_rsrc_t lrsrc = __builtin_amdgcn_make_buffer_rsrc(gp.lo, 0, plane_bytes, kBufferWord3);
-    const int xoff = 16 * (brow + 32 * (lane >> 5));
-    auto load_x = [&](int p, int j, h8v (&a)[4]) {
-        const int so = (16 * p + 2 * j) * 1024;
-        a[0] = __builtin_bit_cast(h8v, __builtin_amdgcn_raw_buffer_load_b128(hrsrc, xoff, so, 0));
-        a[1] = __builtin_bit_cast(h8v, __builtin_amdgcn_raw_buffer_load_b128(lrsrc, xoff, so, 0));
-        a[2] = __builtin_bit_cast(h8v, __builtin_amdgcn_raw_buffer_load_b128(hrsrc, xoff, so + 1024, 0));
-        a[3] = __builtin_bit_cast(h8v, __builtin_amdgcn_raw_buffer_load_b128(lrsrc, xoff, so + 1024, 0));
-    };
-    f32x16 acc[2] = {f32x16{}, f32x16{}};
-    // an item's sums: element r of lane l is row 8 (r / 4) + 4 (l / 32) +
-    // r % 4 of the group, weight row 32 cb + l % 32 of the tile
-    auto store_item = [&](int item) {
-        const int tile = item / ksplit, ks = item % ksplit;
-        // opaque copies: the row addresses and scales are rebuilt here, not
-        // kept live across the unit loop
-        float *ob = out;
-        int w = wave, ln = lane;
-        asm volatile("" : "+s"(ob), "+s"(w), "+v"(ln));
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int gr = 8 * (r >> 2) + 4 * (ln >> 5) + (r & 3);
-            if (gr < grows) {
-                const float sc = xe_scale(erow[w][gr]);
-                float *orow = ob + (size_t)ks * split_stride + (size_t)(32 * w + gr) * m;
-#pragma unroll
-                for (int cb = 0; cb < 2; cb++) {
-                    const int wr = tile * kWave + 32 * cb + (ln & 31);
-                    if (wr < m) orow[wr] = acc[cb][r] * sc;
-                }
-            }
-        }
-        acc[0] = f32x16{};
-        acc[1] = f32x16{};
-    };
-    // E over the whole row (one exponent for every K split of it), from
-    // 16-byte loads of the row's exponents (a row's are padded to 16 bytes),
-    // all issued before the first is used
-    int E = kXeEmpty;
-    {
-        const int ng = 2 * nsb;
-        u32x4 ev[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (16 * i < ng) ev[i] = *reinterpret_cast<const u32x4 *>(xe_row + 16 * i);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int k = 0; k < 16; k++)
-                if (16 * i + k < ng) E = max(E, (int)(int8_t)(ev[i][k >> 2] >> (8 * (k & 3))));
-        for (int g = 64; g < ng; g++) E = max(E, (int)xe_row[g]);  // n > 8192
-    }
-    if (lane < 32) erow[wave][lane] = E;
-    __syncthreads();  // unit 0's fragments ready, erow written
-    // x of the next two blocks is always in flight: xa[i % 4] for block i
-    // of the workgroup's sequence of units x 8 blocks.  Every wave issues
-    // the same loads and products on every unit (waves without rows take
-    // group 0's x and store nothing; past the last unit, a valid panel), so
-    // that the loop has one path and the loads in flight are the same on it.
-    h8v xa[4][4];
-    load_x(panel_of(0), 0, xa[0]);
-    load_x(panel_of(0), 1, xa[1]);
-    for (int u0 = 0; u0 < units; u0 += per) {
-    for (int u = u0; u < u0 + per; u++) {
-        const int b = u & 1, p = panel_of(u);
-        const uint32_t xe2 = xes[b][32 * wave + brow];
-        const _Float16 fg[2] = {xe_factor((int)(int8_t)(xe2 & 0xffu), E), xe_factor((int)(int8_t)(xe2 >> 8), E)};
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const _Float16 f = fg[j >> 2];
-            h8v(&a)[4] = xa[j % 4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) a[i] *= f;
-            // then x of the block two ahead (the next unit's first two)
-            __builtin_amdgcn_sched_barrier(0);
-            if (j < 6) load_x(p, j + 2, xa[(j + 2) % 4]);
-            else load_x(panel_of(u + 1), j - 6, xa[(j + 2) % 4]);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int cb = 0; cb < 2; cb++) {
-                const h8v b0 = wf[b][2 * j][cb][lane], b1 = wf[b][2 * j + 1][cb][lane];
-                f32x16 c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], b0, f32x16{}, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], b0, c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[2], b1, c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[3], b1, c, 0, 0, 0);
-                const uint32_t dw = reinterpret_cast<const uint32_t *>(&dsc[b][32 * cb + (lane & 31)])[j >> 1];
-                const float d = __half2float(__ushort_as_half((unsigned short)(dw >> (16 * (j & 1)))));
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[cb][r] = fmaf(c[r], d, acc[cb][r]);
-                // the sums are added here, not deferred (which would keep
-                // every block's products live)
-                asm volatile("" : "+v"(acc[cb]));
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __syncthreads();  // end of unit u: unit u + 1's fragments ready; every wave is done with parity b
-    }
-    if (active) store_item(item_of(u0));
-    }
 }
 
 // fp32 x[batch][n] -> range-safe fragment-order fp16 planes (hi + lo = x *
@@ -3606,64 +3333,6 @@ int launch_gemm_packed(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, 
         launch_gemm_packed_t<ANEHIP_GGML_Q8_0>(ctx, stream, w, m, n, xp, batch, out, ksplit, per, ss);
     else
         launch_gemm_packed_t<ANEHIP_GGML_Q4_0>(ctx, stream, w, m, n, xp, batch, out, ksplit, per, ss);
-    ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-    return ANEHIP_OK;
-}
-
-// K split of gemm_tall (one tile per item: two tiles per item measured 9.6 us
-// per unit against 4.6 us for one, no gain per row): a divisor of the panel count (at most 16, the partial slices
-// a consumer sums) minimising an estimate of the busiest CU's time,
-// ceil(items / CUs) x panels per split x the measured time of one unit at 256
-// rows (4.6 us on MI355X), plus the traffic of the extra partial slices
-// (written here, read by the consumer: 2 x 4 bytes per row and output, at
-// 256 rows ~2 KiB per output, at ~5 TB/s).
-static int gemm_tall_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n) {
-    const int ptiles = (int)((m + kWave - 1) / kWave);
-    const int nsb = (int)(n / 256), cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const double unit_us = 4.6, part_us_per_row = 2048.0 / 5.0e6;
-    int best = 1;
-    double best_cost = -1.0;
-    for (int k = 1; k <= nsb && k <= 16; k++) {
-        if (nsb % k) continue;
-        const double cost =
-            (double)((ptiles * k + cus - 1) / cus) * (nsb / k) * unit_us + (k - 1) * (double)m * part_us_per_row;
-        if (best_cost < 0.0 || cost < best_cost) {
-            best_cost = cost;
-            best = k;
-        }
-    }
-    return best;
-}
-
-int gemm_rows_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t rows) {
-    return rows <= 32 ? gemm_packed_ksplit(ctx, m, n, rows) : gemm_tall_ksplit(ctx, m, n);
-}
-
-int launch_gemm_rows(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *wp, uint32_t m, uint32_t n,
-                     const Planes &xp, uint32_t rows, float *out, int ksplit) {
-    if (rows <= 32) return launch_gemm_packed(ctx, stream, ggml_type, wp, m, n, xp, rows, out, ksplit);
-    const int nsb = (int)(n / 256), ptiles = (int)((m + kWave - 1) / kWave);
-    if (rows > kTallMaxRows || ksplit < 1 || nsb % ksplit || m % 4 || !xp.hi || !xp.lo || !xp.xe)
-        return set_error(ctx->err, ANEHIP_EINVAL, "gemm_rows: %u rows (at most %d), K split %d of %d panels, m %u",
-                         rows, kTallMaxRows, ksplit, nsb, m);
-    if (4.0 * ksplit * rows * m > 1073741824.0)
-        return set_error(ctx->err, ANEHIP_ESHAPE, "gemm_rows: output of %d x %u x %u floats too large", ksplit, rows, m);
-    // gemm_tall addresses the weights with 32-bit buffer offsets
-    if ((double)ptiles * nsb * Panel<ANEHIP_GGML_Q8_0>::kBytes > 2147483647.0)
-        return set_error(ctx->err, ANEHIP_ESHAPE, "gemm_rows: %u x %u weights too large (2 GiB of panels at most)", m, n);
-    const int items = ptiles * ksplit;
-    // one workgroup per CU, each walking its items' panels in one pipeline
-    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const dim3 grid((unsigned)std::min(items, cus)), block(kWave * (kTallWaves + 1));
-    const uint8_t *w = static_cast<const uint8_t *>(wp);
-    const int per = nsb / ksplit;
-    const size_t ss = (size_t)rows * m;
-    if (ggml_type == ANEHIP_GGML_Q8_0)
-        hipLaunchKernelGGL(gemm_tall<ANEHIP_GGML_Q8_0>, grid, block, 0, stream, w, xp, out, (int)m, (int)n,
-                           (int)rows, ksplit, per, ss);
-    else
-        hipLaunchKernelGGL(gemm_tall<ANEHIP_GGML_Q4_0>, grid, block, 0, stream, w, xp, out, (int)m, (int)n,
-                           (int)rows, ksplit, per, ss);
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
     return ANEHIP_OK;
 }

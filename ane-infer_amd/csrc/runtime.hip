@@ -270,7 +270,10 @@ int anehip_quant_gemm_packed(anehip_ctx *ctx, uint32_t ggml_type, const void *wp
     xp.hi = reinterpret_cast<_Float16 *>(ctx->ws.partial);
     xp.lo = xp.hi + xcount;
     xp.xe = reinterpret_cast<int8_t *>(xp.lo + xcount);
-    if ((rc = launch_split_x(ctx, ctx->stream, x, batch, n, xp))) return rc;
+    xp.uniform = batch > 32;  // the chunk GEMM's planes
+    if ((rc = xp.uniform ? launch_split_rows(ctx, ctx->stream, x, batch, n, xp)
+                         : launch_split_x(ctx, ctx->stream, x, batch, n, xp)))
+        return rc;
     if (ksplit == 1) return launch_gemm_rows(ctx, ctx->stream, ggml_type, wp, m, n, xp, batch, y, 1);
     float *part = ctx->ws.partial + planes;
     if ((rc = launch_gemm_rows(ctx, ctx->stream, ggml_type, wp, m, n, xp, batch, part, ksplit))) return rc;

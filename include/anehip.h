@@ -202,7 +202,7 @@ int anehip_quant_gemv_packed(anehip_ctx *ctx, uint32_t ggml_type, const void *wp
  * the panel copy wp; x [batch][n] fp32.  batch 1 is
  * anehip_quant_gemv_packed; batch > 1 runs on MFMA (the small-batch form of
  * anehip_quant_gemm, same tolerance; above 32 the GEMM anehip_prefill runs
- * its chunks of up to 256 tokens on) and needs m % 4 == 0
+ * its chunks on) and needs m % 4 == 0
  * (ANEHIP_EUNSUPPORTED otherwise); above 32 rows the panels must stay
  * under 2 GiB (ANEHIP_ESHAPE otherwise). */
 int anehip_quant_gemm_packed(anehip_ctx *ctx, uint32_t ggml_type, const void *wp, uint32_t m, uint32_t n,
@@ -357,7 +357,7 @@ int anehip_decode_step_async(anehip_ctx *ctx, const uint32_t *token_ids, uint32_
 
 /*
  * Prefill: tokens[n_tokens] of sequence `seq`, from its current position, in
- * chunks of up to 32 tokens -- the projections on the MFMA GEMM with one row
+ * chunks of up to 960 tokens -- the projections on the MFMA GEMM with one row
  * per token, the DeltaNet recurrence as a scan over each chunk's tokens with
  * the state held on chip, attention causal within the chunk.  Leaves the
  * sequence's state and position as n_tokens decode steps would (the other

@@ -515,9 +515,7 @@ def test_ragged_positions_across_chunk_boundaries(mid_host):
 @pytest.mark.parametrize("n", [100, 300, 600])
 def test_prefill_long_prompt_large_cache(mid_host, n):
     """anehip_prefill into a 2048-position cache of a 100-token prompt (one
-    chunk on the chunk GEMM at 100 rows), a 300-token one (chunks of 256 and
-    44) and a 600-token one (256, 256, 88: the second full chunk replays the
-    graph the first captured; the DeltaNet scan runs 256 tokens per launch);
+    chunk on the chunk GEMM at 100 rows), a 300-token and a 600-token one;
     chunk rows see up to 10 live tiles of attention; the last logits, states
     and KV rows vs the oracle run token by token, then 2 decode steps."""
     spec = mid_host.spec
@@ -537,12 +535,33 @@ def test_prefill_long_prompt_large_cache(mid_host, n):
     oseq.close()
 
 
+@pytest.mark.parametrize("n", [961, 1950])
+def test_prefill_full_chunks(mid_host, n):
+    """Prompts past one chunk of 960 tokens: 961 (a full chunk, then one row on
+    the decode GEMMs) and 1950 (two full chunks, the second replaying the graph
+    the first captured, then 30 rows), vs the oracle run token by token."""
+    spec = mid_host.spec
+    gm = _model(mid_host, 1, 2048)
+    oseq = mid_host.seq(2048)
+    toks = oracle.randint(35, n, n, spec.vocab_size)
+    g = gm.prefill(0, toks)
+    for i, t in enumerate(toks):
+        r = oseq.forward(int(t))
+        if i % 512 == 511:
+            print(f"prefill {n}: oracle at token {i + 1}", flush=True)
+    l2, mx = rel_errs(g, r)
+    print(f"prefill n={n}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
+    assert l2 <= TOL and mx <= TOL
+    _check_state(gm, oseq, 0, spec, "after prefill")
+    assert max(rel_errs(gm.step([int(toks[0])])[0], oseq.forward(int(toks[0])))) <= TOL
+    gm.close()
+    oseq.close()
+
+
 @pytest.mark.parametrize("n", [40, 300])
 def test_qwen35_2b_shape_prefill(big_host, n):
-    """Random-init 24-layer Qwen3.5-2B shape: a 40-token prompt (one chunk) and
-    a 300-token one (a full 256-token chunk, recorded as the prefill's chunk
-    graph and replayed for it, then 44 rows) prefilled from position 0 vs the
-    oracle run token by token: the last logits, every layer's DeltaNet state,
+    """Random-init 24-layer Qwen3.5-2B shape: a 40-token and a 300-token prompt
+    (one chunk each) prefilled from position 0 vs the oracle run token by token: the last logits, every layer's DeltaNet state,
     conv window and KV rows, then one decode step continuing the sequence."""
     spec = big_host.spec
     gm = _model(big_host, 1, 512)

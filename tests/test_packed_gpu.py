@@ -175,13 +175,12 @@ def test_packed_gemm_parity(gpu_ctx, oracle_lib, t, batch, m, n):
 @pytest.mark.parametrize("m,n", [(6144, 2048), (2048, 6144), (8224, 2048), (2048, 2048), (12288, 1792), (100, 256),
                                  (32968, 256)])
 def test_packed_gemm_tall(gpu_ctx, oracle_lib, t, batch, m, n):
-    """More than 32 rows (the prefill's chunk GEMM, gemm_tall): 32-row groups
-    of planes, one per compute wave (33: one full group and one row, six
-    waves without rows; 100 and 256: partial and full), a ragged last weight
-    tile (8224 rows; 100 rows: two tiles, the second ragged), K splits that
-    divide the panel count (12288 x 1792: 7 panels; 2048 x 2048: 8 splits),
-    and workgroups walking several items (32968 x 256: 516 one-panel items,
-    2 or 3 per workgroup, the last tile ragged)."""
+    """More than 32 rows (the prefill's chunk GEMM, gemm_chunk): 32-row groups
+    of planes, two per workgroup (33: one full group and one row; 100 and 256:
+    partial and full), a ragged last weight tile (8224 rows; 100 rows: two
+    tiles, the second ragged), K splits that divide the panel count (12288 x
+    1792: 7 panels; 2048 x 2048) and many weight blocks (32968 x 256: 129
+    blocks of one panel, the last tile ragged)."""
     w = oracle_lib.gen_quant(t, 77, m + 3 * n + t, m, n, std=0.02)
     x = oracle_lib.normal(77, 900 + batch, batch * n).reshape(batch, n)
     dw, dp, _ = _pack(gpu_ctx, t, w, m, n)
@@ -190,6 +189,30 @@ def test_packed_gemm_tall(gpu_ctx, oracle_lib, t, batch, m, n):
     y = dy.download(np.float32, batch * m).reshape(batch, m)
     ref = oracle_lib.gemm(t, w, m, n, x)
     l2, mx = rel_errs(y, ref)
+    print(f"type={t} m={m} n={n} batch={batch}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
+    assert l2 <= TOL and mx <= TOL
+    for b in (dw, dp, dx, dy):
+        b.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", [8, 2])
+@pytest.mark.parametrize("m,n,batch", [(64, 256, 33), (260, 512, 64), (516, 768, 65), (256, 4096, 96), (2056, 2304, 129),
+                                       (1028, 8448, 250)])
+def test_packed_gemm_chunk_edges(gpu_ctx, oracle_lib, t, m, n, batch):
+    """gemm_chunk at the edges of its tiles: 256 weight rows x 64 x rows per
+    workgroup (one tile of four; a block whose last wave has 4 rows; a block
+    exactly full; one wave of the last block), exactly full and one-row row
+    blocks, one and an odd number of panels (the K halves meet inside a
+    panel), K splits of 3 and more, and rows wider than split_rows_kernel
+    holds in registers (8448 columns)."""
+    w = oracle_lib.gen_quant(t, 78, m + 3 * n + t, m, n, std=0.02)
+    x = oracle_lib.normal(78, 900 + batch, batch * n).reshape(batch, n)
+    dw, dp, _ = _pack(gpu_ctx, t, w, m, n)
+    dx, dy = gpu_ctx.to_device(x), gpu_ctx.alloc(batch * m * 4)
+    gpu_ctx.call("quant_gemm_packed", t, dp, m, n, dx, batch, dy)
+    y = dy.download(np.float32, batch * m).reshape(batch, m)
+    l2, mx = rel_errs(y, oracle_lib.gemm(t, w, m, n, x))
     print(f"type={t} m={m} n={n} batch={batch}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
     assert l2 <= TOL and mx <= TOL
     for b in (dw, dp, dx, dy):
@@ -279,7 +302,7 @@ def test_packed_gemm_input_range(gpu_ctx, oracle_lib, t, batch, m, n):
     fp16's range (overflow, underflow, subnormal, zero, mixed groups) match
     the fp32 oracle, on the x-stationary kernels (fp32 rows, per-row scaling
     over the split), on the persistent kernel (range-safe planes) and above
-    32 rows on gemm_tall (range-safe planes, per-row scaling over the split)."""
+    32 rows on gemm_chunk (planes of one exponent per row)."""
     w = oracle_lib.gen_quant(t, 55, m + n + t, m, n, std=0.02)
     x = extreme_rows(oracle_lib, batch, n, 500 + batch)
     dw, dp, _ = _pack(gpu_ctx, t, w, m, n)
