@@ -518,13 +518,15 @@ int launch_deltanet_head(anehip_ctx *ctx, hipStream_t stream, int batch, int n_h
                          const MixIn &beta, const MixIn &alpha, const float *conv_w, const float *ssm_a,
                          const float *dt_bias, float *conv_state, float *S, float *out, int gate_off,
                          const float *norm_w, float eps, const Planes &xp);
-// Prefill: `rows` (<= 32) consecutive tokens of one sequence (mix row t =
-// token t) through the DeltaNet step of every head, the state (the sequence's
-// block S) kept in registers across the rows.  Three kernels: every token's
-// normalised q, k, v, beta and decay to prep (scratch of rows * (3 * dim + 2 *
-// n_heads) floats); the recurrence, raw head outputs to heads [rows][dim]
-// (scratch); row t's gated RMSNorm to the planes and the conv windows (the
-// sequence's block conv_state) advanced by the rows.
+// Prefill: `rows` (<= 1024) consecutive tokens of one sequence (mix row t =
+// token t) through the DeltaNet step of every head, 64 tokens at a time.
+// Three kernels: per chunk and head what does not depend on the state, to
+// prep (scratch of kDnChunkFloats floats per head and 64 rows); the state (the
+// sequence's block S) carried over the chunks, raw head outputs to heads
+// [rows][dim] (scratch); row t's gated RMSNorm to the planes (uniform ones by
+// way of heads) and the conv windows (the sequence's block conv_state)
+// advanced by the rows.
+constexpr size_t kDnChunkFloats = 4 * 64 * 128 + 64 * 64 + 64;
 int launch_deltanet_scan(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, const MixIn &mix,
                          const MixIn &beta, const MixIn &alpha, const float *conv_w, const float *ssm_a,
                          const float *dt_bias, float *conv_state, float *S, float *prep, float *heads,

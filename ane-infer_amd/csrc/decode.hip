@@ -68,6 +68,7 @@ struct Layer {
 // Tokens per prefill chunk: the rows of the chunk's GEMMs (launched per
 // 32-row group) and of its element-wise, DeltaNet and attention kernels.
 constexpr uint32_t kPrefillRows = 960;
+static_assert(kPrefillRows % 64 == 0, "the DeltaNet scan and the chunk GEMM take 64 rows at a time");
 constexpr uint32_t kPrefillGroups = kPrefillRows / 32;
 
 struct Model {
@@ -655,14 +656,15 @@ int pack_weights(anehip_ctx *ctx, Model *M) {
 
 
 // K-split partial floats of the prefill's GEMMs at up to kPrefillRows rows
-// (below 16 rows the split is that of 16), of the batch-1 lm_head GEMV, and the DeltaNet scan's per-token inputs (q, k, v,
-// beta, decay; kept in the ffn partial buffer, which is free at that point).
+// (below 16 rows the split is that of 16), of the batch-1 lm_head GEMV, and the DeltaNet
+// chunks' state-independent parts (kept in the ffn partial buffer, which is
+// free at that point).
 size_t prefill_part_floats(anehip_ctx *ctx, Model *M) {
     const anehip_model_desc &D = M->desc;
     const uint32_t d = D.dim, F = D.hidden_dim;
     const uint32_t g[][2] = {{M->rows_dn, d}, {M->rows_attn, d}, {d, d}, {d, D.n_heads * D.head_dim}, {2 * F, d}, {d, F}};
     size_t mx = (size_t)gemv_packed_ksplit(ctx, D.vocab_size, d) * D.vocab_size;
-    mx = std::max(mx, (size_t)kPrefillRows * (3 * d + 2 * D.ssm_group_count));
+    mx = std::max(mx, (size_t)(kPrefillRows / 64) * D.ssm_group_count * kDnChunkFloats);
     mx = std::max(mx, (size_t)kPrefillRows * F);  // SiLU(gate) * up as fp32 rows
     for (auto &e : g)
         for (uint32_t rows = 16; e[0] && rows <= kPrefillRows; rows++)

@@ -19,7 +19,7 @@
 // which is the reference's per-head order (decay, recall, delta, rank-1
 // update, query) with the three global passes of the Metal kernel fused into
 // one read and one write of the 64 KiB head state.
-#include "common.h"
+#include "panel.h"
 
 namespace anehip {
 
@@ -29,7 +29,6 @@ constexpr int kDk = 128;     // key dim == value dim (ssm_state_size)
 constexpr int kCols = 32;    // value columns per workgroup
 constexpr int kThreads = 256;
 constexpr int kKsize = 4;    // conv width (ssm_conv_kernel)
-constexpr int kWave = 64;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -421,176 +420,378 @@ __global__ __launch_bounds__(kThreads) void deltanet_head_kernel(
     head_to_planes(v, b, h * kDk, chunk, group_exp(fmaxf(mred[0], mred[1]) * inv_rms), xp);
 }
 
-// Prefill: T consecutive tokens of one sequence (mix row t = token t), in
-// three kernels.  Only the state is recurrent: the conv over time, the q / k
-// L2 norms, v, beta and the decay of every token are independent, so
-// dn_prep_kernel forms them for all (token, head) pairs at once; the scan then
-// runs the recurrence alone; dn_scan_finish_kernel applies the gated RMSNorm
+// Prefill: T consecutive tokens of one sequence (mix row t = token t), 64 at
+// a time.  With g_t the product of a chunk's decays up to token t and D_ts =
+// decay_{s+1} ... decay_t, the recurrence of deltanet.rs:485-512 over a chunk
+// that starts from S0 is
+//   delta_t = beta_t (v_t - g_t S0^T k_t - sum_{s<t} D_ts (k_s . k_t) delta_s)
+//   o_t     = g_t S0^T q_t + sum_{s<=t} D_ts (k_s . q_t) delta_s
+//   S       = g_63 S0 + sum_s D_63,s k_s delta_s^T
+// i.e. with L_ts = beta_t D_ts k_s . k_t (s < t), X = (I + L)^-1 (lower
+// triangular, unit diagonal), A_ts = D_ts q_t . k_s (s <= t):
+//   U = X (beta V),  W = X (beta g K)     (dn_chunk_kernel, all chunks at once)
+//   Delta = U - W S0,  O = (g Q) S0 + A Delta,  S = g_63 S0 + (D_63 K)^T Delta
+// (dn_scan_kernel, chunk after chunk).  All products run on
+// v_mfma_f32_16x16x4_f32 in fp32; the decays enter as products of at most 64
+// factors <= 1, never as quotients, so nothing under- or overflows that the
+// token-by-token order keeps.  dn_scan_finish_kernel applies the gated RMSNorm
 // and commits the conv windows.
+//
+// What bounds it: the scan is serial in the chunks, 112 MFMAs of 32 cycles
+// per wave and chunk (1.5 us) plus two barriers; a token-by-token scan pays a
+// chain of LDS reads, FMAs and lane sums of 0.14 us per token (9 us per 64).
+constexpr int kCt = 64;               // tokens per chunk
+constexpr int kRowF = kDk + 4;        // LDS row of a [64][128] matrix: 16-byte reads of 16 rows hit all banks
+constexpr int kTriF = kCt + 4;        // LDS row of a [64][64] matrix
+constexpr int kScanMaxRows = 1024;    // tokens per launch
+// floats that dn_chunk_kernel leaves per (chunk, head): U, W, g Q [64][128]
+// each, (D_63 K)^T [128][64], A [64][64], g_63
+constexpr int kOffW = kCt * kDk, kOffQ = 2 * kCt * kDk, kOffK = 3 * kCt * kDk, kOffA = 4 * kCt * kDk,
+              kOffG = kOffA + kCt * kCt;
+static_assert(kOffG + 64 == kDnChunkFloats, "scratch of a chunk");
 
-// Token b's conv taps for channel ch: the last kKsize values of (the old
-// window, the inputs of tokens 0..b) (conv_shift_and_append + conv_apply,
-// deltanet_cache.rs:34-54), then SiLU.
-template <int KP>
-__device__ __forceinline__ float conv_token(const MixIn &mix, const float *__restrict__ cs,
-                                            const float *__restrict__ conv_w, int ch, int b) {
-    const f32x4 old = *reinterpret_cast<const f32x4 *>(cs + (size_t)ch * kKsize);
-    const f32x4 wk = *reinterpret_cast<const f32x4 *>(conv_w + (size_t)ch * kKsize);
-    float xs[kKsize][KP];
+// 16 x 16 x 16 product on four v_mfma_f32_16x16x4_f32: lane l holds, of A, row
+// l % 16 and columns 4 (l / 16) .. + 3 (a); of B, column l % 16 and rows
+// 4 (l / 16) .. + 3 (b) -- one k order for both -- and of the result column
+// l % 16, rows 4 (l / 16) .. + 3: a result is the next product's B as it is.
+__device__ __forceinline__ f32x4 mma16(f32x4 a, f32x4 b, f32x4 c) {
 #pragma unroll
-    for (int i = 0; i < kKsize; i++) mix.load<KP>(max(b - kKsize + 1 + i, 0), ch, xs[i]);
-    const float ov[kKsize] = {old.x, old.y, old.z, old.w};
-    const float kw[kKsize] = {wk.x, wk.y, wk.z, wk.w};
-    float sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kKsize; i++) {
-        const int src = b - kKsize + 1 + i;  // < 0: from the old window
-        sum += (src >= 0 ? mix.add<KP>(xs[i]) : ov[(kKsize + src) & (kKsize - 1)]) * kw[i];
-    }
-    return silu_ref(sum);
+    for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+    return c;
 }
 
-// grid = (n_heads, T), 256 threads: thread t forms channel t % 128 of q (t <
-// 128) or k, normalised (deltanet.rs:25-31, 461-467), and threads t < 128 also
-// v channel t; thread 0 the token's beta and decay (deltanet.rs:474-480).
-// prep[(b * n_heads + h) * 384 + {0, 128, 256} + c] = q, k, v; bd[(b * n_heads
-// + h) * 2 + {0, 1}] = beta, decay.
+// grid = (chunks of 64 tokens, n_heads), 256 threads.  Conv + SiLU over the
+// tokens' windows (conv_shift_and_append + conv_apply, deltanet_cache.rs:34-54),
+// L2 norms of q and k (deltanet.rs:25-31, 461-467), beta and decay
+// (deltanet.rs:474-480), then the products above.  Tokens past T have k = q =
+// v = 0, beta 0 and decay 1: they change nothing.
 template <int KP>
-__global__ __launch_bounds__(kThreads) void dn_prep_kernel(MixIn mix, MixIn mbeta, MixIn malpha,
-                                                           const float *__restrict__ conv_w,
-                                                           const float *__restrict__ ssm_a,
-                                                           const float *__restrict__ dt_bias,
-                                                           const float *__restrict__ cs, float *__restrict__ prep,
-                                                           float *__restrict__ bd, int n_heads) {
-    __shared__ float red[4];
-    const int t = threadIdx.x, h = blockIdx.x, b = blockIdx.y;
-    const int chunk = n_heads * kDk, e = t & (kDk - 1);
-    const float y = conv_token<KP>(mix, cs, conv_w, t < kDk ? h * kDk + t : chunk + h * kDk + e, b);
-    const float vy = t < kDk ? conv_token<KP>(mix, cs, conv_w, 2 * chunk + h * kDk + t, b) : 0.0f;
-    const float sq = wave_sum(y * y);
-    if ((t & 63) == 0) red[t >> 6] = sq;
-    __syncthreads();
-    float *out = prep + ((size_t)b * n_heads + h) * 3 * kDk;
-    if (t < kDk) {
-        const float inv = 1.0f / sqrtf((red[0] + red[1]) + 1e-12f);
-        out[t] = (y * inv) * (1.0f / sqrtf((float)kDk));
-        out[2 * kDk + t] = vy;
-    } else {
-        out[kDk + e] = y * (1.0f / sqrtf((red[2] + red[3]) + 1e-12f));
+__global__ __launch_bounds__(kThreads) void dn_chunk_kernel(MixIn mix, MixIn mbeta, MixIn malpha,
+                                                            const float *__restrict__ conv_w,
+                                                            const float *__restrict__ ssm_a,
+                                                            const float *__restrict__ dt_bias,
+                                                            const float *__restrict__ cs, float *__restrict__ scr,
+                                                            int n_heads, int T) {
+    __shared__ __align__(16) float qkv[3][kCt * kRowF];
+    __shared__ __align__(16) float tri[2][kCt * kTriF];  // D, then X; L
+    __shared__ float sb[kCt], sg[kCt], sd[kCt];          // beta, g, D_63
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, lg = lane >> 4;
+    const int c0 = blockIdx.x * kCt, h = blockIdx.y, chunk = n_heads * kDk;
+    float *out = scr + ((size_t)blockIdx.x * n_heads + h) * kDnChunkFloats;
+    float *Q = qkv[0], *K = qkv[1], *V = qkv[2];
+
+    // conv: thread (channel t % 128, token half t / 128) walks its 32 tokens
+    // of q, k and v with the window in registers, 8 loads in flight
+    const int ch = t & (kDk - 1), b0 = c0 + (t >> 7) * (kCt / 2);
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        const int gch = p * chunk + h * kDk + ch;
+        const f32x4 old = *reinterpret_cast<const f32x4 *>(cs + (size_t)gch * kKsize);
+        const f32x4 kw = *reinterpret_cast<const f32x4 *>(conv_w + (size_t)gch * kKsize);
+        float w[3][KP], x[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) mix.load<KP>(min(max(b0 - 3 + i, 0), T - 1), gch, w[i]);
+#pragma unroll
+        for (int i = 0; i < 3; i++) x[i] = b0 - 3 + i >= 0 ? mix.add<KP>(w[i]) : old[(b0 + 1 + i) & 3];
+        for (int i0 = 0; i0 < kCt / 2; i0 += 8) {
+            float v[8][KP];
+#pragma unroll
+            for (int i = 0; i < 8; i++) mix.load<KP>(min(b0 + i0 + i, T - 1), gch, v[i]);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float xn = mix.add<KP>(v[i]);
+                float y = 0.0f;
+                y += x[0] * kw.x;
+                y += x[1] * kw.y;
+                y += x[2] * kw.z;
+                y += xn * kw.w;
+                qkv[p][(b0 - c0 + i0 + i) * kRowF + ch] = b0 + i0 + i < T ? silu_ref(y) : 0.0f;
+                x[0] = x[1];
+                x[1] = x[2];
+                x[2] = xn;
+            }
+        }
     }
-    if (t == 0) {
+    if (wave == 0) {
+        // lane = token: beta, decay; then column s = lane of D
+        const int b = min(c0 + lane, T - 1);
         float xb[KP], xa[KP];
         mbeta.load<KP>(b, h, xb);
         malpha.load<KP>(b, h, xa);
-        float *o = bd + ((size_t)b * n_heads + h) * 2;
-        o[0] = 1.0f / (1.0f + expf(-mbeta.add<KP>(xb)));
-        o[1] = expf(ssm_a[h] * logf(1.0f + expf(malpha.add<KP>(xa) + dt_bias[h])));
-    }
-}
-
-// The recurrence is independent per value column j (recall sk_j, delta_j,
-// column j of the rank-1 update and the query o_j), so a head is split over
-// kDk / C single-wave workgroups of C columns each, grid = (kDk / C, n_heads).
-// The workgroup copies its head's q and k, its columns' v and the tokens' beta
-// and decay into LDS, kScanMaxT tokens at a time; the token loop then has no
-// global load.  Lane l holds rows R (l % G) .. + R - 1 of column C g + l / G (G =
-// 64 / C lanes per column, R = 128 / G rows per lane) in registers across all
-// T steps (state read and written once per chunk); a sum over rows is 4
-// interleaved partial sums of R / 4 rows, then a DPP sum over the column's G
-// consecutive lanes.  Raw head outputs go to out[t][chunk].
-constexpr int kScanCols = 4;
-constexpr int kScanMaxT = 32;    // tokens staged in LDS at a time
-constexpr int kScanMaxRows = 1024;  // tokens per launch
-constexpr int kDropOffset = 0x7ffffff0;  // buffer offset past any output: the store is dropped
-
-// sum over each 16-lane row: row_ror 8, 4, 2, 1
-__device__ __forceinline__ float sum16(float v) {
-    return dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(v))));
-}
-
-template <int C>
-__global__ __launch_bounds__(kWave) void deltanet_scan_kernel(const float *__restrict__ prep,
-                                                              const float *__restrict__ bd, float *__restrict__ S,
-                                                              float *__restrict__ out, int n_heads, int T) {
-    constexpr int G = kWave / C, R = kDk / G;
-    static_assert(G == 8 || G == 16, "a column's lanes are summed within one DPP row");
-    static_assert(C % 2 == 0 && C + 2 <= kWave, "lanes C, C + 1 carry beta and decay");
-    __shared__ __align__(16) float qks[kScanMaxT][2 * kDk];  // q then k of each token
-    __shared__ float exs[kScanMaxT][kWave];  // lanes 0..C-1: v of the columns, C, C+1: beta, decay
-    const int l = threadIdx.x, h = blockIdx.y;
-    const int chunk = n_heads * kDk;
-    const int rgp = l % G, jl = l / G, j = blockIdx.x * C + jl;
-    float *Sh = S + (size_t)h * kDk * kDk + j;
-    float st[R];
+        const bool in = c0 + lane < T;
+        const float alpha = in ? expf(ssm_a[h] * logf(1.0f + expf(malpha.add<KP>(xa) + dt_bias[h]))) : 1.0f;
+        sb[lane] = in ? 1.0f / (1.0f + expf(-mbeta.add<KP>(xb))) : 0.0f;
+        const int ai = __builtin_bit_cast(int, alpha);
+        const float a0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, 0));
+        float p = 1.0f;
 #pragma unroll
-    for (int r = 0; r < R; r++) st[r] = Sh[(size_t)(R * rgp + r) * kDk];
-    const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, 4 * T * chunk, 0x00020000);
-    const auto colsum = [](float v) { return G == 16 ? sum16(v) : sum8(v); };
-    // the tokens in sub-chunks of kScanMaxT, the state in registers throughout
-    for (int c0 = 0; c0 < T; c0 += kScanMaxT) {
-        if (c0) __syncthreads();  // the previous sub-chunk's reads of qks / exs are done
-        // all loads of a half of the sub-chunk in flight at once (clamped to
-        // the last token; slots past T are never read): lane l copies float4 l
-        // of q | k, lanes 0..C-1 also v of column l, lanes >= C beta (even) /
-        // decay (odd)
-#pragma unroll
-        for (int b0 = 0; b0 < kScanMaxT; b0 += kScanMaxT / 2) {
-            float4 qk[kScanMaxT / 2];
-            float ex[kScanMaxT / 2];
-#pragma unroll
-            for (int i = 0; i < kScanMaxT / 2; i++) {
-                const int b = min(c0 + b0 + i, T - 1);
-                const float *src = prep + ((size_t)b * n_heads + h) * 3 * kDk;
-                qk[i] = reinterpret_cast<const float4 *>(src)[l];
-                ex[i] = l < C ? src[2 * kDk + blockIdx.x * C + l] : bd[((size_t)b * n_heads + h) * 2 + (l & 1)];
-            }
-#pragma unroll
-            for (int i = 0; i < kScanMaxT / 2; i++) {
-                reinterpret_cast<float4 *>(qks[b0 + i])[l] = qk[i];
-                exs[b0 + i][l] = ex[i];
-            }
+        for (int i = 0; i < kCt; i++) {
+            const float a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, i));
+            p = i > lane ? p * a : 1.0f;
+            tri[0][i * kTriF + lane] = i >= lane ? p : 0.0f;
+            if (lane == 0) sg[i] = a0 * p;
         }
+        sd[lane] = p;
+    }
+    __syncthreads();
+    // L2 norms: 16 lanes per token, 8 columns each, 4 tokens of a wave at a time
+#pragma unroll
+    for (int it = 0; it < 4; it++) {
+        const int o = (16 * wave + 4 * it + lg) * kRowF + 8 * li;
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            f32x4 *r = reinterpret_cast<f32x4 *>(&qkv[p][o]);
+            f32x4 a = r[0], c = r[1];
+            float ss = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) ss += a[e] * a[e] + c[e] * c[e];
+            const float inv = 1.0f / sqrtf(row_sum16(ss) + 1e-12f), f = p == 0 ? 1.0f / sqrtf((float)kDk) : 1.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                a[e] = (a[e] * inv) * f;
+                c[e] = (c[e] * inv) * f;
+            }
+            r[0] = a;
+            r[1] = c;
+        }
+    }
+    __syncthreads();
+    // the 10 lower 16 x 16 tiles of K K^T (-> L, LDS) and of Q K^T (-> A), 5 per wave
+    auto tile_of = [](int p, int &i, int &j) {
+        i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3;
+        j = p - i * (i + 1) / 2;
+    };
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+        const int p = wave + 4 * n;
+        const bool kk = p < 10;
+        int i, j;
+        tile_of(kk ? p : p - 10, i, j);
+        const float *ra = (kk ? K : Q) + (16 * i + li) * kRowF + 4 * lg, *rb = K + (16 * j + li) * kRowF + 4 * lg;
+        f32x4 s0 = {}, s1 = {};
+#pragma unroll
+        for (int q = 0; q < 8; q += 2) {
+            s0 = mma16(*reinterpret_cast<const f32x4 *>(ra + 16 * q), *reinterpret_cast<const f32x4 *>(rb + 16 * q), s0);
+            s1 = mma16(*reinterpret_cast<const f32x4 *>(ra + 16 * q + 16),
+                       *reinterpret_cast<const f32x4 *>(rb + 16 * q + 16), s1);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int r = 16 * i + 4 * lg + e, c = 16 * j + li;
+            const float v = (s0[e] + s1[e]) * tri[0][r * kTriF + c];
+            if (kk) tri[1][r * kTriF + c] = c < r ? sb[r] * v : 0.0f;
+            else out[kOffA + r * kCt + c] = c <= r ? v : 0.0f;
+        }
+    }
+    // A's upper tiles are zero
+    for (int e = t; e < 6 * 64; e += kThreads) {
+        const int p = e >> 6, i = p < 3 ? 0 : p < 5 ? 1 : 2, j = p < 3 ? p + 1 : p < 5 ? p - 1 : 3;
+        *reinterpret_cast<f32x4 *>(out + kOffA + (16 * i + ((e & 63) >> 2)) * kCt + 16 * j + 4 * (e & 3)) = f32x4{};
+    }
+    // g Q and (D_63 K)^T
+    for (int e = t; e < kCt * kDk / 4; e += kThreads) {
+        const int r = e >> 5, c = 4 * (e & 31);
+        const f32x4 q = *reinterpret_cast<const f32x4 *>(Q + r * kRowF + c);
+        *reinterpret_cast<f32x4 *>(out + kOffQ + r * kDk + c) = q * sg[r];
+    }
+    for (int i = wave; i < kDk; i += 4) out[kOffK + i * kCt + lane] = sd[lane] * K[lane * kRowF + i];
+    if (t == 0) out[kOffG] = sg[kCt - 1];
+    __syncthreads();  // L is whole, D no longer needed
+    float *X = tri[0];
+    const float *L = tri[1];
+    // X's diagonal blocks by forward substitution: wave w block w, lane column
+    // s = li: x_t = [t = s] - sum_{r<t} L_tr x_r
+    {
+        float x[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            float p[4] = {r == li ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int q = 0; q < (r + 3) / 4; q++) {
+                const f32x4 lr = *reinterpret_cast<const f32x4 *>(L + (16 * wave + r) * kTriF + 16 * wave + 4 * q);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (4 * q + e < r) p[e] -= lr[e] * x[4 * q + e];
+            }
+            x[r] = (p[0] + p[1]) + (p[2] + p[3]);
+        }
+        if (lg == 0)
+#pragma unroll
+            for (int r = 0; r < 16; r++) X[(16 * wave + r) * kTriF + 16 * wave + li] = x[r];
+    }
+    // X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj, one block diagonal at a time
+    auto row4 = [&](const float *m, int i, int k) {
+        return *reinterpret_cast<const f32x4 *>(m + (16 * i + li) * kTriF + 16 * k + 4 * lg);
+    };
+    for (int d = 1; d < 4; d++) {
         __syncthreads();
-        const int te = min(kScanMaxT, T - c0);
-        for (int bb = 0; bb < te; bb++) {
-            const int b = c0 + bb;
-            const float beta = exs[bb][C], decay = exs[bb][C + 1], v = exs[bb][jl];
-            float kr[R], qr[R];
+        const int i = wave + d, j = wave;
+        if (i < 4) {
+            f32x4 p = {};
+            for (int k = j; k < i; k++) {
+                f32x4 xb;
 #pragma unroll
-            for (int r = 0; r < R; r += 4) {
-                const float4 k4 = *reinterpret_cast<const float4 *>(&qks[bb][kDk + R * rgp + r]);
-                const float4 q4 = *reinterpret_cast<const float4 *>(&qks[bb][R * rgp + r]);
-                kr[r] = k4.x, kr[r + 1] = k4.y, kr[r + 2] = k4.z, kr[r + 3] = k4.w;
-                qr[r] = q4.x, qr[r + 1] = q4.y, qr[r + 2] = q4.z, qr[r + 3] = q4.w;
+                for (int e = 0; e < 4; e++) xb[e] = X[(16 * k + 4 * lg + e) * kTriF + 16 * j + li];
+                p = mma16(row4(L, i, k), xb, p);
             }
-            // S' = decay S; sk_j = sum_i S'_ij k_i
-            float p[4] = {0.f, 0.f, 0.f, 0.f};
+            const f32x4 v = mma16(row4(X, i, i), p, f32x4{});
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                st[r] *= decay;
-                p[r & 3] += st[r] * kr[r];
-            }
-            const float sk = colsum((p[0] + p[1]) + (p[2] + p[3]));
-            const float delta = beta * (v - sk);
-            // S'' = S' + k delta^T; o_j = sum_i S''_ij q_i
-#pragma unroll
-            for (int r = 0; r < 4; r++) p[r] = 0.f;
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                st[r] += kr[r] * delta;
-                p[r & 3] += st[r] * qr[r];
-            }
-            const float o = colsum((p[0] + p[1]) + (p[2] + p[3]));
-            // lanes of row group 0 store (the others' offset is past the buffer: dropped)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), orsrc,
-                                                  rgp == 0 ? 4 * (b * chunk + h * kDk + j) : kDropOffset, 0, 0);
+            for (int e = 0; e < 4; e++) X[(16 * i + 4 * lg + e) * kTriF + 16 * j + li] = -v[e];
         }
     }
+    __syncthreads();
+    // U = X (beta V) and W = X (beta g K): 2 column tiles of each per wave
+    f32x4 xa[10];
 #pragma unroll
-    for (int r = 0; r < R; r++) Sh[(size_t)(R * rgp + r) * kDk] = st[r];
+    for (int p = 0; p < 10; p++) {
+        int i, k;
+        tile_of(p, i, k);
+        xa[p] = row4(X, i, k);
+    }
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+        const float *src = n < 2 ? V : K;
+        float *dst = out + (n < 2 ? 0 : kOffW);
+        const int c = 16 * (2 * wave + (n & 1)) + li;
+        f32x4 b[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = 16 * k + 4 * lg + e;
+                b[k][e] = src[r * kRowF + c] * (n < 2 ? sb[r] : sb[r] * sg[r]);
+            }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            f32x4 s = {};
+#pragma unroll
+            for (int k = 0; k <= i; k++) s = mma16(xa[i * (i + 1) / 2 + k], b[k], s);
+#pragma unroll
+            for (int e = 0; e < 4; e++) dst[(16 * i + 4 * lg + e) * kDk + c] = s[e];
+        }
+    }
 }
 
-// After deltanet_scan_kernel: row b of the gated RMSNorm (deltanet.rs:517-533)
+// grid = (kDk / 16, n_heads), 256 threads: 16 value columns of one head (the
+// columns of Delta, O and S are independent).  Every wave holds the state of
+// the 16 columns in registers as the B operand of a product over the key
+// dim (S0 tile j: rows 16 j + 4 (l / 16) .. + 3, column l % 16); wave w takes
+// tokens 16 w .. + 15 of Delta and O and state tiles 2 w, 2 w + 1.  Delta and
+// the new state tiles cross the waves through LDS.  A chunk's operands are
+// loaded while the chunk before it is processed.  Raw head outputs go to
+// heads[t][chunk].
+__global__ __launch_bounds__(kThreads) void dn_scan_kernel(const float *__restrict__ scr, float *__restrict__ S,
+                                                           float *__restrict__ heads, int n_heads, int T) {
+    __shared__ f32x4 dl[4][64], sl[8][64];
+    const int t = threadIdx.x, lane = t & 63, li = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int h = blockIdx.y, chunk = n_heads * kDk, col = 16 * blockIdx.x + li;
+    const int chunks = (T + kCt - 1) / kCt;
+    float *Sh = S + (size_t)h * kDk * kDk + col;
+    f32x4 st[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) st[j][e] = Sh[(size_t)(16 * j + 4 * lg + e) * kDk];
+    f32x4 w4[8], q4[8], k4[2][4], a4[4], u;
+    float g;
+    auto base = [&](int c) { return scr + ((size_t)min(c, chunks - 1) * n_heads + h) * kDnChunkFloats; };
+    auto load_w = [&](int c) {
+        const float *p = base(c);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            w4[j] = *reinterpret_cast<const f32x4 *>(p + kOffW + (16 * wave + li) * kDk + 16 * j + 4 * lg);
+#pragma unroll
+        for (int e = 0; e < 4; e++) u[e] = p[(16 * wave + 4 * lg + e) * kDk + col];
+    };
+    auto load_q = [&](int c) {
+        const float *p = base(c) + kOffQ + (16 * wave + li) * kDk + 4 * lg;
+#pragma unroll
+        for (int j = 0; j < 8; j++) q4[j] = *reinterpret_cast<const f32x4 *>(p + 16 * j);
+    };
+    auto load_k = [&](int c) {
+        const float *p = base(c);
+        g = p[kOffG];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                k4[i][j] = *reinterpret_cast<const f32x4 *>(p + kOffK + (16 * (2 * wave + i) + li) * kCt + 16 * j + 4 * lg);
+    };
+    auto load_a = [&](int c) {
+        const float *p = base(c) + kOffA + (16 * wave + li) * kCt + 4 * lg;
+#pragma unroll
+        for (int j = 0; j < 4; j++) a4[j] = *reinterpret_cast<const f32x4 *>(p + 16 * j);
+    };
+    load_w(0);
+    load_q(0);
+    load_k(0);
+    load_a(0);
+    for (int c = 0; c < chunks; c++) {
+        f32x4 s0 = {}, s1 = {};
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            s0 = mma16(w4[j], st[j], s0);
+            s1 = mma16(w4[j + 1], st[j + 1], s1);
+        }
+        dl[wave][lane] = u - (s0 + s1);
+        load_w(c + 1);
+        f32x4 o = {}, o1 = {};
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            o = mma16(q4[j], st[j], o);
+            o1 = mma16(q4[j + 1], st[j + 1], o1);
+        }
+        load_q(c + 1);
+        lds_barrier();
+        f32x4 dv[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) dv[j] = dl[j][lane];
+        // the wave's own two state tiles (from LDS after the first chunk)
+        f32x4 n0, n1;
+        if (c == 0) {
+            n0 = wave == 0 ? st[0] : wave == 1 ? st[2] : wave == 2 ? st[4] : st[6];
+            n1 = wave == 0 ? st[1] : wave == 1 ? st[3] : wave == 2 ? st[5] : st[7];
+        } else {
+            n0 = sl[2 * wave][lane];
+            n1 = sl[2 * wave + 1][lane];
+        }
+        n0 *= g;
+        n1 *= g;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            n0 = mma16(k4[0][j], dv[j], n0);
+            n1 = mma16(k4[1][j], dv[j], n1);
+        }
+        sl[2 * wave][lane] = n0;
+        sl[2 * wave + 1][lane] = n1;
+        load_k(c + 1);
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+            o = mma16(a4[j], dv[j], o);
+            o1 = mma16(a4[j + 1], dv[j + 1], o1);
+        }
+        load_a(c + 1);
+        o += o1;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int tok = c * kCt + 16 * wave + 4 * lg + e;
+            if (tok < T) heads[(size_t)tok * chunk + h * kDk + col] = o[e];
+        }
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < 8; j++) st[j] = sl[j][lane];
+    }
+    // each wave writes its own two tiles
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const f32x4 v = sl[2 * wave + i][lane];
+#pragma unroll
+        for (int e = 0; e < 4; e++) Sh[(size_t)(16 * (2 * wave + i) + 4 * lg + e) * kDk] = v[e];
+    }
+}
+
+// After dn_scan_kernel: row b of the gated RMSNorm (deltanet.rs:517-533)
 // of the raw head outputs to the planes, and (row 0's workgroups) the conv
 // windows of the head's q, k and v channels after the T tokens: the last
 // kKsize values of (old window, the T inputs).  grid = (n_heads, T), 128 threads.
@@ -654,12 +855,12 @@ int launch_deltanet_scan(anehip_ctx *ctx, hipStream_t stream, int rows, int n_he
     if (kp > 16 || rows < 1 || rows > kScanMaxRows)
         return set_error(ctx->err, ANEHIP_EINVAL, "deltanet_scan: %d K splits (at most 16), %d rows (1..%d)", kp, rows,
                          kScanMaxRows);
-    float *bd = prep + (size_t)rows * n_heads * 3 * kDk;
+    const int chunks = (rows + kCt - 1) / kCt;
 #define DN_SCAN(KP)                                                                                                  \
-    hipLaunchKernelGGL(dn_prep_kernel<KP>, dim3(n_heads, rows), dim3(kThreads), 0, stream, mix, beta, alpha, conv_w, \
-                       ssm_a, dt_bias, conv_state, prep, bd, n_heads);                                               \
-    hipLaunchKernelGGL(deltanet_scan_kernel<kScanCols>, dim3(kDk / kScanCols, n_heads), dim3(kWave), 0, stream,     \
-                       prep, bd, S, heads, n_heads, rows);                                                           \
+    hipLaunchKernelGGL(dn_chunk_kernel<KP>, dim3(chunks, n_heads), dim3(kThreads), 0, stream, mix, beta, alpha,      \
+                       conv_w, ssm_a, dt_bias, conv_state, prep, n_heads, rows);                                     \
+    hipLaunchKernelGGL(dn_scan_kernel, dim3(kDk / 16, n_heads), dim3(kThreads), 0, stream, prep, S, heads, n_heads,  \
+                       rows);                                                                                        \
     hipLaunchKernelGGL(dn_scan_finish_kernel<KP>, dim3(n_heads, rows), dim3(kDk), 0, stream, mix, conv_state, heads, \
                        gate_off, norm_w, xp, n_heads, eps, rows)
     if (kp <= 1) {

@@ -535,6 +535,31 @@ def test_prefill_long_prompt_large_cache(mid_host, n):
     oseq.close()
 
 
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 129])
+def test_prefill_scan_chunk_edges(mid_host, n):
+    """Prompts around the DeltaNet scan's 64-token chunks (two tokens, fewer
+    than the conv window; one short of a chunk, one chunk, one token over; two
+    and one), from a state that three decode steps left, vs the oracle run
+    token by token: logits, states, conv windows, then a decode step."""
+    spec = mid_host.spec
+    gm = _model(mid_host, 1, 256)
+    oseq = mid_host.seq(256)
+    toks = oracle.randint(36, n, n + 4, spec.vocab_size)
+    for t in toks[:3]:
+        gm.step([int(t)])
+        oseq.forward(int(t))
+    g = gm.prefill(0, toks[3:3 + n])
+    for t in toks[3:3 + n]:
+        r = oseq.forward(int(t))
+    l2, mx = rel_errs(g, r)
+    print(f"prefill n={n}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
+    assert l2 <= TOL and mx <= TOL
+    _check_state(gm, oseq, 0, spec, "after prefill")
+    assert max(rel_errs(gm.step([int(toks[-1])])[0], oseq.forward(int(toks[-1])))) <= TOL
+    gm.close()
+    oseq.close()
+
+
 @pytest.mark.parametrize("n", [961, 1950])
 def test_prefill_full_chunks(mid_host, n):
     """Prompts past one chunk of 960 tokens: 961 (a full chunk, then one row on
