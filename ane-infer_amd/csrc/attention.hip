@@ -83,6 +83,51 @@ constexpr size_t kNtKvBytes = (size_t)32 << 20;
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+// Sharing of the launch's workgroups over sequences of different lengths (2
+// to 64 of them): every chunk gets at most `s` tiles, s the smallest (to 3 %)
+// for which the chunks of all sequences and kv heads fit the W workgroups, so
+// that a long sequence gets more of them than a short one.  (Chunks per
+// sequence fixed by the batch alone, the longest sequence's set the time:
+// batch 32, 2 kv heads, lengths spread over 2k-8k: 77 us a step against 65.)
+// Lane b of each wave holds sequence b's chunks per kv head (n) and its first
+// workgroup (start): kv head k's chunk c is workgroup start + k n + c.  With as
+// many tiles in every sequence the fixed split stands (even), and costs the
+// kernels no more than the positions' load.
+struct AttnPlan {
+    int pos, tiles, n, start;
+    bool even;
+};
+constexpr int kMaxPlanBatch = 64;
+// inclusive sum over the lanes of the wave up to this one
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1, 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2, 3
+    return v;
+}
+__device__ __forceinline__ AttnPlan attn_plan(const uint32_t *__restrict__ pos_arr, int batch, int n_kv, int W,
+                                              int max_tiles) {
+    const int lane = threadIdx.x & 63;
+    AttnPlan P;
+    P.pos = (int)pos_arr[min(lane, batch - 1)];
+    P.tiles = min(P.pos / kCh + 1, max_tiles);
+    P.even = __ballot(P.tiles != __builtin_amdgcn_readfirstlane(P.tiles)) == 0;
+    P.n = P.start = 0;
+    if (P.even) return P;
+    if (lane >= batch) P.tiles = 0;
+    const int total = __builtin_amdgcn_readlane(wave_scan(P.tiles), 63) * n_kv;
+    // ends at s = max_tiles at the latest: one chunk each, and batch x n_kv <= W
+    for (int s = (total + W - 1) / W;; s += 1 + s / 32) {
+        P.n = (P.tiles + s - 1) / s;
+        const int end = wave_scan(P.n * n_kv);
+        P.start = end - P.n * n_kv;
+        if (__builtin_amdgcn_readlane(end, 63) <= W || s >= max_tiles) return P;
+    }
+}
+
 // grid = (chunks, n_kv_heads, batch); chunk c takes the live tiles
 // [tb, te) of 64 positions that chunk_tiles() gives it.  mix: per
 // sequence [q_full | k | v] rows (K-split partial slices); q_full is
@@ -118,16 +163,19 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // one sincos per rotary pair and writes the q fragments straight from the
 // wave that normalised the head.
 //
+// PLAN: where the sequences' lengths differ, the launch's W workgroups (their
+// linear index) are shared out by attn_plan(); partials in workgroup order.
+//
 // Cache addressing: row b's cache is at cache_off + b * row_stride halves
 // (decode: every row its own sequence; prefill: row_stride 0, every row a
 // token of one sequence whose K / V rows the prefill append kernel wrote
 // before this launch -- then `append` is false and no row is written here).
-template <int G, bool NT>
+template <int G, bool NT, bool PLAN>
 __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
     MixIn mix, const float *__restrict__ q_norm, const float *__restrict__ k_norm,
     const float *__restrict__ inv_freq, const uint32_t *__restrict__ pos_arr, __half *__restrict__ k_cache,
     __half *__restrict__ v_cache, int max_seq, int n_heads, int n_kv, float *__restrict__ part_o,
-    float *__restrict__ part_ml, size_t cache_off, size_t row_stride, bool append) {
+    float *__restrict__ part_ml, size_t cache_off, size_t row_stride, bool append, int batch) {
     __shared__ __align__(16) h8v qf[8][2][64];
     __shared__ __align__(16) __half knew[kHd], vnew[kHd];
     __shared__ int qexp[G];
@@ -136,16 +184,18 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int li = lane & 15, lg = lane >> 4;
-    const int c = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+    int c = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+    const int nch = gridDim.x, slot0 = (b * n_kv + kvh) * nch + c;
     // inputs that do not depend on the position first: this wave's q head
     // (wave < G) or k / v rows (wave G % 4, used by the chunk holding pos),
     // the norm weights and the RoPE frequencies
     const bool is_q = wave < G, is_k = wave == G % 4;
-    const int hq = kvh * G + (wave < G ? wave : 0);
-    const int kin = n_heads * 2 * kHd + kvh * kHd;
-    const int vin = n_heads * 2 * kHd + n_kv * kHd + kvh * kHd;
+    int hq, kin, vin;
     float4 aq[8], ak[8], av[8];
-    {
+    auto load_inputs = [&]() {
+        hq = kvh * G + (wave < G ? wave : 0);
+        kin = n_heads * 2 * kHd + kvh * kHd;
+        vin = n_heads * 2 * kHd + n_kv * kHd + kvh * kHd;
         const float *r0 = mix.p + (size_t)b * mix.stride + 4 * lane;
 #pragma unroll
         for (int q = 0; q < 8; q++)
@@ -157,15 +207,35 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
                     av[q] = *reinterpret_cast<const float4 *>(rq + vin);
                 }
             }
-    }
+    };
+    load_inputs();
     const float4 wq = *reinterpret_cast<const float4 *>(q_norm + 4 * lane);
     const float4 wk = *reinterpret_cast<const float4 *>(k_norm + 4 * lane);
     const float2 fr = *reinterpret_cast<const float2 *>(inv_freq + 2 * lane);
-    const uint32_t pos = pos_arr[b];
+    uint32_t pos;
+    int tb = 0, te = 0;  // tiles [tb, te)
+    bool shared_out = false;
+    if constexpr (PLAN) {
+        const AttnPlan P = attn_plan(pos_arr, batch, n_kv, batch * n_kv * nch, (max_seq + kCh - 1) / kCh);
+        if (!P.even) {
+            shared_out = true;
+            b = 63 - __builtin_clzll(__ballot(P.start <= slot0 && lane < batch));
+            const int n = __builtin_amdgcn_readlane(P.n, b), r = slot0 - __builtin_amdgcn_readlane(P.start, b);
+            const int tiles = __builtin_amdgcn_readlane(P.tiles, b);
+            kvh = r / n;
+            c = r % n;
+            if (kvh >= n_kv) return;  // uniform exit: past the last chunk
+            load_inputs();
+            // 32-bit: c < 256 and tiles < 2^15 (a cache row is below 1 GiB)
+            tb = (int)((uint32_t)(c * tiles) / (uint32_t)n);
+            te = (int)((uint32_t)((c + 1) * tiles) / (uint32_t)n);
+        }
+        pos = (uint32_t)__builtin_amdgcn_readlane(P.pos, b);
+    } else {
+        pos = pos_arr[b];
+    }
     const int len = (int)pos + 1;
-    const int nch = gridDim.x;
-    int tb, te;  // tiles [tb, te)
-    if (!chunk_tiles(len, nch, c, &tb, &te)) return;  // uniform exit: nothing of this sequence here
+    if (!shared_out && !chunk_tiles(len, nch, c, &tb, &te)) return;  // uniform exit: nothing of this sequence here
     const size_t cache_base = cache_off + (size_t)b * row_stride + (size_t)kvh * max_seq * kHd;
     const bool has_new = (int)pos < te * kCh;
     const __amdgpu_buffer_rsrc_t krs =
@@ -390,7 +460,7 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
             L += sw * wl[w][hh];
             acc = make_float4(acc.x + sw * v.x, acc.y + sw * v.y, acc.z + sw * v.z, acc.w + sw * v.w);
         }
-        const size_t slot = (((size_t)b * n_kv + kvh) * nch + c) * G + hh;
+        const size_t slot = (size_t)slot0 * G + hh;
         const float inv = 1.0f / kPScale;
         *reinterpret_cast<float4 *>(part_o + slot * kHd + 4 * d4) =
             make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
@@ -426,40 +496,53 @@ __global__ __launch_bounds__(64) void attn_append_kernel(MixIn mix, const float 
     }
 }
 
-// grid = (n_heads, batch), 256 threads: thread (g = t / 64, l = t % 64) takes
-// dims 4l..4l+3 of chunks g, g + 4, g + 8, ...; merges them with a log-sum-exp
-// rescale against the maximum over all chunks, adds the 4 groups through
-// LDS, normalises and multiplies by sigmoid(gate) (deltanet.rs:667-669).
+// grid = (n_heads, batch), 64 GR threads: thread (g = t / 64, l = t % 64) takes
+// dims 4l..4l+3 of chunks g, g + GR, g + 2 GR, ...; merges them with a
+// log-sum-exp rescale against the maximum over all chunks, adds the GR groups
+// through LDS, normalises and multiplies by sigmoid(gate) (deltanet.rs:667-669).
+// GR = 16 where a head has more than 16 chunks (up to 8 per group, all loaded
+// at once; with 4 groups of 32 chunks one after the other batch 1 at 32k
+// positions took 14.6 us; a step there 30.6 -> 22.5), 4 else.
 // out: [batch][n_heads * 256] fp32, or range-safe fragment-order planes xp
-// (Planes) when xp.hi is not null.
-template <int G>
-__global__ __launch_bounds__(kThreads) void attn_combine_kernel(MixIn mix, const uint32_t *__restrict__ pos_arr,
-                                                                const float *__restrict__ part_o,
-                                                                const float *__restrict__ part_ml, int nch,
-                                                                int n_heads, int n_kv, float *__restrict__ out,
-                                                                Planes xp) {
-    __shared__ float red[4];
-    __shared__ float4 accs[4][64];
-    __shared__ float dens[4][64];
+// (Planes) when xp.hi is not null.  plan_w > 0: the partials of a launch of
+// plan_w workgroups that attn_plan() may have shared out.
+template <int G, int GR>
+__global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const uint32_t *__restrict__ pos_arr,
+                                                               const float *__restrict__ part_o,
+                                                               const float *__restrict__ part_ml, int nch,
+                                                               int n_heads, int n_kv, float *__restrict__ out,
+                                                               Planes xp, int plan_w, int max_seq) {
+    constexpr int PRE = GR == 16 ? 8 : 4;  // chunks of a group loaded before the maximum is known
+    __shared__ float red[GR];
+    __shared__ float4 accs[GR][64];
+    __shared__ float dens[GR][64];
     const int t = threadIdx.x, g = t >> 6, l = t & 63, h = blockIdx.x, b = blockIdx.y;
     const int kvh = h / G, hh = h % G;
-    const int len = (int)pos_arr[b] + 1;
-    const int nc = active_chunks(len, nch);
-    const size_t base = ((size_t)b * n_kv + kvh) * nch;
     // the gate's K-split slices (independent of the partials) and this
-    // group's first 4 chunks (g, g + 4, g + 8, g + 12; the only ones at batch
-    // 32) are loaded together, before the maximum is known
+    // group's first PRE chunks are loaded together, before the maximum is known
     float4 gq[8];
     {
         const float *g0 = mix.p + (size_t)b * mix.stride + h * 2 * kHd + kHd + 4 * l;
 #pragma unroll
         for (int q = 0; q < 8; q++) gq[q] = *reinterpret_cast<const float4 *>(g0 + (size_t)min(q, mix.kp - 1) * mix.split);
     }
-    float4 p4[4];
-    float pm[4], pl[4];
+    int nc;
+    size_t base;
+    AttnPlan P;
+    P.even = true;
+    if (plan_w) P = attn_plan(pos_arr, (int)gridDim.y, n_kv, plan_w, (max_seq + kCh - 1) / kCh);
+    if (P.even) {
+        nc = active_chunks((plan_w ? __builtin_amdgcn_readlane(P.pos, b) : (int)pos_arr[b]) + 1, nch);
+        base = ((size_t)b * n_kv + kvh) * nch;
+    } else {
+        nc = __builtin_amdgcn_readlane(P.n, b);
+        base = (size_t)(__builtin_amdgcn_readlane(P.start, b) + kvh * nc);
+    }
+    float4 p4[PRE];
+    float pm[PRE], pl[PRE];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const size_t slot = (base + min(g + 4 * i, nc - 1)) * G + hh;
+    for (int i = 0; i < PRE; i++) {
+        const size_t slot = (base + min(g + GR * i, nc - 1)) * G + hh;
         p4[i] = *reinterpret_cast<const float4 *>(part_o + slot * kHd + 4 * l);
         pm[i] = part_ml[slot * 2];
         pl[i] = part_ml[slot * 2 + 1];
@@ -474,50 +557,45 @@ __global__ __launch_bounds__(kThreads) void attn_combine_kernel(MixIn mix, const
         gate = make_float4(gate.x + v.x, gate.y + v.y, gate.z + v.z, gate.w + v.w);
     }
     // maximum over the chunks: each group's (the same in all its lanes), then
-    // over the 4 groups
+    // over the groups
     float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 4; i++) mx = g + 4 * i < nc ? fmaxf(mx, pm[i]) : mx;
-    for (int c2 = g + 16; c2 < nc; c2 += 4) mx = fmaxf(mx, part_ml[((base + c2) * G + hh) * 2]);
+    for (int i = 0; i < PRE; i++) mx = g + GR * i < nc ? fmaxf(mx, pm[i]) : mx;
+    for (int c2 = g + GR * PRE; c2 < nc; c2 += GR) mx = fmaxf(mx, part_ml[((base + c2) * G + hh) * 2]);
     if (l == 0) red[g] = mx;
     __syncthreads();
-    const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    // this group's chunks in order: the 4 loaded above, then 4 per trip with
+    float M = red[0];
+#pragma unroll
+    for (int k = 1; k < GR; k++) M = fmaxf(M, red[k]);
+    // this group's chunks in order: those loaded above, then 4 per trip with
     // their loads issued together
     float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
     float den = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (g + 4 * i < nc) {
+    for (int i = 0; i < PRE; i++) {
+        if (g + GR * i < nc) {
             const float w = expf(pm[i] - M);
             num = make_float4(num.x + w * p4[i].x, num.y + w * p4[i].y, num.z + w * p4[i].z, num.w + w * p4[i].w);
             den += w * pl[i];
         }
     }
-    int cc = g + 16;
-    for (; cc + 12 < nc; cc += 16) {
+    for (int cc = g + GR * PRE; cc < nc; cc += 4 * GR) {
         float4 o4[4];
         float m4[4], l4[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const size_t slot = (base + cc + 4 * i) * G + hh;
+            const size_t slot = (base + min(cc + GR * i, nc - 1)) * G + hh;
             o4[i] = *reinterpret_cast<const float4 *>(part_o + slot * kHd + 4 * l);
             m4[i] = part_ml[slot * 2];
             l4[i] = part_ml[slot * 2 + 1];
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
+            if (cc + GR * i >= nc) break;
             const float w = expf(m4[i] - M);
             num = make_float4(num.x + w * o4[i].x, num.y + w * o4[i].y, num.z + w * o4[i].z, num.w + w * o4[i].w);
             den += w * l4[i];
         }
-    }
-    for (; cc < nc; cc += 4) {
-        const size_t slot = (base + cc) * G + hh;
-        const float4 o = *reinterpret_cast<const float4 *>(part_o + slot * kHd + 4 * l);
-        const float w = expf(part_ml[slot * 2] - M);
-        num = make_float4(num.x + w * o.x, num.y + w * o.y, num.z + w * o.z, num.w + w * o.w);
-        den += w * part_ml[slot * 2 + 1];
     }
     accs[g][l] = num;
     dens[g][l] = den;
@@ -526,7 +604,7 @@ __global__ __launch_bounds__(kThreads) void attn_combine_kernel(MixIn mix, const
     float4 s = accs[0][l];
     float dsum = dens[0][l];
 #pragma unroll
-    for (int k = 1; k < 4; k++) {
+    for (int k = 1; k < GR; k++) {
         const float4 o = accs[k][l];
         s = make_float4(s.x + o.x, s.y + o.y, s.z + o.z, s.w + o.w);
         dsum += dens[k][l];
@@ -589,21 +667,29 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
     dim3 g1(nch, n_kv, batch), g2(n_heads, batch);
     // the caches this launch can read (prefill rows share one sequence's)
     const bool nt = (size_t)(row_stride ? batch : 1) * n_kv * max_seq * 2 * kHd * sizeof(__half) >= kNtKvBytes;
-#define ANEHIP_ATTN_CASE(GG)                                                                                   \
-    case GG:                                                                                                   \
-        if (nt)                                                                                                \
-            hipLaunchKernelGGL((attn_partial_kernel<GG, true>), g1, dim3(kThreads), 0, stream, mix, q_norm,    \
-                               k_norm, inv_freq, pos, k_cache, v_cache, max_seq, n_heads, n_kv, part_o,       \
-                               part_ml, cache_off, row_stride, append);                                       \
-        else                                                                                                   \
-            hipLaunchKernelGGL((attn_partial_kernel<GG, false>), g1, dim3(kThreads), 0, stream, mix, q_norm,   \
-                               k_norm, inv_freq, pos, k_cache, v_cache, max_seq, n_heads, n_kv, part_o,       \
-                               part_ml, cache_off, row_stride, append);                                       \
-        ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                           \
-        if (!out && !xp.hi) return ANEHIP_OK; /* partials only */                                              \
-        hipLaunchKernelGGL(attn_combine_kernel<GG>, g2, dim3(kThreads), 0, stream, mix, pos, part_o, part_ml,  \
-                           nch, n_heads, n_kv, out, xp);                                                      \
-        ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                           \
+    // sequences of their own, at least two workgroups each to share out
+    const bool plan = row_stride && batch >= 2 && batch <= kMaxPlanBatch && nch >= 2;
+    const int W = batch * n_kv * nch;
+    const bool many = nch > 16;  // chunks per head, with a plan on average
+#define ANEHIP_ATTN_PART(GG, NT, PLAN)                                                                          \
+    hipLaunchKernelGGL((attn_partial_kernel<GG, NT, PLAN>), g1, dim3(kThreads), 0, stream, mix, q_norm, k_norm, \
+                       inv_freq, pos, k_cache, v_cache, max_seq, n_heads, n_kv, part_o, part_ml, cache_off,     \
+                       row_stride, append, batch)
+#define ANEHIP_ATTN_CASE(GG)                                                                                    \
+    case GG:                                                                                                    \
+        if (nt && plan) ANEHIP_ATTN_PART(GG, true, true);                                                       \
+        else if (nt) ANEHIP_ATTN_PART(GG, true, false);                                                         \
+        else if (plan) ANEHIP_ATTN_PART(GG, false, true);                                                       \
+        else ANEHIP_ATTN_PART(GG, false, false);                                                                \
+        ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                            \
+        if (!out && !xp.hi) return ANEHIP_OK; /* partials only */                                               \
+        if (many)                                                                                               \
+            hipLaunchKernelGGL((attn_combine_kernel<GG, 16>), g2, dim3(64 * 16), 0, stream, mix, pos, part_o,   \
+                               part_ml, nch, n_heads, n_kv, out, xp, plan ? W : 0, max_seq);                    \
+        else                                                                                                    \
+            hipLaunchKernelGGL((attn_combine_kernel<GG, 4>), g2, dim3(64 * 4), 0, stream, mix, pos, part_o,     \
+                               part_ml, nch, n_heads, n_kv, out, xp, plan ? W : 0, max_seq);                    \
+        ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                            \
         return ANEHIP_OK;
     switch (G) {
         ANEHIP_ATTN_CASE(1)
@@ -613,6 +699,7 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
             return set_error(ctx->err, ANEHIP_EUNSUPPORTED, "attention: %d query heads per kv head (1, 2 or 4)", G);
     }
 #undef ANEHIP_ATTN_CASE
+#undef ANEHIP_ATTN_PART
 }
 
 }  // namespace

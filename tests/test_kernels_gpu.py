@@ -190,6 +190,18 @@ def test_attention_live_length_split(gpu_ctx, oracle_lib):
     _attn_case(gpu_ctx, oracle_lib, 8, 8, 2, 8192, [0, 63, 64, 700, 4095, 5000, 8000, 8191], seed=77, tol=5e-4)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,max_seq,positions", [
+    (8, 2, 4096, [4095, 0]), (4, 4, 2048, [5, 2047, 64]), (2, 1, 640, [639] + 5 * [0]),
+    (4, 1, 1000, [17 * i % 1000 for i in range(33)]), (2, 2, 700, [(37 * i) % 700 for i in range(64)]),
+    (2, 2, 130, [i for i in range(65)]), (4, 2, 300, 3 * [255])])
+def test_attention_shared_out_workgroups(gpu_ctx, oracle_lib, n_heads, n_kv, max_seq, positions):
+    """Launches whose workgroups are shared out by length (batch 2 to 64, at
+    least two per sequence and kv head): one long sequence beside empty ones,
+    more chunks for one head than the combine loads at once, batches that do
+    not divide the workgroups, equal lengths; batch 65 keeps the fixed split."""
+    _attn_case(gpu_ctx, oracle_lib, len(positions), n_heads, n_kv, max_seq, positions, seed=max_seq + len(positions), tol=5e-4)
+
+
 @pytest.mark.parametrize("n_heads,n_kv", [(8, 2), (4, 2), (2, 2)])
 def test_attention_gqa_ratios(gpu_ctx, oracle_lib, n_heads, n_kv):
     _attn_case(gpu_ctx, oracle_lib, 1, n_heads, n_kv, 200, [150], seed=n_heads * 10 + n_kv)
