@@ -200,7 +200,7 @@ int launch_quant_gemm(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, c
 int gemm_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, int max_k = 8);
 inline int split_len(int nsb, int ksplit) { return (nsb + ksplit - 1) / ksplit; }
 // xsplit: device scratch of batch * n floats (x split into fp16 hi / lo
-// planes for the MFMA path); may be null when batch == 1.
+// planes for the MFMA path); may be null up to batch 16.
 int launch_gemm_raw(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w, uint32_t m,
                     uint32_t n, const float *x, uint32_t batch, float *out, int ksplit, void *xsplit);
 int launch_sum_partials(anehip_ctx *ctx, hipStream_t stream, const float *part, float *y, size_t count,

@@ -2528,252 +2528,122 @@ __device__ __forceinline__ float blk_scale(const uint32_t *wl, int blk) {
     return half_at(wl, blk * QTraits<T>::kBlockBytes);
 }
 
-// grid = (row tiles of 64, K splits); 4 waves per workgroup, as the GEMV.
-// NT = 16-wide batch tiles (1: batch <= 16, 2: batch <= 32).  xh / xl: fp16
-// planes [batch][n].  Output as quant_gemm_tiled.
+// GEMM over GGUF blocks at batch 2..16, x-stationary: 8 waves per workgroup,
+// wave w holds the x fragments (hi + lo) of super-block ks * 8 + w in
+// registers, split from the fp32 rows by the wave itself (one exponent per
+// batch row over its super-block; the wave's sums are multiplied by 2^E, exact,
+// before the waves' are added), and the workgroup walks the row tiles (16 RS
+// rows) t = blockIdx.x, + gridDim.x, ...  Per tile each wave stages its rows x
+// 1 super-block of GGUF blocks through its own LDS slice and issues the next
+// tile's loads at once (in flight while this tile is multiplied), then the 8
+// waves' sums are added through LDS (the staging area, after a barrier).
+// grid = (workgroups per split, K splits of 8 super-blocks, the last possibly
+// fewer, groups of 16 batch rows); out[ks * split_stride + b * m + r].
 //
-// Operands: A = activations (16 batch rows x 32 columns), B = weights (32
-// columns x 16 weight rows), so D[b][r] = sum_k x[b][k] W[r][k]; a lane's four
-// D values share one weight row and therefore one block scale.
-template <uint32_t T, int NT>
-__global__ __launch_bounds__(kWave *kWavesPerWg) void quant_gemm_mfma(const uint8_t *__restrict__ W, Planes xp,
-                                                                     float *__restrict__ out, int m, int n,
-                                                                     int batch, int sb_per_split,
-                                                                     size_t split_stride) {
+// What bounds it on few tiles: the chain x -> weights -> LDS -> fragments
+// (about 20 VALU operations per 16 x 8 weights: 4 us for a 64-row tile, two
+// waves per SIMD).  So the tile is the smallest of 64, 32, 16 rows that still
+// gives one workgroup per CU at most.  Measured (graphs of back-to-back calls,
+// weights rotated past the caches; before: x split into planes, 4-wave
+// workgroups over 2 K splits, their sum), Q8_0 at batch 8 / 32:
+//   2048 x 2048 6.3 / 7.7 us (12.8 / 21.8), 6144 x 2048 7.9 / 12.2 (13.4 /
+//   22.9), 12288 x 2048 11.4 / 22.9 (16.9 / 31.3), 2048 x 6144 10.0 / 14.3
+//   (13.8 / 24.0); with 64-row tiles only: 10.5, 10.8, 11.3, 13.0 at batch 8.
+template <uint32_t T, int RS>
+__global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__ W, const float *__restrict__ x,
+                                                     float *__restrict__ out, int m, int n, int batch,
+                                                     size_t split_stride) {
     constexpr int V = QTraits<T>::kSbVec;
-    __shared__ u32x4 lds[kWavesPerWg][V * kWave];
-    __shared__ int xeE[32];
-    const _Float16 *__restrict__ xh = xp.hi;
-    const _Float16 *__restrict__ xl = xp.lo;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int tile = blockIdx.x;
-    const int ks = blockIdx.y;
-    const int nsb = n >> 8;
-    const size_t row_bytes = (size_t)nsb * QTraits<T>::kSbBytes;
-    const int row0 = tile * kWave;
-    const int sb_begin = ks * sb_per_split;
-    const int sb_end = min(nsb, sb_begin + sb_per_split);
-    const int li = lane & 15;  // A row (batch) / B column (weight row) within a 16 tile
-    const int g = lane >> 4;   // k group (8 columns) / D row group
-
-    f32x4 acc[4][NT];
-#pragma unroll
-    for (int rs = 0; rs < 4; rs++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) acc[rs][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    u32x4 regs[V];
-    uint32_t off[V];
-    tile_offsets<T>(off, (uint32_t)row_bytes, m - row0, lane);
-    const uint8_t *tile_base = W + (size_t)row0 * row_bytes;
-    const uint32_t *lds_words = reinterpret_cast<const uint32_t *>(lds[wave]);
+    constexpr int NW = 8, R = 16 * RS;          // rows per tile
+    constexpr int C = V * R, VJ = (C + kWave - 1) / kWave;  // a wave's 16-byte chunks of a tile, per lane
     constexpr int kSegWords = QTraits<T>::kSbBytes / 4;
-
-    // the two group exponents of super-block s for batch row li + 16 nt,
-    // loaded with that super-block's weights (one super-block ahead), so the
-    // block loop multiplies by a factor already in registers
-    auto xe_pair = [&](int s, int nt) {
-        const int8_t *e = xp.xe + (size_t)min(li + 16 * nt, batch - 1) * xe_stride(n) + 2 * s;
-        return make_int2(e[0], e[1]);
-    };
-    int2 xen[NT];
-    int sb = sb_begin + wave;
-    if (sb < sb_end) {
-        load_tile<T>(regs, tile_base + (size_t)sb * QTraits<T>::kSbBytes, off);
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) xen[nt] = xe_pair(sb, nt);
-    }
-    // range-safe planes: the split's groups (2 per super-block) of batch row
-    // li + 16 nt brought to one exponent En[nt] (read after the first weight
-    // loads were issued)
-    int En[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        const int b = min(li + 16 * nt, batch - 1);
-        En[nt] = xe_max(xp.xe, b, 2 * sb_begin, 2 * (sb_end - sb_begin), n);
-        if (wave == 0 && g == 0) xeE[li + 16 * nt] = En[nt];  // read after the reduction barrier
-    }
-    for (; sb < sb_end; sb += kWavesPerWg) {
-        _Float16 fgrp[NT][2];
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            fgrp[nt][0] = xe_factor(xen[nt].x, En[nt]);
-            fgrp[nt][1] = xe_factor(xen[nt].y, En[nt]);
-        }
-        // A fragments of block blk: x[b = li + 16 nt][sb*256 + 32 blk + 8 g +
-        // e]; rows past the batch read row batch - 1 (branch-free; those MFMA
-        // output rows are never stored)
-        auto load_x = [&](int blk, f16x8 (&ah)[NT], f16x8 (&al)[NT]) {
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const int b = min(li + 16 * nt, batch - 1);
-                const size_t xo = (size_t)b * n + (size_t)sb * 256 + 32 * blk + 8 * g;
-                ah[nt] = *reinterpret_cast<const f16x8 *>(xh + xo);
-                al[nt] = *reinterpret_cast<const f16x8 *>(xl + xo);
-            }
-        };
-        f16x8 nh[2][NT], nl[2][NT];  // the next block pair's fragments
-        load_x(0, nh[0], nl[0]);
-        load_x(1, nh[1], nl[1]);
-        stage_tile<T>(regs, lds[wave], lane);
-        // blocks in pairs (even, odd): a runtime loop bounds the live
-        // registers; each pair's x is loaded one pair ahead (unconditionally:
-        // the last pair re-reads its own, which keeps the loop body
-        // straight-line and the waits exact).  The next super-block's weights
-        // are loaded after the loop: loads complete in issue order, so an x
-        // load issued after them would wait for their HBM round trip.
-#pragma unroll 1
-        for (int bp = 0; bp < 4; bp++) {
-            f16x8 ch[2][NT], cl[2][NT];
-#pragma unroll
-            for (int odd = 0; odd < 2; odd++)
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) {
-                    ch[odd][nt] = nh[odd][nt];
-                    cl[odd][nt] = nl[odd][nt];
-                }
-            const int np = min(bp + 1, 3);
-            load_x(2 * np, nh[0], nl[0]);
-            load_x(2 * np + 1, nh[1], nl[1]);
-#pragma unroll
-            for (int odd = 0; odd < 2; odd++) {
-                const int blk = 2 * bp + odd;
-                f16x8 ah[NT], al[NT];
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) {
-                    const _Float16 f = bp < 2 ? fgrp[nt][0] : fgrp[nt][1];
-                    ah[nt] = ch[odd][nt] * f;
-                    al[nt] = cl[odd][nt] * f;
-                }
-#pragma unroll
-                for (int rs = 0; rs < 4; rs++) {
-                    const uint32_t *wl = lds_words + (rs * 16 + li) * kSegWords;
-                    const f16x8 bw = odd ? w_frag<T, 1>(wl, blk, g) : w_frag<T, 0>(wl, blk, g);
-                    const float d = blk_scale<T>(wl, blk);
-#pragma unroll
-                    for (int nt = 0; nt < NT; nt++) {
-                        f32x4 c =
-                            __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[nt], bw, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[nt], bw, c, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 4; r++) acc[rs][nt][r] = fmaf(c[r], d, acc[rs][nt][r]);
-                    }
-                }
-            }
-        }
-        if (sb + kWavesPerWg < sb_end) {
-            load_tile<T>(regs, tile_base + (size_t)(sb + kWavesPerWg) * QTraits<T>::kSbBytes, off);
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) xen[nt] = xe_pair(sb + kWavesPerWg, nt);
-        }
-        wave_sync_lds();
-    }
-    // reduce the 4 waves through LDS (the staging buffer is free now)
-    __syncthreads();
-    float *red = reinterpret_cast<float *>(&lds[0][0]);  // [4 waves][4 rs][NT][4][64]
-    constexpr int per = 4 * NT * 4;
-#pragma unroll
-    for (int rs = 0; rs < 4; rs++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) red[((wave * per) + (rs * NT + nt) * 4 + r) * kWave + lane] = acc[rs][nt][r];
-    __syncthreads();
-    if (wave != 0) return;
-    float *dst = out + (size_t)ks * split_stride;
-#pragma unroll
-    for (int rs = 0; rs < 4; rs++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int idx = (rs * NT + nt) * 4 + r;
-                float sum = red[idx * kWave + lane];
-#pragma unroll
-                for (int v = 1; v < kWavesPerWg; v++) sum += red[(v * per + idx) * kWave + lane];
-                const int row = row0 + rs * 16 + li;
-                const int b = 16 * nt + 4 * g + r;
-                if (row < m && b < batch) dst[(size_t)b * m + row] = ldexpf(sum, xeE[b]);
-            }
-}
-
-// x-stationary form of quant_gemm_mfma for matrices of many row tiles at
-// batch 2..16 (lm_head): 8 waves per workgroup, wave w holds the x fragments
-// (hi + lo, brought to one exponent per batch row over the split's 16
-// groups, as quant_gemm_mfma) of super-block ks * 8 + w in registers, and
-// the workgroup walks the row tiles t = blockIdx.x, + gridDim.x, ...  Per
-// tile each wave stages its 64 rows x 1 super-block of GGUF blocks through
-// its own LDS slice and issues the next tile's loads at once (in flight
-// while this tile is multiplied), then the 8 waves' sums are added through
-// LDS (the staging area, after a barrier).  The x fragments are loaded once
-// per workgroup instead of once per tile (lm_head at batch 16: 2374 tiles x
-// 128 KiB of x from L2 otherwise).  grid = (workgroups per split, K splits
-// of 8 super-blocks); output as quant_gemm_mfma.
-template <uint32_t T>
-__global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__ W, Planes xp, float *__restrict__ out,
-                                                     int m, int n, int batch, size_t split_stride) {
-    constexpr int V = QTraits<T>::kSbVec;
-    constexpr int NW = 8;
-    constexpr int kSegWords = QTraits<T>::kSbBytes / 4;
-    constexpr int RED = 16;  // sums per lane: [row group rs][element r]
-    static_assert(NW * RED * kWave * 4 <= NW * V * kWave * 16, "the reduction fits the staging area");
-    __shared__ u32x4 lds[NW][V * kWave];
-    __shared__ int xeE[16];
+    constexpr int RED = 4 * RS;  // sums per lane: [row group rs][element r]
+    static_assert(NW * RED * kWave * 4 <= NW * C * 16, "the reduction fits the staging area");
+    __shared__ u32x4 lds[NW][C];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int G = gridDim.x, ks = blockIdx.y;
-    const int nsb = n >> 8, tiles = (m + kWave - 1) / kWave;
+    const int nsb = n >> 8, tiles = (m + R - 1) / R;
+    x += (size_t)16 * blockIdx.z * n;
+    out += (size_t)16 * blockIdx.z * m;
+    batch = min(batch - 16 * (int)blockIdx.z, 16);
     const uint32_t row_bytes = (uint32_t)nsb * QTraits<T>::kSbBytes;
-    const int sb = ks * NW + wave;
+    const bool on = ks * NW + wave < nsb;  // waves past the last super-block add zeros
+    const int sb = on ? ks * NW + wave : nsb - 1;
     const int li = lane & 15, g = lane >> 4;
     int t = blockIdx.x;
     if (t >= tiles) return;  // uniform
-    // chunk c = 64 j + lane of a tile's super-block column: (row c / V, part
-    // c % V), rows past m clamped to the last row (never stored)
-    u32x4 regs[V];
-    auto issue = [&](int tt) {
-        const int rows_left = m - tt * kWave;
-        const uint8_t *base = W + (size_t)tt * kWave * row_bytes + (size_t)sb * QTraits<T>::kSbBytes;
+    // x[b = li][sb * 256 + 32 blk + 8 g + e] (rows past the batch read row
+    // batch - 1; their outputs are never stored): these loads go out before
+    // the first tile's weights
+    float4 xv[8][2];
+    {
+        const float *xr = x + (size_t)min(li, batch - 1) * n + (size_t)sb * 256 + 8 * g;
 #pragma unroll
-        for (int j = 0; j < V; j++) {
-            const int c = j * kWave + lane;
+        for (int blk = 0; blk < 8; blk++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) xv[blk][i] = *reinterpret_cast<const float4 *>(xr + 32 * blk + 4 * i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // chunk c = 64 j + lane of a tile's super-block column: (row c / V, part
+    // c % V), rows past m clamped to the last row (never stored), chunks past
+    // the tile to its last
+    u32x4 regs[VJ];
+    auto chunk = [&](int j) { return C % kWave ? min(j * kWave + lane, C - 1) : j * kWave + lane; };
+    auto issue = [&](int tt) {
+        const int rows_left = m - tt * R;
+        const uint8_t *base = W + (size_t)tt * R * row_bytes + (size_t)sb * QTraits<T>::kSbBytes;
+#pragma unroll
+        for (int j = 0; j < VJ; j++) {
+            const int c = chunk(j);
             const uint32_t o = (uint32_t)min(c / V, rows_left - 1) * row_bytes + (uint32_t)(c % V) * 16u;
             regs[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + o));
         }
     };
     issue(t);
-    // A fragments x[b = li][sb * 256 + 32 blk + 8 g + e] (rows past the batch
-    // read row batch - 1; their outputs are never stored), loaded after the
-    // first tile's weights were issued
+    __builtin_amdgcn_sched_barrier(0);
     h8v ah[8], al[8];
+    int Er[4];  // exponents of the batch rows whose sums the lane holds: 4 g + r
     {
-        const int b = min(li, batch - 1);
-        const int En = xe_max(xp.xe, b, 2 * ks * NW, 2 * NW, n);
-        if (wave == 0 && g == 0) xeE[li] = En;
-        const int8_t *e = xp.xe + (size_t)b * xe_stride(n) + 2 * sb;
-        const _Float16 f0 = xe_factor(e[0], En), f1 = xe_factor(e[1], En);
+        float amax = 0.0f;
+#pragma unroll
+        for (int blk = 0; blk < 8; blk++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float4 v = xv[blk][i];
+                amax = fmaxf(fmaxf(amax, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+            }
+        const int E = group_exp(lanes_max4(amax));
 #pragma unroll
         for (int blk = 0; blk < 8; blk++) {
-            const size_t xo = (size_t)b * n + (size_t)sb * 256 + 32 * blk + 8 * g;
-            const _Float16 f = blk < 4 ? f0 : f1;
-            ah[blk] = *reinterpret_cast<const h8v *>(xp.hi + xo) * f;
-            al[blk] = *reinterpret_cast<const h8v *>(xp.lo + xo) * f;
+            const float4 v0 = xv[blk][0], v1 = xv[blk][1];
+            const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                _Float16 hh, ll;
+                split_scaled(on ? f[e] : 0.0f, E, hh, ll);
+                ah[blk][e] = hh;
+                al[blk][e] = ll;
+            }
         }
+#pragma unroll
+        for (int r = 0; r < 4; r++) Er[r] = __shfl(E, 4 * g + r);
     }
     const uint32_t *lw = reinterpret_cast<const uint32_t *>(lds[wave]);
     float *red = reinterpret_cast<float *>(&lds[0][0]);  // [wave][RED][lane], after the tile's barrier
     float *dst = out + (size_t)ks * split_stride;
     for (; t < tiles; t += G) {
-        stage_tile<T>(regs, lds[wave], lane);
-        if (t + G < tiles) issue(t + G);
-        f32x4 acc[4];
 #pragma unroll
-        for (int rs = 0; rs < 4; rs++) acc[rs] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < VJ; j++) lds[wave][chunk(j)] = regs[j];
+        wave_sync_lds();
+        if (t + G < tiles) issue(t + G);
+        f32x4 acc[RS];
+#pragma unroll
+        for (int rs = 0; rs < RS; rs++) acc[rs] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int blk = 0; blk < 8; blk++) {
 #pragma unroll
-            for (int rs = 0; rs < 4; rs++) {
+            for (int rs = 0; rs < RS; rs++) {
                 const uint32_t *wl = lw + (rs * 16 + li) * kSegWords;
                 const h8v bw = (blk & 1) ? w_frag<T, 1>(wl, blk, g) : w_frag<T, 0>(wl, blk, g);
                 const float d = blk_scale<T>(wl, blk);
@@ -2786,21 +2656,22 @@ __global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__
         }
         __syncthreads();  // every wave is done with its slice
 #pragma unroll
-        for (int rs = 0; rs < 4; rs++)
+        for (int rs = 0; rs < RS; rs++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) red[(wave * RED + rs * 4 + r) * kWave + lane] = acc[rs][r];
+            for (int r = 0; r < 4; r++) red[(wave * RED + rs * 4 + r) * kWave + lane] = ldexpf(acc[rs][r], Er[r]);
         __syncthreads();
         // outputs (tile row rs * 16 + l % 16, batch row 4 (l / 16) + r), the
         // 8 waves added in wave order
 #pragma unroll
-        for (int k = 0; k < RED * kWave / 512; k++) {
+        for (int k = 0; k < (RED * kWave + 511) / 512; k++) {
             const int o = (int)threadIdx.x + 512 * k;
+            if (o >= RED * kWave) break;
             const int idx = o >> 6, l = o & 63;
             float s = red[idx * kWave + l];
 #pragma unroll
             for (int w = 1; w < NW; w++) s += red[(w * RED + idx) * kWave + l];
-            const int row = t * kWave + (idx >> 2) * 16 + (l & 15), b = 4 * (l >> 4) + (idx & 3);
-            if (row < m && b < batch) dst[(size_t)b * m + row] = ldexpf(s, xeE[b]);
+            const int row = t * R + (idx >> 2) * 16 + (l & 15), b = 4 * (l >> 4) + (idx & 3);
+            if (row < m && b < batch) dst[(size_t)b * m + row] = s;
         }
         __syncthreads();  // the staging area is free again
     }
@@ -2813,9 +2684,9 @@ __global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__
 // pair's two segments are shared through LDS by waves q and q + 4, and each
 // batch half's 4 waves are added per tile.  The lane's load offsets are
 // recomputed per tile (held across the loop they cost 34 registers and the
-// kernel spilled).  lm_head 151936 x 2048 at batch 17 / 32: 126.8-128.0 /
-// 133.4-133.6 us against 134.3-141.8 / 160.3-166.1 us on quant_gemm_mfma<T,
-// 2> (graphs of back-to-back launches).
+// kernel spilled); x comes as planes (Planes, row-major), brought to one
+// exponent per batch row over the split.  lm_head 151936 x 2048 at batch 32
+// 133-134 us, against 160-166 with the x fragments reloaded for every tile.
 template <uint32_t T>
 __global__ __launch_bounds__(512) void quant_gemm_xs32(const uint8_t *__restrict__ W, Planes xp,
                                                        float *__restrict__ out, int m, int n, int batch,
@@ -2832,7 +2703,7 @@ __global__ __launch_bounds__(512) void quant_gemm_xs32(const uint8_t *__restrict
     const int G = gridDim.x, ks = blockIdx.y;
     const int nsb = n >> 8, tiles = (m + kWave - 1) / kWave;
     const uint32_t row_bytes = (uint32_t)nsb * QTraits<T>::kSbBytes;
-    const int sb0 = ks * 8 + 2 * q;
+    const int sb0 = ks * 8 + 2 * q;  // past the last super-block: its copy, multiplied by zeros
     const int li = lane & 15, g = lane >> 4;
     int t = blockIdx.x;
     if (t >= tiles) return;  // uniform
@@ -2841,7 +2712,7 @@ __global__ __launch_bounds__(512) void quant_gemm_xs32(const uint8_t *__restrict
         int ln = lane;
         asm volatile("" : "+v"(ln));  // not loop-invariant: the offsets are not kept in registers
         const int rows_left = m - tt * kWave;
-        const uint8_t *base = W + (size_t)tt * kWave * row_bytes + (size_t)(sb0 + hh) * QTraits<T>::kSbBytes;
+        const uint8_t *base = W + (size_t)tt * kWave * row_bytes + (size_t)min(sb0 + hh, nsb - 1) * QTraits<T>::kSbBytes;
 #pragma unroll
         for (int j = 0; j < V; j++) {
             const int c = j * kWave + ln;
@@ -2853,18 +2724,21 @@ __global__ __launch_bounds__(512) void quant_gemm_xs32(const uint8_t *__restrict
     h8v ah[2][8], al[2][8];
     {
         const int b = min(li + 16 * hh, batch - 1);
-        const int En = xe_max(xp.xe, b, 2 * ks * 8, 16, n);
+        const int En = xe_max(xp.xe, b, 2 * ks * 8, min(16, 2 * (nsb - ks * 8)), n);
         if (q == 0 && g == 0) xeE[li + 16 * hh] = En;
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            const int8_t *e = xp.xe + (size_t)b * xe_stride(n) + 2 * (sb0 + s);
+            const int sb = min(sb0 + s, nsb - 1);
+            const int8_t *e = xp.xe + (size_t)b * xe_stride(n) + 2 * sb;
+            const bool on = sb0 + s < nsb;
             const _Float16 f0 = xe_factor(e[0], En), f1 = xe_factor(e[1], En);
+            const h8v zero = {};
 #pragma unroll
             for (int blk = 0; blk < 8; blk++) {
-                const size_t xo = (size_t)b * n + (size_t)(sb0 + s) * 256 + 32 * blk + 8 * g;
+                const size_t xo = (size_t)b * n + (size_t)sb * 256 + 32 * blk + 8 * g;
                 const _Float16 f = blk < 4 ? f0 : f1;
-                ah[s][blk] = *reinterpret_cast<const h8v *>(xp.hi + xo) * f;
-                al[s][blk] = *reinterpret_cast<const h8v *>(xp.lo + xo) * f;
+                ah[s][blk] = on ? *reinterpret_cast<const h8v *>(xp.hi + xo) * f : zero;
+                al[s][blk] = on ? *reinterpret_cast<const h8v *>(xp.lo + xo) * f : zero;
             }
         }
     }
@@ -2996,29 +2870,17 @@ int dispatch_fused(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t 
     }
 }
 
-template <uint32_t T, int NT>
-int launch_mfma(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m, uint32_t n, const Planes &xp,
-                uint32_t batch, float *out, size_t split_stride, int ksplit) {
-    const int tiles = (int)((m + kWave - 1) / kWave);
-    const int per = split_len((int)(n / 256), ksplit);
-    hipLaunchKernelGGL((quant_gemm_mfma<T, NT>), dim3(tiles, ksplit), dim3(kWave * kWavesPerWg), 0, stream,
-                       static_cast<const uint8_t *>(w), xp, out, (int)m, (int)n, (int)batch, per, split_stride);
-    ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-    return ANEHIP_OK;
-}
-
 template <uint32_t T>
 int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m, uint32_t n, const float *x,
                  uint32_t batch, float *out, int ksplit, _Float16 *xsplit) {
     const size_t split_stride = (size_t)batch * m;
     const int tiles = (int)((m + kWave - 1) / kWave), cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    // many row tiles (at least 4 per CU) with K splits of 8 super-blocks: the
-    // x-stationary kernels, one workgroup per CU walking the row tiles with
-    // the split's x staged once (batch 1: as digits in LDS; batch 2..32: as
-    // MFMA fragments in registers)
-    const bool xs = (int)(n / 256) == 8 * ksplit && tiles >= 4 * cus;
+    // the x-stationary kernels: one workgroup per CU walks the row tiles with
+    // the x of its K split of 8 super-blocks staged once (batch 1, where there
+    // are at least 4 tiles per CU: as digits in LDS; batch 2..32: as MFMA
+    // fragments in registers)
     if (batch == 1) {
-        if (xs) {
+        if ((int)(n / 256) == 8 * ksplit && tiles >= 4 * cus) {
             hipLaunchKernelGGL((gemv_fused_xs<T>), dim3(min(tiles, cus), ksplit), dim3(512), 0, stream,
                                static_cast<const uint8_t *>(w), x, out, (int)m, (int)n, split_stride);
             ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
@@ -3028,8 +2890,26 @@ int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m,
         in.x = x;
         return dispatch_fused<T>(ctx, stream, w, m, n, in, out, ksplit);
     }
-    // batch 2..32: split x into range-safe fp16 hi/lo planes (row-major),
-    // then the MFMA kernel
+    const uint8_t *wb = static_cast<const uint8_t *>(w);
+    // 17..32 rows as two groups of 16 side by side where each workgroup has
+    // one tile to do, or two (the second group's weights come from the L2 or
+    // the MALL)
+    const int groups = batch <= 16 ? 1 : 2;
+    if (batch <= 16 || tiles * ksplit <= cus) {
+        const int work = ksplit * groups;
+        auto rows_tiles = [&](int r) { return (int)((m + r - 1) / r); };
+#define ANEHIP_XS(RS)                                                                                       \
+    hipLaunchKernelGGL((quant_gemm_xs<T, RS>), dim3(min(rows_tiles(16 * RS), cus), ksplit, groups), dim3(512), \
+                       0, stream, wb, x, out, (int)m, (int)n, (int)batch, split_stride)
+        if (rows_tiles(16) * work <= cus) ANEHIP_XS(1);
+        else if (rows_tiles(32) * work <= cus) ANEHIP_XS(2);
+        else ANEHIP_XS(4);
+#undef ANEHIP_XS
+        ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
+        return ANEHIP_OK;
+    }
+    const dim3 grid(min(tiles, cus), ksplit);
+    // 17..32: x split into range-safe fp16 hi / lo planes (row-major) first
     const size_t count = (size_t)batch * n;
     Planes xp;
     xp.hi = xsplit;
@@ -3039,37 +2919,10 @@ int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m,
     hipLaunchKernelGGL(split_x_kernel, dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, stream, x, xp, (int)batch,
                        (int)n);
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-    // (lm_head 151936 x 2048 at batch 4 / 16 / 32: 75.6-77.2 / 80.1-82.9 /
-    // 133.4-133.6 us against 95.8-102.8 / 104.7-113.5 / 160.3-166.1 us on
-    // quant_gemm_mfma, graphs of back-to-back launches)
-    if (xs) {
-        const dim3 grid(min(tiles, cus), ksplit);
-        const uint8_t *wb = static_cast<const uint8_t *>(w);
-        if (batch <= 16)
-            hipLaunchKernelGGL((quant_gemm_xs<T>), grid, dim3(512), 0, stream, wb, xp, out, (int)m, (int)n,
-                               (int)batch, split_stride);
-        else
-            hipLaunchKernelGGL((quant_gemm_xs32<T>), grid, dim3(512), 0, stream, wb, xp, out, (int)m, (int)n,
-                               (int)batch, split_stride);
-        ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-        return ANEHIP_OK;
-    }
-    if (batch <= 16) return launch_mfma<T, 1>(ctx, stream, w, m, n, xp, batch, out, split_stride, ksplit);
-    // 17..32 rows: a matrix that stays in the 256 MiB MALL takes two 16-row
-    // passes (the second reads the weights from the MALL), a larger one the
-    // 32-row kernel.  Measured on MI355X (graphs of back-to-back launches):
-    // 6144 x 2048 at 32 rows 24.7 us in one 32-row pass against 9.3 us for
-    // one 16-row pass.
-    if ((double)m * (n / 32) * QTraits<T>::kBlockBytes <= 128.0 * (1 << 20)) {
-        int rc = launch_mfma<T, 1>(ctx, stream, w, m, n, xp, 16, out, split_stride, ksplit);
-        if (rc) return rc;
-        Planes x2;
-        x2.hi = xp.hi + (size_t)16 * n;
-        x2.lo = xp.lo + (size_t)16 * n;
-        x2.xe = xp.xe + (size_t)16 * xe_stride((int)n);
-        return launch_mfma<T, 1>(ctx, stream, w, m, n, x2, batch - 16, out + (size_t)16 * m, split_stride, ksplit);
-    }
-    return launch_mfma<T, 2>(ctx, stream, w, m, n, xp, batch, out, split_stride, ksplit);
+    hipLaunchKernelGGL((quant_gemm_xs32<T>), grid, dim3(512), 0, stream, wb, xp, out, (int)m, (int)n, (int)batch,
+                       split_stride);
+    ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
+    return ANEHIP_OK;
 }
 
 }  // namespace
@@ -3585,7 +3438,7 @@ int launch_gemv_fused(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, c
 int launch_gemm_raw(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w, uint32_t m, uint32_t n,
                     const float *x, uint32_t batch, float *out, int ksplit, void *xsplit) {
     _Float16 *xs = static_cast<_Float16 *>(xsplit);
-    if (batch > 1 && !xs) return set_error(ctx->err, ANEHIP_EINVAL, "gemm: batch > 1 needs an x split buffer");
+    if (batch > 16 && !xs) return set_error(ctx->err, ANEHIP_EINVAL, "gemm: batch > 16 needs an x split buffer");
     if (ggml_type == ANEHIP_GGML_Q8_0)
         return dispatch_raw<ANEHIP_GGML_Q8_0>(ctx, stream, w, m, n, x, batch, out, ksplit, xs);
     return dispatch_raw<ANEHIP_GGML_Q4_0>(ctx, stream, w, m, n, x, batch, out, ksplit, xs);
@@ -3616,14 +3469,14 @@ int launch_quant_gemm(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, c
                       uint32_t n, const float *x, uint32_t batch, float *y) {
     // the sum_partials consumer takes any number of splits, so the batch-1
     // kernel never needs more than kMaxSliceSb super-blocks per split
-    const int ksplit = gemm_ksplit(ctx, m, n, batch == 1 ? 1 << 20 : kMaxSplit);
+    const int ksplit = batch == 1 ? gemm_ksplit(ctx, m, n, 1 << 20) : (int)((n / 256 + 7) / 8);
     const size_t count = (size_t)batch * m;
     // workspace: [ksplit partials][x hi/lo planes (2 * batch * n halves)][group exponents]
-    const size_t part = ksplit > 1 ? (size_t)ksplit * count : 0;
-    const size_t xs_floats = batch > 1 ? (size_t)batch * n + (xe_bytes(n) + 3) / 4 : 0;
+    const size_t part = ksplit > 1 ? ((size_t)ksplit * count + 3) & ~(size_t)3 : 0;
+    const size_t xs_floats = batch > 16 ? (size_t)batch * n + (xe_bytes(n) + 3) / 4 : 0;
     int rc = ensure_workspace(ctx, part + xs_floats);
     if (rc) return rc;
-    void *xs = batch > 1 ? static_cast<void *>(ctx->ws.partial + part) : nullptr;
+    void *xs = batch > 16 ? static_cast<void *>(ctx->ws.partial + part) : nullptr;
     if (ksplit == 1) return launch_gemm_raw(ctx, stream, ggml_type, w, m, n, x, batch, y, 1, xs);
     rc = launch_gemm_raw(ctx, stream, ggml_type, w, m, n, x, batch, ctx->ws.partial, ksplit, xs);
     if (rc) return rc;

@@ -75,7 +75,7 @@ def test_gemv_parity(gpu_ctx, oracle_lib, t, m, n):
 @pytest.mark.parametrize("m,n", [(6144, 2048), (2048, 6144)])
 def test_small_batch_gemm_parity(gpu_ctx, oracle_lib, t, batch, m, n):
     """Ragged batches: batch is not padded to any tile; rows are read exactly
-    (17 and 32 rows: two 16-row passes, the second of 1 or 16 rows)."""
+    (17 and 32 rows: two groups of 16, the second with 1 or 16 rows)."""
     w = oracle_lib.gen_quant(t, 77, m + n + t, m, n, std=0.02)
     x = oracle_lib.normal(77, 1000 + batch, batch * n).reshape(batch, n)
     y = _run(gpu_ctx, t, w, m, n, x)
@@ -83,6 +83,29 @@ def test_small_batch_gemm_parity(gpu_ctx, oracle_lib, t, batch, m, n):
     l2, mx = rel_errs(y, ref)
     print(f"type={t} m={m} n={n} batch={batch}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
     assert l2 <= TOL and mx <= TOL
+
+
+@pytest.mark.parametrize("t", [8, 2])
+@pytest.mark.parametrize("m,n,batch", [(1, 256, 2), (17, 2304, 16), (33, 4352, 17), (4100, 2048, 9), (4113, 512, 31),
+                                       (8200, 1792, 5), (8255, 2048, 32), (16400, 256, 3), (17000, 2304, 20)])
+def test_gguf_gemm_tile_edges(gpu_ctx, oracle_lib, t, m, n, batch):
+    """The GGUF-layout GEMM's tile heights and batch groups: 16-row tiles (one
+    row; one past a tile), 32-row tiles (4100 and 4113 rows: a last tile of 4
+    and 17), 64-row tiles (8200, 8255: 8 and 63), more tiles than CUs (16400:
+    a second tile for one workgroup), super-block counts that leave waves
+    without one (1, 2, 7 of 8; 9 and 17 over 2 and 3 K splits), and 17..32
+    rows as two groups side by side or on the 32-row kernel with a short last
+    K split."""
+    w = oracle_lib.gen_quant(t, 41, m + n + batch, m, n, std=0.02)
+    x = oracle_lib.normal(41, batch, batch * n).reshape(batch, n)
+    dw, dx, dy = gpu_ctx.to_device(w), gpu_ctx.to_device(x), gpu_ctx.alloc(batch * m * 4)
+    gpu_ctx.quant_gemm(t, dw, m, n, dx, batch, dy)
+    y = dy.download(np.float32, batch * m).reshape(batch, m)
+    l2, mx = rel_errs(y, oracle_lib.gemm(t, w, m, n, x))
+    print(f"type={t} m={m} n={n} batch={batch}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
+    assert l2 <= TOL and mx <= TOL
+    for b in (dw, dx, dy):
+        b.free()
 
 
 @pytest.mark.parametrize("t", [8, 2])
