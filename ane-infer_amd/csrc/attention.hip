@@ -25,7 +25,7 @@
 // current position's k/v are rounded to fp16 before use, exactly as if they
 // had been written to the cache and read back (the reference writes first,
 // deltanet.rs:625, then reads every position).
-#include "common.h"
+#include "panel.h"
 
 namespace anehip {
 
@@ -58,16 +58,6 @@ __device__ __forceinline__ void norm_rope_head(const MixIn &mix, int b, int base
     dst[3] = a2 * s1 + a3 * c1;
 }
 
-// Barrier for LDS traffic only: waves do not wait for their outstanding
-// global loads (the next tile's K / V) here.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kWord3 = 0x00020000;  // raw buffer resource word 3 (gfx9 family)
 constexpr float kPScale = 16384.0f;  // 2^14: probabilities in the PV MFMA operands
@@ -80,8 +70,6 @@ constexpr float kPScale = 16384.0f;  // 2^14: probabilities in the PV MFMA opera
 // 1248 / 1241 / 1166 tok/s against 1254 / 1245 / 1130 with it on none.
 constexpr int kCpolNt = 2;
 constexpr size_t kNtKvBytes = (size_t)32 << 20;
-
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // Sharing of the launch's workgroups over sequences of different lengths (2
 // to 64 of them): every chunk gets at most `s` tiles, s the smallest (to 3 %)
@@ -629,6 +617,256 @@ __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const 
     }
 }
 
+// Prefill: T consecutive tokens of one sequence (row t at position pos_arr[t],
+// its K / V row already appended) against the cache.  A workgroup takes 32
+// query rows of one kv head -- 32 / G tokens x the G query heads -- so that the
+// K / V rows they share are read once for all of them; its 4 waves take every
+// fourth tile of 32 positions, each with an online softmax of its own, and
+// merge at the end.  On v_mfma_f32_32x32x16_f16 (operands A[i][k] / B[k][j] in
+// lane i (j) + 32 (k / 8), elements k % 8; D[i][j] in lane j + 32 (i / 4 % 2),
+// element 4 (i / 8) + i % 4), the query row always the lane's column:
+//  * scores S[pos][row] = K q^T / 16: A = 32 K rows straight from the cache, B =
+//    q as range-scaled fp16 hi + lo from LDS;
+//  * O[dim][row] += V^T P^T: the lane's 16 scores of a tile are two steps' B
+//    operand as they are (x 2^14, fp16 hi + lo) if step u's k slot (h, j) means
+//    position 16 u + 8 (j / 4) + 4 h + j % 4; A = V rows loaded as 8-byte pieces
+//    (dims 128 q + 4 i .. + 3), MFMA (q, c) taking element c of the 8 rows' pieces,
+//    so that its row i is dim 128 q + 4 i + c.
+// K and V of the wave's next tile are in flight while a tile is processed
+// (sums 128, K 64 and V 64 registers: one wave per SIMD; q beside them spilled).
+//
+// The decode kernel with one row per workgroup read every position's K / V
+// once per row and ran 4 of 16 MFMA columns: 130 us at 960 rows of 8 heads from
+// position 0 and 158 at 540 from 960 on, plus 17 for its merge; here 39 and 51,
+// 64 MFMAs of 32 cycles per wave and tile, the rest the softmax between the two
+// products, which one wave per SIMD doesn't hide.
+// A row's masked scores weigh 0, but the V rows of later tokens of its group
+// enter the product with that 0: an infinity there shows as a NaN in this row
+// too, and not only in the rows from that token on (whose results it ends
+// anyway, the prompt's logits with them).
+constexpr int kQRows = 32;    // query rows per workgroup
+constexpr int kPTile = 32;    // positions per tile
+constexpr int kMergeF = 66;   // LDS row of the merge: reads along the dims hit all banks
+
+template <int G>
+__global__ __launch_bounds__(kThreads, 1) void attn_prefill_kernel(
+    MixIn mix, const float *__restrict__ q_norm, const float *__restrict__ inv_freq,
+    const uint32_t *__restrict__ pos_arr, const __half *__restrict__ k_cache, const __half *__restrict__ v_cache,
+    size_t cache_off, int max_seq, int n_heads, int T, float *__restrict__ out) {
+    constexpr int QT = kQRows / G;  // tokens per workgroup
+    __shared__ __align__(16) h8v qs[16 * 2 * 64];             // q fragments [k-step][hi, lo][lane]
+    __shared__ __align__(16) float lds[4 * 4 * 16 * kMergeF];  // the merge's [wave][c][element][lane]
+    __shared__ int qexp[kQRows];
+    __shared__ float wm[4][kQRows], wl[4][kQRows];
+    const int t = threadIdx.x, lane = t & 63, col = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // the last tokens see the most positions: they go first
+    const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * QT, kvh = blockIdx.y;
+    const size_t base = cache_off + (size_t)kvh * max_seq * kHd;
+    const int last = (int)pos_arr[min(t0 + QT, T) - 1], plim = (int)pos_arr[min(t0 + col / G, T - 1)];
+    const int tiles = last / kPTile + 1;
+    const __amdgpu_buffer_rsrc_t krs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(k_cache) + base, 0, (last + 1) * kHd * 2, kWord3);
+    const __amdgpu_buffer_rsrc_t vrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(v_cache) + base, 0, (last + 1) * kHd * 2, kWord3);
+    u32x4 kr[16];
+    u32x2 vr[2][2][8];  // [step][q][slot]
+    // positions past `last` read zeros without a memory access
+    auto load_k = [&](int ti) {
+#pragma unroll
+        for (int s = 0; s < 16; s++)
+            kr[s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  krs, ((ti * kPTile + col) * kHd + 16 * s + 8 * h) * 2, 0, 0));
+    };
+    auto load_v = [&](int ti) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+                    vr[u][q][j] = __builtin_bit_cast(
+                        u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                                   vrs, ((ti * kPTile + 16 * u + 8 * (j >> 2) + 4 * h + (j & 3)) * kHd + 128 * q + 4 * col) * 2,
+                                   0, 0));
+    };
+    load_k(wave);
+    load_v(wave);
+    // wave w normalises and rotates query rows 8 w .. + 7 (every row's loads
+    // first, one sincos per rotary pair and token) and writes their B
+    // fragments (scaled by 1/16 and 2^-qe, fp16 hi + lo)
+    constexpr int QR = kQRows / 4;
+    float4 xq[QR];
+    auto row_in = [&](int i) {
+        const int r = QR * wave + i, tok = min(t0 + r / G, T - 1);
+        return mix.p + (size_t)tok * mix.stride + (kvh * G + r % G) * 2 * kHd + 4 * lane;
+    };
+#pragma unroll
+    for (int i = 0; i < QR; i++) xq[i] = *reinterpret_cast<const float4 *>(row_in(i));
+    for (int q = 1; q < mix.kp; q++)
+#pragma unroll
+        for (int i = 0; i < QR; i++) {
+            const float4 v = *reinterpret_cast<const float4 *>(row_in(i) + (size_t)q * mix.split);
+            xq[i] = make_float4(xq[i].x + v.x, xq[i].y + v.y, xq[i].z + v.z, xq[i].w + v.w);
+        }
+    const float4 wv = *reinterpret_cast<const float4 *>(q_norm + 4 * lane);
+    const float2 fr = *reinterpret_cast<const float2 *>(inv_freq + 2 * lane);
+    float sn0 = 0.0f, cs0 = 0.0f, sn1 = 0.0f, cs1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < QR; i++) {
+        const int r = QR * wave + i;
+        if (i % G == 0) {
+            const float fpos = (float)pos_arr[min(t0 + r / G, T - 1)];
+            sincosf(fpos * fr.x, &sn0, &cs0);
+            sincosf(fpos * fr.y, &sn1, &cs1);
+        }
+        // norm_rope_head's arithmetic
+        const float4 x4 = xq[i];
+        const float inv_rms =
+            rsqrtf(wave_sum(x4.x * x4.x + x4.y * x4.y + x4.z * x4.z + x4.w * x4.w) / (float)kHd + 1e-6f);
+        const float a0 = (x4.x * inv_rms) * wv.x, a1 = (x4.y * inv_rms) * wv.y;
+        const float a2 = (x4.z * inv_rms) * wv.z, a3 = (x4.w * inv_rms) * wv.w;
+        const float q4[4] = {a0 * cs0 - a1 * sn0, a0 * sn0 + a1 * cs0, a2 * cs1 - a3 * sn1, a2 * sn1 + a3 * cs1};
+        const float qm = wave_max64(fmaxf(fmaxf(fabsf(q4[0]), fabsf(q4[1])), fmaxf(fabsf(q4[2]), fabsf(q4[3]))));
+        const int qe = group_exp(qm * 0.0625f);
+        if (lane == 0) qexp[r] = qe;
+        h4v hi, lo;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float x = ldexpf(q4[c] * 0.0625f, -qe);
+            hi[c] = (_Float16)x;
+            lo[c] = (_Float16)(x - (float)hi[c]);
+        }
+        // dims 4 lane .. + 3: k-step lane / 4, lane group (lane % 4) / 2, half lane % 2
+        const int o = (lane >> 2) * 128 + r + 32 * ((lane & 3) >> 1);
+        reinterpret_cast<h4v *>(&qs[o])[lane & 1] = hi;
+        reinterpret_cast<h4v *>(&qs[o + 64])[lane & 1] = lo;
+    }
+    lds_barrier();
+    const int qe = qexp[col];
+    float m_run = -INFINITY, l_run = 0.0f;
+    f32x16 o[2][4] = {};  // [q][c]: dims 128 q + 4 i + c
+    for (int ti = wave; ti < tiles; ti += 4) {
+        asm volatile("" ::: "memory");  // q is read again for every tile, not kept in registers
+        // two steps' q fragments are read while the two before are multiplied
+        f32x16 sc = {}, sl = {};
+        h8v qa[2][4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) qa[0][i] = qs[i * 64 + lane];
+#pragma unroll
+        for (int s = 0; s < 16; s += 2) {
+            const int k = (s >> 1) & 1;
+            if (s < 14) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) qa[k ^ 1][i] = qs[(2 * s + 4 + i) * 64 + lane];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const h8v a = __builtin_bit_cast(h8v, kr[s + i]);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qa[k][2 * i], sc, 0, 0, 0);
+                sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qa[k][2 * i + 1], sl, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        load_k(ti + 4);
+        float tm = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int pos = ti * kPTile + 8 * (e >> 2) + 4 * h + (e & 3);
+            sc[e] = pos <= plim ? ldexpf(sc[e] + sl[e], qe) : -INFINITY;
+            tm = fmaxf(tm, sc[e]);
+        }
+        const float mn = fmaxf(m_run, lanes_max2(tm));
+        const float mref = mn == -INFINITY ? 0.0f : mn;
+        const float scale = expf(m_run - mref);
+        float ps = 0.0f;
+        h8v ph[2], pl[2];
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const float pe = expf(sc[e] - mref);
+            ps += pe;
+            const float x = pe * kPScale;
+            ph[e >> 3][e & 7] = (_Float16)x;
+            pl[e >> 3][e & 7] = (_Float16)(x - (float)ph[e >> 3][e & 7]);
+        }
+        l_run = l_run * scale + lanes_sum2(ps);
+        // the sums need scaling only where a row's maximum moved
+        if (__ballot(mn != m_run)) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) o[k >> 2][k & 3] *= scale;
+        }
+        m_run = mn;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    u32x4 w;
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        w[k] = __builtin_amdgcn_perm(vr[u][q][2 * k + 1][c >> 1], vr[u][q][2 * k][c >> 1],
+                                                     c & 1 ? 0x07060302u : 0x05040100u);
+                    const h8v a = __builtin_bit_cast(h8v, w);
+                    o[q][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph[u], o[q][c], 0, 0, 0);
+                    o[q][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[u], o[q][c], 0, 0, 0);
+                }
+        load_v(ti + 4);
+    }
+    // merge: every wave's sums times exp(m - M) / L of the row, added over the
+    // waves 128 dims at a time, times sigmoid(gate) (deltanet.rs:667-669).
+    // Thread (i = t % 32) finishes dims 128 q + 4 i .. + 3 of rows t / 32 + 8 k;
+    // its gates are loaded ahead of the exchange.
+    const int mi = t & 31;
+    float4 gate[2][kQRows / 8];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int k = 0; k < kQRows / 8; k++) {
+            const int r = (t >> 5) + 8 * k;
+            gate[q][k] = mix.at4(min(t0 + r / G, T - 1), (kvh * G + r % G) * 2 * kHd + kHd + 128 * q + 4 * mi);
+        }
+    if (h == 0) {
+        wm[wave][col] = m_run;
+        wl[wave][col] = l_run;
+    }
+    lds_barrier();
+    float M = wm[0][col];
+#pragma unroll
+    for (int w = 1; w < 4; w++) M = fmaxf(M, wm[w][col]);
+    float L = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) L += expf(wm[w][col] - M) * wl[w][col];
+    const float f = expf(m_run - M) / (L * kPScale);
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        if (q) lds_barrier();  // the first half's sums were read
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) lds[((wave * 4 + c) * 16 + e) * kMergeF + lane] = o[q][c][e] * f;
+        lds_barrier();
+#pragma unroll
+        for (int k = 0; k < kQRows / 8; k++) {
+            const int r = (t >> 5) + 8 * k, tok = t0 + r / G, head = kvh * G + r % G;
+            const int at = ((mi >> 3) * 4 + (mi & 3)) * kMergeF + r + 32 * ((mi >> 2) & 1);
+            float v[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                v[c] = 0.0f;
+#pragma unroll
+                for (int w = 0; w < 4; w++) v[c] += lds[(w * 4 + c) * 16 * kMergeF + at];
+            }
+            const float4 g = gate[q][k];
+            if (tok < T)
+                *reinterpret_cast<float4 *>(out + ((size_t)tok * n_heads + head) * kHd + 128 * q + 4 * mi) =
+                    make_float4(v[0] * (1.0f / (1.0f + expf(-g.x))), v[1] * (1.0f / (1.0f + expf(-g.y))),
+                                v[2] * (1.0f / (1.0f + expf(-g.z))), v[3] * (1.0f / (1.0f + expf(-g.w))));
+        }
+    }
+}
+
 // Chunks per (sequence, kv head): at most 128, at most one per 64-position
 // tile of the cache, and about one workgroup per CU over the launch
 // (kAttnWorkgroups / (batch x kv heads): batch 32 with 2 kv heads 4 chunks,
@@ -720,10 +958,27 @@ int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int 
     hipLaunchKernelGGL(attn_append_kernel, dim3(n_kv, rows), dim3(64), 0, stream, mix, k_norm, inv_freq, pos, k_cache,
                        v_cache, cache_off, max_seq, n_heads, n_kv);
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-    if (int rc = attention_impl(ctx, stream, rows, n_heads, n_kv, max_seq, mix, q_norm, k_norm, inv_freq, pos, k_cache,
-                                v_cache, part, out, xp.uniform ? Planes{} : xp, cache_off, 0, false))
-        return rc;
-    return xp.uniform ? launch_split_rows(ctx, stream, out, (uint32_t)rows, (uint32_t)(n_heads * kHd), xp) : ANEHIP_OK;
+    if ((size_t)max_seq * kHd * 2 >= (size_t)1 << 30)
+        return set_error(ctx->err, ANEHIP_EUNSUPPORTED, "attention: max_seq %d too large", max_seq);
+    // few rows: one workgroup of the decode kernel per row and kv head has less
+    // to set up (16 rows from position 0: 8.8 + 4.1 us with its merge, against
+    // 23.8 + 4.6 with the planes' launch); above, both sides' launches are those
+    // of the uniform planes, and 33 rows of a 4-layer model take 535 us against 659
+    if (rows <= kPrefillFewRows && !xp.uniform)
+        return attention_impl(ctx, stream, rows, n_heads, n_kv, max_seq, mix, q_norm, k_norm, inv_freq, pos, k_cache,
+                              v_cache, part, nullptr, xp, cache_off, 0, false);
+    const int G = n_heads / n_kv;
+#define ANEHIP_ATTN_PREFILL(GG)                                                                                      \
+    hipLaunchKernelGGL(attn_prefill_kernel<GG>, dim3((rows * GG + kQRows - 1) / kQRows, n_kv), dim3(kThreads), 0,     \
+                       stream, mix, q_norm, inv_freq, pos, k_cache, v_cache, cache_off, max_seq, n_heads, rows, out)
+    if (G == 4) ANEHIP_ATTN_PREFILL(4);
+    else if (G == 2) ANEHIP_ATTN_PREFILL(2);
+    else if (G == 1) ANEHIP_ATTN_PREFILL(1);
+    else return set_error(ctx->err, ANEHIP_EUNSUPPORTED, "attention: %d query heads per kv head (1, 2 or 4)", G);
+#undef ANEHIP_ATTN_PREFILL
+    ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
+    return xp.uniform ? launch_split_rows(ctx, stream, out, (uint32_t)rows, (uint32_t)(n_heads * kHd), xp)
+                      : launch_split_x(ctx, stream, out, (uint32_t)rows, (uint32_t)(n_heads * kHd), xp);
 }
 
 }  // namespace anehip

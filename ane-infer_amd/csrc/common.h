@@ -391,6 +391,11 @@ __device__ __forceinline__ float lanes_max2(float v) {
     const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
 }
+__device__ __forceinline__ float lanes_sum2(float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __builtin_bit_cast(float, (uint32_t)b[0]) + __builtin_bit_cast(float, (uint32_t)b[1]);
+}
 __device__ __forceinline__ float lanes_max4(float v) {
     const uint32_t u = __builtin_bit_cast(uint32_t, v);
     const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
@@ -525,7 +530,8 @@ int launch_deltanet_head(anehip_ctx *ctx, hipStream_t stream, int batch, int n_h
 // sequence's block S) carried over the chunks, raw head outputs to heads
 // [rows][dim] (scratch); row t's gated RMSNorm to the planes (uniform ones by
 // way of heads) and the conv windows (the sequence's block conv_state)
-// advanced by the rows.
+// advanced by the rows.  Up to 32 rows are scanned token by token (scratch of
+// 386 floats per row and head).
 constexpr size_t kDnChunkFloats = 4 * 64 * 128 + 64 * 64 + 64;
 int launch_deltanet_scan(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, const MixIn &mix,
                          const MixIn &beta, const MixIn &alpha, const float *conv_w, const float *ssm_a,
@@ -552,8 +558,11 @@ int launch_attention(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads
 // Prefill of `rows` consecutive tokens of one sequence (row t at position
 // pos[t], q / k / v in mix row t): appends every row's k / v to the cache at
 // cache_off (halves; the sequence's [kv_head][max_seq][256] block), then
-// attends row t over positions [0, pos[t]] and writes fragment-order planes
-// (uniform ones by way of out, [rows][n_heads * 256] fp32).
+// attends row t over positions [0, pos[t]]: out [rows][n_heads * 256] fp32
+// (scratch), then its fragment-order planes.  Up to kPrefillFewRows rows into
+// planes that are not uniform run on the decode kernel instead, with part as
+// its scratch (attn_partial_floats of up to as many rows).
+constexpr int kPrefillFewRows = 32;
 int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, int n_kv, int max_seq,
                              const MixIn &mix, const float *q_norm, const float *k_norm, const float *inv_freq,
                              const uint32_t *pos, __half *k_cache, __half *v_cache, size_t cache_off, float *part,

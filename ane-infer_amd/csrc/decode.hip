@@ -678,11 +678,8 @@ int alloc_prefill(anehip_ctx *ctx, Model *M) {
     const size_t d = D.dim;
     const size_t part = prefill_part_floats(ctx, M);
     size_t attn = 0;
-    if (M->rows_attn) {
-        const int G = (int)(D.n_heads / D.n_kv_heads);
-        for (uint32_t r = 1; r <= kPrefillRows; r++)
-            attn = std::max(attn, attn_partial_floats((int)r, (int)D.n_kv_heads, (int)M->max_seq, G));
-    }
+    for (int r = 1; M->rows_attn && r <= kPrefillFewRows; r++)
+        attn = std::max(attn, attn_partial_floats(r, (int)D.n_kv_heads, (int)M->max_seq, (int)(D.n_heads / D.n_kv_heads)));
     struct {
         void **p;
         size_t bytes;

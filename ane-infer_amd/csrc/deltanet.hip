@@ -460,84 +460,102 @@ __device__ __forceinline__ f32x4 mma16(f32x4 a, f32x4 b, f32x4 c) {
     return c;
 }
 
-// grid = (chunks of 64 tokens, n_heads), 256 threads.  Conv + SiLU over the
+// grid = (chunks of 64 tokens, n_heads), 512 threads.  Conv + SiLU over the
 // tokens' windows (conv_shift_and_append + conv_apply, deltanet_cache.rs:34-54),
 // L2 norms of q and k (deltanet.rs:25-31, 461-467), beta and decay
 // (deltanet.rs:474-480), then the products above.  Tokens past T have k = q =
-// v = 0, beta 0 and decay 1: they change nothing.
+// v = 0, beta 0 and decay 1: they change nothing, and 16-token tiles of them
+// are skipped (zeros).  Bound by its chain of stages, one workgroup per CU:
+// 36 us for 15 chunks of 16 heads on 4 waves, 32 on 8, a wave per 16 x 16
+// tile row and half.
+constexpr int kChunkThreads = 512;
 template <int KP>
-__global__ __launch_bounds__(kThreads) void dn_chunk_kernel(MixIn mix, MixIn mbeta, MixIn malpha,
-                                                            const float *__restrict__ conv_w,
-                                                            const float *__restrict__ ssm_a,
-                                                            const float *__restrict__ dt_bias,
-                                                            const float *__restrict__ cs, float *__restrict__ scr,
-                                                            int n_heads, int T) {
+__global__ __launch_bounds__(kChunkThreads) void dn_chunk_kernel(MixIn mix, MixIn mbeta, MixIn malpha,
+                                                                 const float *__restrict__ conv_w,
+                                                                 const float *__restrict__ ssm_a,
+                                                                 const float *__restrict__ dt_bias,
+                                                                 const float *__restrict__ cs,
+                                                                 float *__restrict__ scr, int n_heads, int T) {
     __shared__ __align__(16) float qkv[3][kCt * kRowF];
     __shared__ __align__(16) float tri[2][kCt * kTriF];  // D, then X; L
     __shared__ float sb[kCt], sg[kCt], sd[kCt];          // beta, g, D_63
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, lg = lane >> 4;
+    const int t = threadIdx.x, lane = t & 63, li = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int c0 = blockIdx.x * kCt, h = blockIdx.y, chunk = n_heads * kDk;
+    const int nt = (min(kCt, T - c0) + 15) >> 4;  // 16-token tiles that hold a token
     float *out = scr + ((size_t)blockIdx.x * n_heads + h) * kDnChunkFloats;
     float *Q = qkv[0], *K = qkv[1], *V = qkv[2];
 
-    // conv: thread (channel t % 128, token half t / 128) walks its 32 tokens
-    // of q, k and v with the window in registers, 8 loads in flight
-    const int ch = t & (kDk - 1), b0 = c0 + (t >> 7) * (kCt / 2);
-#pragma unroll
-    for (int p = 0; p < 3; p++) {
-        const int gch = p * chunk + h * kDk + ch;
-        const f32x4 old = *reinterpret_cast<const f32x4 *>(cs + (size_t)gch * kKsize);
-        const f32x4 kw = *reinterpret_cast<const f32x4 *>(conv_w + (size_t)gch * kKsize);
-        float w[3][KP], x[3];
-#pragma unroll
-        for (int i = 0; i < 3; i++) mix.load<KP>(min(max(b0 - 3 + i, 0), T - 1), gch, w[i]);
-#pragma unroll
-        for (int i = 0; i < 3; i++) x[i] = b0 - 3 + i >= 0 ? mix.add<KP>(w[i]) : old[(b0 + 1 + i) & 3];
-        for (int i0 = 0; i0 < kCt / 2; i0 += 8) {
-            float v[8][KP];
-#pragma unroll
-            for (int i = 0; i < 8; i++) mix.load<KP>(min(b0 + i0 + i, T - 1), gch, v[i]);
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const float xn = mix.add<KP>(v[i]);
-                float y = 0.0f;
-                y += x[0] * kw.x;
-                y += x[1] * kw.y;
-                y += x[2] * kw.z;
-                y += xn * kw.w;
-                qkv[p][(b0 - c0 + i0 + i) * kRowF + ch] = b0 + i0 + i < T ? silu_ref(y) : 0.0f;
-                x[0] = x[1];
-                x[1] = x[2];
-                x[2] = xn;
-            }
-        }
-    }
-    if (wave == 0) {
-        // lane = token: beta, decay; then column s = lane of D
+    // each wave: lane = token: beta, decay; its 2 nt rows of D (lane = column)
+    {
         const int b = min(c0 + lane, T - 1);
         float xb[KP], xa[KP];
         mbeta.load<KP>(b, h, xb);
         malpha.load<KP>(b, h, xa);
+        // conv: thread (channel t % 128, token quarter t / 128) walks its 4 nt
+        // tokens of q, k and v with the window in registers, the next 4
+        // tokens' loads in flight
+        const int ch = t & (kDk - 1), b0 = c0 + (t >> 7) * 4 * nt;
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            const int gch = p * chunk + h * kDk + ch;
+            const f32x4 old = *reinterpret_cast<const f32x4 *>(cs + (size_t)gch * kKsize);
+            const f32x4 kw = *reinterpret_cast<const f32x4 *>(conv_w + (size_t)gch * kKsize);
+            float w[3][KP], v[2][4][KP], x[3];
+            auto load4 = [&](float (&d)[4][KP], int k) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) mix.load<KP>(min(b0 + 4 * k + i, T - 1), gch, d[i]);
+            };
+#pragma unroll
+            for (int i = 0; i < 3; i++) mix.load<KP>(min(max(b0 - 3 + i, 0), T - 1), gch, w[i]);
+            load4(v[0], 0);
+#pragma unroll
+            for (int i = 0; i < 3; i++) x[i] = b0 - 3 + i >= 0 ? mix.add<KP>(w[i]) : old[(b0 + 1 + i) & 3];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (k >= nt) break;
+                if (k + 1 < nt) load4(v[(k + 1) & 1], k + 1);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float xn = mix.add<KP>(v[k & 1][i]);
+                    float y = 0.0f;
+                    y += x[0] * kw.x;
+                    y += x[1] * kw.y;
+                    y += x[2] * kw.z;
+                    y += xn * kw.w;
+                    const int tok = b0 + 4 * k + i;
+                    qkv[p][(tok - c0) * kRowF + ch] = tok < T ? silu_ref(y) : 0.0f;
+                    x[0] = x[1];
+                    x[1] = x[2];
+                    x[2] = xn;
+                }
+            }
+        }
         const bool in = c0 + lane < T;
         const float alpha = in ? expf(ssm_a[h] * logf(1.0f + expf(malpha.add<KP>(xa) + dt_bias[h]))) : 1.0f;
-        sb[lane] = in ? 1.0f / (1.0f + expf(-mbeta.add<KP>(xb))) : 0.0f;
+        const float beta = in ? 1.0f / (1.0f + expf(-mbeta.add<KP>(xb))) : 0.0f;
         const int ai = __builtin_bit_cast(int, alpha);
         const float a0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, 0));
         float p = 1.0f;
-#pragma unroll
-        for (int i = 0; i < kCt; i++) {
+        for (int i = 0; i < 2 * nt * (wave + 1); i++) {
             const float a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, i));
             p = i > lane ? p * a : 1.0f;
-            tri[0][i * kTriF + lane] = i >= lane ? p : 0.0f;
-            if (lane == 0) sg[i] = a0 * p;
+            if (i >= 2 * nt * wave) {
+                tri[0][i * kTriF + lane] = i >= lane ? p : 0.0f;
+                if (lane == 0) sg[i] = a0 * p;
+            }
         }
-        sd[lane] = p;
+        if (wave == 7) {
+            sd[lane] = p;
+            sb[lane] = beta;
+        }
     }
     __syncthreads();
     // L2 norms: 16 lanes per token, 8 columns each, 4 tokens of a wave at a time
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const int o = (16 * wave + 4 * it + lg) * kRowF + 8 * li;
+    for (int it = 0; it < 2; it++) {
+        const int tok = 8 * wave + 4 * it + lg, o = tok * kRowF + 8 * li;
+        if (8 * wave >= 16 * nt) break;
 #pragma unroll
         for (int p = 0; p < 2; p++) {
             f32x4 *r = reinterpret_cast<f32x4 *>(&qkv[p][o]);
@@ -556,18 +574,14 @@ __global__ __launch_bounds__(kThreads) void dn_chunk_kernel(MixIn mix, MixIn mbe
         }
     }
     __syncthreads();
-    // the 10 lower 16 x 16 tiles of K K^T (-> L, LDS) and of Q K^T (-> A), 5 per wave
+    // the lower 16 x 16 tiles of K K^T (-> L, LDS), all waves, then of Q K^T
+    // (-> A) by waves 4-7 while waves 0-3 invert L's diagonal blocks
     auto tile_of = [](int p, int &i, int &j) {
         i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3;
         j = p - i * (i + 1) / 2;
     };
-#pragma unroll
-    for (int n = 0; n < 5; n++) {
-        const int p = wave + 4 * n;
-        const bool kk = p < 10;
-        int i, j;
-        tile_of(kk ? p : p - 10, i, j);
-        const float *ra = (kk ? K : Q) + (16 * i + li) * kRowF + 4 * lg, *rb = K + (16 * j + li) * kRowF + 4 * lg;
+    auto gram = [&](const float *rows, int i, int j) {
+        const float *ra = rows + (16 * i + li) * kRowF + 4 * lg, *rb = K + (16 * j + li) * kRowF + 4 * lg;
         f32x4 s0 = {}, s1 = {};
 #pragma unroll
         for (int q = 0; q < 8; q += 2) {
@@ -575,34 +589,40 @@ __global__ __launch_bounds__(kThreads) void dn_chunk_kernel(MixIn mix, MixIn mbe
             s1 = mma16(*reinterpret_cast<const f32x4 *>(ra + 16 * q + 16),
                        *reinterpret_cast<const f32x4 *>(rb + 16 * q + 16), s1);
         }
+        s0 += s1;
+#pragma unroll
+        for (int e = 0; e < 4; e++) s0[e] *= tri[0][(16 * i + 4 * lg + e) * kTriF + 16 * j + li];
+        return s0;
+    };
+    const int pairs = nt * (nt + 1) / 2;
+    for (int p = wave; p < pairs; p += 8) {
+        int i, j;
+        tile_of(p, i, j);
+        const f32x4 v = gram(K, i, j);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int r = 16 * i + 4 * lg + e, c = 16 * j + li;
-            const float v = (s0[e] + s1[e]) * tri[0][r * kTriF + c];
-            if (kk) tri[1][r * kTriF + c] = c < r ? sb[r] * v : 0.0f;
-            else out[kOffA + r * kCt + c] = c <= r ? v : 0.0f;
+            tri[1][r * kTriF + c] = c < r ? sb[r] * v[e] : 0.0f;
         }
     }
-    // A's upper tiles are zero
-    for (int e = t; e < 6 * 64; e += kThreads) {
-        const int p = e >> 6, i = p < 3 ? 0 : p < 5 ? 1 : 2, j = p < 3 ? p + 1 : p < 5 ? p - 1 : 3;
-        *reinterpret_cast<f32x4 *>(out + kOffA + (16 * i + ((e & 63) >> 2)) * kCt + 16 * j + 4 * (e & 3)) = f32x4{};
-    }
-    // g Q and (D_63 K)^T
-    for (int e = t; e < kCt * kDk / 4; e += kThreads) {
-        const int r = e >> 5, c = 4 * (e & 31);
-        const f32x4 q = *reinterpret_cast<const f32x4 *>(Q + r * kRowF + c);
-        *reinterpret_cast<f32x4 *>(out + kOffQ + r * kDk + c) = q * sg[r];
-    }
-    for (int i = wave; i < kDk; i += 4) out[kOffK + i * kCt + lane] = sd[lane] * K[lane * kRowF + i];
-    if (t == 0) out[kOffG] = sg[kCt - 1];
-    __syncthreads();  // L is whole, D no longer needed
+    __syncthreads();  // L is whole
     float *X = tri[0];
     const float *L = tri[1];
-    // X's diagonal blocks by forward substitution: wave w block w, lane column
-    // s = li: x_t = [t = s] - sum_{r<t} L_tr x_r
-    {
-        float x[16];
+    float x[16];
+    if (wave >= 4) {
+        for (int p = wave - 4; p < pairs; p += 4) {
+            int i, j;
+            tile_of(p, i, j);
+            const f32x4 v = gram(Q, i, j);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = 16 * i + 4 * lg + e, c = 16 * j + li;
+                out[kOffA + r * kCt + c] = c <= r ? v[e] : 0.0f;
+            }
+        }
+    } else if (wave < nt) {
+        // X's diagonal blocks by forward substitution: wave w block w, lane
+        // column s = li: x_t = [t = s] - sum_{r<t} L_tr x_r
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             float p[4] = {r == li ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f};
@@ -615,18 +635,34 @@ __global__ __launch_bounds__(kThreads) void dn_chunk_kernel(MixIn mix, MixIn mbe
             }
             x[r] = (p[0] + p[1]) + (p[2] + p[3]);
         }
-        if (lg == 0)
-#pragma unroll
-            for (int r = 0; r < 16; r++) X[(16 * wave + r) * kTriF + 16 * wave + li] = x[r];
     }
+    // the tiles of A above the diagonal or without tokens are zero
+    for (int e = t; e < 16 * 64; e += kChunkThreads) {
+        const int i = e >> 8, j = (e >> 6) & 3;
+        if (j > i || i >= nt)
+            *reinterpret_cast<f32x4 *>(out + kOffA + (16 * i + ((e & 63) >> 2)) * kCt + 16 * j + 4 * (e & 3)) = f32x4{};
+    }
+    // g Q and (D_63 K)^T (rows without tokens: zeros)
+    for (int e = t; e < kCt * kDk / 4; e += kChunkThreads) {
+        const int r = e >> 5, c = 4 * (e & 31);
+        const f32x4 q = *reinterpret_cast<const f32x4 *>(Q + r * kRowF + c);
+        *reinterpret_cast<f32x4 *>(out + kOffQ + r * kDk + c) = r < 16 * nt ? q * sg[r] : f32x4{};
+    }
+    for (int i = wave; i < kDk; i += 8)
+        out[kOffK + i * kCt + lane] = lane < 16 * nt ? sd[lane] * K[lane * kRowF + i] : 0.0f;
+    if (t == 0) out[kOffG] = sg[16 * nt - 1];
+    __syncthreads();  // D is no longer needed
+    if (wave < nt && lg == 0)
+#pragma unroll
+        for (int r = 0; r < 16; r++) X[(16 * wave + r) * kTriF + 16 * wave + li] = x[r];
     // X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj, one block diagonal at a time
     auto row4 = [&](const float *m, int i, int k) {
         return *reinterpret_cast<const f32x4 *>(m + (16 * i + li) * kTriF + 16 * k + 4 * lg);
     };
-    for (int d = 1; d < 4; d++) {
+    for (int d = 1; d < nt; d++) {
         __syncthreads();
         const int i = wave + d, j = wave;
-        if (i < 4) {
+        if (i < nt) {
             f32x4 p = {};
             for (int k = j; k < i; k++) {
                 f32x4 xb;
@@ -640,32 +676,30 @@ __global__ __launch_bounds__(kThreads) void dn_chunk_kernel(MixIn mix, MixIn mbe
         }
     }
     __syncthreads();
-    // U = X (beta V) and W = X (beta g K): 2 column tiles of each per wave
-    f32x4 xa[10];
+    // U = X (beta V) by waves 0-3, W = X (beta g K) by waves 4-7: 2 column
+    // tiles per wave
+    const float *src = wave < 4 ? V : K;
+    float *dst = out + (wave < 4 ? 0 : kOffW);
 #pragma unroll
-    for (int p = 0; p < 10; p++) {
-        int i, k;
-        tile_of(p, i, k);
-        xa[p] = row4(X, i, k);
-    }
-#pragma unroll
-    for (int n = 0; n < 4; n++) {
-        const float *src = n < 2 ? V : K;
-        float *dst = out + (n < 2 ? 0 : kOffW);
-        const int c = 16 * (2 * wave + (n & 1)) + li;
+    for (int n = 0; n < 2; n++) {
+        const int c = 16 * (2 * (wave & 3) + n) + li;
         f32x4 b[4];
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int k = 0; k < 4; k++) {
+            if (k >= nt) break;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int r = 16 * k + 4 * lg + e;
-                b[k][e] = src[r * kRowF + c] * (n < 2 ? sb[r] : sb[r] * sg[r]);
+                b[k][e] = src[r * kRowF + c] * (wave < 4 ? sb[r] : sb[r] * sg[r]);
             }
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             f32x4 s = {};
+            if (i < nt) {
 #pragma unroll
-            for (int k = 0; k <= i; k++) s = mma16(xa[i * (i + 1) / 2 + k], b[k], s);
+                for (int k = 0; k <= i; k++) s = mma16(row4(X, i, k), b[k], s);
+            }
 #pragma unroll
             for (int e = 0; e < 4; e++) dst[(16 * i + 4 * lg + e) * kDk + c] = s[e];
         }
@@ -791,6 +825,160 @@ __global__ __launch_bounds__(kThreads) void dn_scan_kernel(const float *__restri
     }
 }
 
+// Up to kScanFewRows tokens are not a chunk's work: the products above are of
+// 64-token tiles and their chain (conv, Gram matrices, inverse, U and W, then
+// the scan) takes as long for one token as for 64.  They are scanned token by
+// token instead, after dn_prep_kernel has formed q, k, v, beta and decay of
+// all of them: 4.6 + 9.8 us for 16 tokens against 14.9 + 9.8, 4.6 + 12 for 32,
+// and 0.14 us more for each further one, so above 32 the gap closes.
+constexpr int kScanFewRows = 32;
+
+// Token b's conv taps for channel ch: the last kKsize values of (the old
+// window, the inputs of tokens 0..b) (conv_shift_and_append + conv_apply,
+// deltanet_cache.rs:34-54), then SiLU.
+template <int KP>
+__device__ __forceinline__ float conv_token(const MixIn &mix, const float *__restrict__ cs,
+                                            const float *__restrict__ conv_w, int ch, int b) {
+    const f32x4 old = *reinterpret_cast<const f32x4 *>(cs + (size_t)ch * kKsize);
+    const f32x4 wk = *reinterpret_cast<const f32x4 *>(conv_w + (size_t)ch * kKsize);
+    float xs[kKsize][KP];
+#pragma unroll
+    for (int i = 0; i < kKsize; i++) mix.load<KP>(max(b - kKsize + 1 + i, 0), ch, xs[i]);
+    const float ov[kKsize] = {old.x, old.y, old.z, old.w};
+    const float kw[kKsize] = {wk.x, wk.y, wk.z, wk.w};
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kKsize; i++) {
+        const int src = b - kKsize + 1 + i;  // < 0: from the old window
+        sum += (src >= 0 ? mix.add<KP>(xs[i]) : ov[(kKsize + src) & (kKsize - 1)]) * kw[i];
+    }
+    return silu_ref(sum);
+}
+
+// grid = (n_heads, T), 256 threads: thread t forms channel t % 128 of q (t <
+// 128) or k, normalised (deltanet.rs:25-31, 461-467), and threads t < 128 also
+// v channel t; thread 0 the token's beta and decay (deltanet.rs:474-480).
+// prep[(b * n_heads + h) * 384 + {0, 128, 256} + c] = q, k, v; bd[(b * n_heads
+// + h) * 2 + {0, 1}] = beta, decay.
+template <int KP>
+__global__ __launch_bounds__(kThreads) void dn_prep_kernel(MixIn mix, MixIn mbeta, MixIn malpha,
+                                                           const float *__restrict__ conv_w,
+                                                           const float *__restrict__ ssm_a,
+                                                           const float *__restrict__ dt_bias,
+                                                           const float *__restrict__ cs, float *__restrict__ prep,
+                                                           float *__restrict__ bd, int n_heads) {
+    __shared__ float red[4];
+    const int t = threadIdx.x, h = blockIdx.x, b = blockIdx.y;
+    const int chunk = n_heads * kDk, e = t & (kDk - 1);
+    const float y = conv_token<KP>(mix, cs, conv_w, t < kDk ? h * kDk + t : chunk + h * kDk + e, b);
+    const float vy = t < kDk ? conv_token<KP>(mix, cs, conv_w, 2 * chunk + h * kDk + t, b) : 0.0f;
+    const float sq = wave_sum(y * y);
+    if ((t & 63) == 0) red[t >> 6] = sq;
+    __syncthreads();
+    float *out = prep + ((size_t)b * n_heads + h) * 3 * kDk;
+    if (t < kDk) {
+        const float inv = 1.0f / sqrtf((red[0] + red[1]) + 1e-12f);
+        out[t] = (y * inv) * (1.0f / sqrtf((float)kDk));
+        out[2 * kDk + t] = vy;
+    } else {
+        out[kDk + e] = y * (1.0f / sqrtf((red[2] + red[3]) + 1e-12f));
+    }
+    if (t == 0) {
+        float xb[KP], xa[KP];
+        mbeta.load<KP>(b, h, xb);
+        malpha.load<KP>(b, h, xa);
+        float *o = bd + ((size_t)b * n_heads + h) * 2;
+        o[0] = 1.0f / (1.0f + expf(-mbeta.add<KP>(xb)));
+        o[1] = expf(ssm_a[h] * logf(1.0f + expf(malpha.add<KP>(xa) + dt_bias[h])));
+    }
+}
+
+// The recurrence is independent per value column j (recall sk_j, delta_j,
+// column j of the rank-1 update and the query o_j), so a head is split over
+// kDk / kScanCols single-wave workgroups, grid = (kDk / kScanCols, n_heads).
+// The workgroup copies its head's q and k, its columns' v and the tokens' beta
+// and decay into LDS; the token loop then has no global load.  Lane l holds
+// rows R (l % G) .. + R - 1 of column C g + l / G (G = 64 / C lanes per column,
+// R = 128 / G rows per lane) in registers across all T steps (state read and
+// written once); a sum over rows is 4 interleaved partial sums of R / 4 rows,
+// then a DPP sum over the column's G lanes.  Raw head outputs go to
+// out[t][chunk].
+constexpr int kScanCols = 4;
+constexpr int kDropOffset = 0x7ffffff0;  // buffer offset past any output: the store is dropped
+
+__global__ __launch_bounds__(kWave) void dn_scan_few_kernel(const float *__restrict__ prep,
+                                                              const float *__restrict__ bd, float *__restrict__ S,
+                                                              float *__restrict__ out, int n_heads, int T) {
+    constexpr int C = kScanCols, G = kWave / C, R = kDk / G;
+    static_assert(G == 16, "a column's lanes are one DPP row");
+    static_assert(C % 2 == 0 && C + 2 <= kWave, "lanes C, C + 1 carry beta and decay");
+    __shared__ __align__(16) float qks[kScanFewRows][2 * kDk];  // q then k of each token
+    __shared__ float exs[kScanFewRows][kWave];  // lanes 0..C-1: v of the columns, C, C+1: beta, decay
+    const int l = threadIdx.x, h = blockIdx.y;
+    const int chunk = n_heads * kDk;
+    const int rgp = l % G, jl = l / G, j = blockIdx.x * C + jl;
+    float *Sh = S + (size_t)h * kDk * kDk + j;
+    float st[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) st[r] = Sh[(size_t)(R * rgp + r) * kDk];
+    const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, 4 * T * chunk, 0x00020000);
+    // all loads of half the tokens in flight at once (clamped to the last
+    // token; slots past T are never read): lane l copies float4 l of q | k,
+    // lanes 0..C-1 also v of column l, lanes >= C beta (even) / decay (odd)
+#pragma unroll
+    for (int b0 = 0; b0 < kScanFewRows; b0 += kScanFewRows / 2) {
+        float4 qk[kScanFewRows / 2];
+        float ex[kScanFewRows / 2];
+#pragma unroll
+        for (int i = 0; i < kScanFewRows / 2; i++) {
+            const int b = min(b0 + i, T - 1);
+            const float *src = prep + ((size_t)b * n_heads + h) * 3 * kDk;
+            qk[i] = reinterpret_cast<const float4 *>(src)[l];
+            ex[i] = l < C ? src[2 * kDk + blockIdx.x * C + l] : bd[((size_t)b * n_heads + h) * 2 + (l & 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < kScanFewRows / 2; i++) {
+            reinterpret_cast<float4 *>(qks[b0 + i])[l] = qk[i];
+            exs[b0 + i][l] = ex[i];
+        }
+    }
+    __syncthreads();
+    for (int b = 0; b < T; b++) {
+        const float beta = exs[b][C], decay = exs[b][C + 1], v = exs[b][jl];
+        float kr[R], qr[R];
+#pragma unroll
+        for (int r = 0; r < R; r += 4) {
+            const float4 k4 = *reinterpret_cast<const float4 *>(&qks[b][kDk + R * rgp + r]);
+            const float4 q4 = *reinterpret_cast<const float4 *>(&qks[b][R * rgp + r]);
+            kr[r] = k4.x, kr[r + 1] = k4.y, kr[r + 2] = k4.z, kr[r + 3] = k4.w;
+            qr[r] = q4.x, qr[r + 1] = q4.y, qr[r + 2] = q4.z, qr[r + 3] = q4.w;
+        }
+        // S' = decay S; sk_j = sum_i S'_ij k_i
+        float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            st[r] *= decay;
+            p[r & 3] += st[r] * kr[r];
+        }
+        const float sk = row_sum16((p[0] + p[1]) + (p[2] + p[3]));
+        const float delta = beta * (v - sk);
+        // S'' = S' + k delta^T; o_j = sum_i S''_ij q_i
+#pragma unroll
+        for (int r = 0; r < 4; r++) p[r] = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            st[r] += kr[r] * delta;
+            p[r & 3] += st[r] * qr[r];
+        }
+        const float o = row_sum16((p[0] + p[1]) + (p[2] + p[3]));
+        // lanes of row group 0 store (the others' offset is past the buffer: dropped)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), orsrc,
+                                              rgp == 0 ? 4 * (b * chunk + h * kDk + j) : kDropOffset, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) Sh[(size_t)(R * rgp + r) * kDk] = st[r];
+}
+
 // After dn_scan_kernel: row b of the gated RMSNorm (deltanet.rs:517-533)
 // of the raw head outputs to the planes, and (row 0's workgroups) the conv
 // windows of the head's q, k and v channels after the T tokens: the last
@@ -856,14 +1044,30 @@ int launch_deltanet_scan(anehip_ctx *ctx, hipStream_t stream, int rows, int n_he
         return set_error(ctx->err, ANEHIP_EINVAL, "deltanet_scan: %d K splits (at most 16), %d rows (1..%d)", kp, rows,
                          kScanMaxRows);
     const int chunks = (rows + kCt - 1) / kCt;
+#define DN_FINISH(KP)                                                                                                \
+    hipLaunchKernelGGL(dn_scan_finish_kernel<KP>, dim3(n_heads, rows), dim3(kDk), 0, stream, mix, conv_state, heads, \
+                       gate_off, norm_w, xp, n_heads, eps, rows)
 #define DN_SCAN(KP)                                                                                                  \
-    hipLaunchKernelGGL(dn_chunk_kernel<KP>, dim3(chunks, n_heads), dim3(kThreads), 0, stream, mix, beta, alpha,      \
+    hipLaunchKernelGGL(dn_chunk_kernel<KP>, dim3(chunks, n_heads), dim3(kChunkThreads), 0, stream, mix, beta, alpha, \
                        conv_w, ssm_a, dt_bias, conv_state, prep, n_heads, rows);                                     \
     hipLaunchKernelGGL(dn_scan_kernel, dim3(kDk / 16, n_heads), dim3(kThreads), 0, stream, prep, S, heads, n_heads,  \
                        rows);                                                                                        \
-    hipLaunchKernelGGL(dn_scan_finish_kernel<KP>, dim3(n_heads, rows), dim3(kDk), 0, stream, mix, conv_state, heads, \
-                       gate_off, norm_w, xp, n_heads, eps, rows)
-    if (kp <= 1) {
+    DN_FINISH(KP)
+#define DN_FEW(KP)                                                                                                   \
+    hipLaunchKernelGGL(dn_prep_kernel<KP>, dim3(n_heads, rows), dim3(kThreads), 0, stream, mix, beta, alpha, conv_w, \
+                       ssm_a, dt_bias, conv_state, prep, prep + (size_t)rows * 3 * n_heads * kDk, n_heads);          \
+    hipLaunchKernelGGL(dn_scan_few_kernel, dim3(kDk / kScanCols, n_heads), dim3(kWave), 0, stream, prep,             \
+                       prep + (size_t)rows * 3 * n_heads * kDk, S, heads, n_heads, rows);                            \
+    DN_FINISH(KP)
+    if (rows <= kScanFewRows) {
+        if (kp <= 1) {
+            DN_FEW(1);
+        } else if (kp <= 4) {
+            DN_FEW(4);
+        } else {
+            DN_FEW(16);
+        }
+    } else if (kp <= 1) {
         DN_SCAN(1);
     } else if (kp <= 4) {
         DN_SCAN(4);
@@ -871,6 +1075,8 @@ int launch_deltanet_scan(anehip_ctx *ctx, hipStream_t stream, int rows, int n_he
         DN_SCAN(16);
     }
 #undef DN_SCAN
+#undef DN_FEW
+#undef DN_FINISH
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
     if (xp.uniform) return launch_split_rows(ctx, stream, heads, (uint32_t)rows, (uint32_t)(n_heads * kDk), xp);
     return ANEHIP_OK;

@@ -535,10 +535,11 @@ def test_prefill_long_prompt_large_cache(mid_host, n):
     oseq.close()
 
 
-@pytest.mark.parametrize("n", [2, 63, 64, 65, 129])
+@pytest.mark.parametrize("n", [2, 32, 33, 48, 49, 63, 64, 65, 129])
 def test_prefill_scan_chunk_edges(mid_host, n):
     """Prompts around the DeltaNet scan's 64-token chunks (two tokens, fewer
-    than the conv window; one short of a chunk, one chunk, one token over; two
+    than the conv window; the last prompt scanned token by token and the first
+    that is not; a chunk of three and of four 16-token tiles; one short of a chunk, one chunk, one token over; two
     and one), from a state that three decode steps left, vs the oracle run
     token by token: logits, states, conv windows, then a decode step."""
     spec = mid_host.spec
@@ -553,6 +554,33 @@ def test_prefill_scan_chunk_edges(mid_host, n):
         r = oseq.forward(int(t))
     l2, mx = rel_errs(g, r)
     print(f"prefill n={n}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
+    assert l2 <= TOL and mx <= TOL
+    _check_state(gm, oseq, 0, spec, "after prefill")
+    assert max(rel_errs(gm.step([int(toks[-1])])[0], oseq.forward(int(toks[-1])))) <= TOL
+    gm.close()
+    oseq.close()
+
+
+@pytest.mark.parametrize("n_heads,n_kv", [(2, 2), (4, 2), (4, 1), (8, 2)])
+@pytest.mark.parametrize("n", [32, 33, 61])
+def test_prefill_attention_groups(n_heads, n_kv, n):
+    """1, 2 and 4 query heads per kv head, so 32-, 16- and 8-token workgroups
+    of the prefill attention with a ragged last one, from position 3 on (no
+    tile starts at a token group's first position); 32 rows are the last that
+    run the decode kernels.  Vs the oracle run token by token."""
+    host = HostModel(anehip.Spec(**dict(SMALL, n_heads=n_heads, n_kv_heads=n_kv)), seed=9)
+    spec = host.spec
+    gm = _model(host, 1, 128)
+    oseq = host.seq(128)
+    toks = oracle.randint(37, n, n + 4, spec.vocab_size)
+    for t in toks[:3]:
+        gm.step([int(t)])
+        oseq.forward(int(t))
+    g = gm.prefill(0, toks[3:3 + n])
+    for t in toks[3:3 + n]:
+        r = oseq.forward(int(t))
+    l2, mx = rel_errs(g, r)
+    print(f"prefill {n_heads}/{n_kv} n={n}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
     assert l2 <= TOL and mx <= TOL
     _check_state(gm, oseq, 0, spec, "after prefill")
     assert max(rel_errs(gm.step([int(toks[-1])])[0], oseq.forward(int(toks[-1])))) <= TOL
