@@ -346,7 +346,10 @@ int launch_chunk(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const 
     if (rows <= 32 || ksplit < 1 || nsb % ksplit || m % 4 || !xp.hi || !xp.lo || !xp.xe || !xp.uniform)
         return set_error(ctx->err, ANEHIP_EINVAL, "gemm_rows: %u rows, K split %d of %d panels, m %u, %s planes", rows,
                          ksplit, nsb, m, xp.uniform ? "uniform" : "grouped");
-    if (4.0 * rows * m > 1073741824.0)
+    // (offsets are 64-bit; the FFN's rows, two sums to a value, may take twice
+    // the 1 GiB of a plain product, so that a chunk of 960 rows takes any F that
+    // one of 256 did)
+    if ((SILU ? 1.0 : 4.0) * rows * m > 1073741824.0)
         return set_error(ctx->err, ANEHIP_ESHAPE, "gemm_rows: output of %u x %u floats too large", rows, m);
     // the weights are addressed with 32-bit buffer offsets
     if ((double)ptiles * nsb * Panel<ANEHIP_GGML_Q8_0>::kBytes > 2147483647.0)

@@ -588,6 +588,22 @@ def test_prefill_attention_groups(n_heads, n_kv, n):
     oseq.close()
 
 
+def test_prefill_large_ffn():
+    """A full chunk of 960 tokens of a model whose FFN rows pass 1 GiB (hidden
+    140032, one kv head, random init): the last logits against the same prompt
+    in prefills of 480, whose products stay below it."""
+    spec = anehip.Spec(**dict(SMALL, hidden_dim=140032))
+    with anehip.Model(spec) as gm:
+        gm.randomize(seed=4)
+        gm.alloc_state(2, 960)
+        toks = oracle.randint(38, 1, 960, spec.vocab_size)
+        whole = gm.prefill(0, toks)
+        gm.prefill(1, toks[:480])
+        l2, mx = rel_errs(whole, gm.prefill(1, toks[480:]))
+    print(f"prefill hidden {spec.hidden_dim}: rel_l2={l2:.2e} rel_max={mx:.2e}", flush=True)
+    assert l2 <= TOL and mx <= TOL
+
+
 @pytest.mark.parametrize("n", [961, 1950])
 def test_prefill_full_chunks(mid_host, n):
     """Prompts past one chunk of 960 tokens: 961 (a full chunk, then one row on
