@@ -86,6 +86,7 @@ struct AttnPlan {
     bool even;
 };
 constexpr int kMaxPlanBatch = 64;
+constexpr int kPlanTiles = 8;
 // inclusive sum over the lanes of the wave up to this one
 __device__ __forceinline__ int wave_scan(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
@@ -96,11 +97,15 @@ __device__ __forceinline__ int wave_scan(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2, 3
     return v;
 }
-__device__ __forceinline__ AttnPlan attn_plan(const uint32_t *__restrict__ pos_arr, int batch, int n_kv, int W,
-                                              int max_tiles) {
+// pos: plan_pos(), loaded by the caller ahead of its other loads (vector loads
+// complete in order: behind them, the plan would wait for all of them).
+__device__ __forceinline__ uint32_t plan_pos(const uint32_t *__restrict__ pos_arr, int batch) {
+    return pos_arr[min((int)threadIdx.x & 63, batch - 1)];
+}
+__device__ __forceinline__ AttnPlan attn_plan(uint32_t pos, int batch, int n_kv, int W, int max_tiles) {
     const int lane = threadIdx.x & 63;
     AttnPlan P;
-    P.pos = (int)pos_arr[min(lane, batch - 1)];
+    P.pos = (int)pos;
     P.tiles = min(P.pos / kCh + 1, max_tiles);
     P.even = __ballot(P.tiles != __builtin_amdgcn_readfirstlane(P.tiles)) == 0;
     P.n = P.start = 0;
@@ -179,6 +184,8 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
     // the norm weights and the RoPE frequencies
     const bool is_q = wave < G, is_k = wave == G % 4;
     int hq, kin, vin;
+    uint32_t lane_pos = 0;
+    if constexpr (PLAN) lane_pos = plan_pos(pos_arr, batch);
     float4 aq[8], ak[8], av[8];
     auto load_inputs = [&]() {
         hq = kvh * G + (wave < G ? wave : 0);
@@ -204,7 +211,7 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
     int tb = 0, te = 0;  // tiles [tb, te)
     bool shared_out = false;
     if constexpr (PLAN) {
-        const AttnPlan P = attn_plan(pos_arr, batch, n_kv, batch * n_kv * nch, (max_seq + kCh - 1) / kCh);
+        const AttnPlan P = attn_plan(lane_pos, batch, n_kv, batch * n_kv * nch, (max_seq + kCh - 1) / kCh);
         if (!P.even) {
             shared_out = true;
             b = 63 - __builtin_clzll(__ballot(P.start <= slot0 && lane < batch));
@@ -488,13 +495,16 @@ __global__ __launch_bounds__(64) void attn_append_kernel(MixIn mix, const float 
 // dims 4l..4l+3 of chunks g, g + GR, g + 2 GR, ...; merges them with a
 // log-sum-exp rescale against the maximum over all chunks, adds the GR groups
 // through LDS, normalises and multiplies by sigmoid(gate) (deltanet.rs:667-669).
-// GR = 16 where a head has more than 16 chunks (up to 8 per group, all loaded
-// at once; with 4 groups of 32 chunks one after the other batch 1 at 32k
-// positions took 14.6 us; a step there 30.6 -> 22.5), 4 else.
+// GR = 16 where a head has more than kManyChunks chunks (up to 8 per group, all
+// loaded at once; with 4 groups of 32 chunks one after the other batch 1 at 32k
+// positions took 14.6 us; a step there 30.6 -> 22.5), 4 else: every 16 chunks
+// past the first 16 cost those ~1.5 us, the larger workgroup ~3 (20 chunks of 2
+// sequences 6.8 us traced, against 4.0).
+constexpr int kManyChunks = 48;
 // out: [batch][n_heads * 256] fp32, or range-safe fragment-order planes xp
-// (Planes) when xp.hi is not null.  plan_w > 0: the partials of a launch of
-// plan_w workgroups that attn_plan() may have shared out.
-template <int G, int GR>
+// (Planes) when xp.hi is not null.  PLAN: the partials of a launch of plan_w
+// workgroups that attn_plan() may have shared out.
+template <int G, int GR, bool PLAN>
 __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const uint32_t *__restrict__ pos_arr,
                                                                const float *__restrict__ part_o,
                                                                const float *__restrict__ part_ml, int nch,
@@ -509,22 +519,24 @@ __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const 
     // the gate's K-split slices (independent of the partials) and this
     // group's first PRE chunks are loaded together, before the maximum is known
     float4 gq[8];
+    uint32_t lane_pos = 0;
+    int nc;
+    size_t base = ((size_t)b * n_kv + kvh) * nch;
+    if constexpr (PLAN) lane_pos = plan_pos(pos_arr, (int)gridDim.y);
+    else nc = active_chunks((int)pos_arr[b] + 1, nch);
     {
         const float *g0 = mix.p + (size_t)b * mix.stride + h * 2 * kHd + kHd + 4 * l;
 #pragma unroll
         for (int q = 0; q < 8; q++) gq[q] = *reinterpret_cast<const float4 *>(g0 + (size_t)min(q, mix.kp - 1) * mix.split);
     }
-    int nc;
-    size_t base;
-    AttnPlan P;
-    P.even = true;
-    if (plan_w) P = attn_plan(pos_arr, (int)gridDim.y, n_kv, plan_w, (max_seq + kCh - 1) / kCh);
-    if (P.even) {
-        nc = active_chunks((plan_w ? __builtin_amdgcn_readlane(P.pos, b) : (int)pos_arr[b]) + 1, nch);
-        base = ((size_t)b * n_kv + kvh) * nch;
-    } else {
-        nc = __builtin_amdgcn_readlane(P.n, b);
-        base = (size_t)(__builtin_amdgcn_readlane(P.start, b) + kvh * nc);
+    if constexpr (PLAN) {
+        const AttnPlan P = attn_plan(lane_pos, (int)gridDim.y, n_kv, plan_w, (max_seq + kCh - 1) / kCh);
+        if (P.even) {
+            nc = active_chunks(__builtin_amdgcn_readlane(P.pos, b) + 1, nch);
+        } else {
+            nc = __builtin_amdgcn_readlane(P.n, b);
+            base = (size_t)(__builtin_amdgcn_readlane(P.start, b) + kvh * nc);
+        }
     }
     float4 p4[PRE];
     float pm[PRE], pl[PRE];
@@ -905,14 +917,20 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
     dim3 g1(nch, n_kv, batch), g2(n_heads, batch);
     // the caches this launch can read (prefill rows share one sequence's)
     const bool nt = (size_t)(row_stride ? batch : 1) * n_kv * max_seq * 2 * kHd * sizeof(__half) >= kNtKvBytes;
-    // sequences of their own, at least two workgroups each to share out
-    const bool plan = row_stride && batch >= 2 && batch <= kMaxPlanBatch && nch >= 2;
+    // sequences of their own, at least two workgroups each to share out, and
+    // chunks that can grow to kPlanTiles tiles: equal lengths pay the plan
+    // without a use for it (20.0 against 19.4 us at batch 32, 5 tiles a chunk)
+    const bool plan = row_stride && batch >= 2 && batch <= kMaxPlanBatch && nch >= 2 &&
+                      (max_seq + kCh - 1) / kCh >= kPlanTiles * nch;
     const int W = batch * n_kv * nch;
-    const bool many = nch > 16;  // chunks per head, with a plan on average
+    const bool many = nch > kManyChunks;  // chunks per head, with a plan on average
 #define ANEHIP_ATTN_PART(GG, NT, PLAN)                                                                          \
     hipLaunchKernelGGL((attn_partial_kernel<GG, NT, PLAN>), g1, dim3(kThreads), 0, stream, mix, q_norm, k_norm, \
                        inv_freq, pos, k_cache, v_cache, max_seq, n_heads, n_kv, part_o, part_ml, cache_off,     \
                        row_stride, append, batch)
+#define ANEHIP_ATTN_COMBINE(GG, GR, PLAN)                                                                       \
+    hipLaunchKernelGGL((attn_combine_kernel<GG, GR, PLAN>), g2, dim3(64 * GR), 0, stream, mix, pos, part_o,     \
+                       part_ml, nch, n_heads, n_kv, out, xp, W, max_seq)
 #define ANEHIP_ATTN_CASE(GG)                                                                                    \
     case GG:                                                                                                    \
         if (nt && plan) ANEHIP_ATTN_PART(GG, true, true);                                                       \
@@ -921,12 +939,10 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
         else ANEHIP_ATTN_PART(GG, false, false);                                                                \
         ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                            \
         if (!out && !xp.hi) return ANEHIP_OK; /* partials only */                                               \
-        if (many)                                                                                               \
-            hipLaunchKernelGGL((attn_combine_kernel<GG, 16>), g2, dim3(64 * 16), 0, stream, mix, pos, part_o,   \
-                               part_ml, nch, n_heads, n_kv, out, xp, plan ? W : 0, max_seq);                    \
-        else                                                                                                    \
-            hipLaunchKernelGGL((attn_combine_kernel<GG, 4>), g2, dim3(64 * 4), 0, stream, mix, pos, part_o,     \
-                               part_ml, nch, n_heads, n_kv, out, xp, plan ? W : 0, max_seq);                    \
+        if (many && plan) ANEHIP_ATTN_COMBINE(GG, 16, true);                                                    \
+        else if (many) ANEHIP_ATTN_COMBINE(GG, 16, false);                                                      \
+        else if (plan) ANEHIP_ATTN_COMBINE(GG, 4, true);                                                        \
+        else ANEHIP_ATTN_COMBINE(GG, 4, false);                                                                 \
         ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                            \
         return ANEHIP_OK;
     switch (G) {
@@ -937,6 +953,7 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
             return set_error(ctx->err, ANEHIP_EUNSUPPORTED, "attention: %d query heads per kv head (1, 2 or 4)", G);
     }
 #undef ANEHIP_ATTN_CASE
+#undef ANEHIP_ATTN_COMBINE
 #undef ANEHIP_ATTN_PART
 }
 
