@@ -2891,6 +2891,11 @@ int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m,
         return dispatch_fused<T>(ctx, stream, w, m, n, in, out, ksplit);
     }
     const uint8_t *wb = static_cast<const uint8_t *>(w);
+    // With several K splits (or groups) each has its share of the CUs and its
+    // workgroups walk the tiles, so that x is staged once per workgroup and
+    // the next tile's weights are in flight: 16384 x 8192 (4 splits) at batch
+    // 9 / 17 / 32 (Q4_0) 38 / 64 / 63 us, with a workgroup per tile and split 45 /
+    // 84 / 90.
     // 17..32 rows as two groups of 16 side by side where each workgroup has
     // one tile to do, or two (the second group's weights come from the L2 or
     // the MALL)
@@ -2898,8 +2903,9 @@ int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m,
     if (batch <= 16 || tiles * ksplit <= cus) {
         const int work = ksplit * groups;
         auto rows_tiles = [&](int r) { return (int)((m + r - 1) / r); };
+        const int per_work = max(1, cus / work);
 #define ANEHIP_XS(RS)                                                                                       \
-    hipLaunchKernelGGL((quant_gemm_xs<T, RS>), dim3(min(rows_tiles(16 * RS), cus), ksplit, groups), dim3(512), \
+    hipLaunchKernelGGL((quant_gemm_xs<T, RS>), dim3(min(rows_tiles(16 * RS), per_work), ksplit, groups), dim3(512), \
                        0, stream, wb, x, out, (int)m, (int)n, (int)batch, split_stride)
         if (rows_tiles(16) * work <= cus) ANEHIP_XS(1);
         else if (rows_tiles(32) * work <= cus) ANEHIP_XS(2);
@@ -2908,7 +2914,7 @@ int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m,
         ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
         return ANEHIP_OK;
     }
-    const dim3 grid(min(tiles, cus), ksplit);
+    const dim3 grid(min(tiles, max(1, cus / ksplit)), ksplit);
     // 17..32: x split into range-safe fp16 hi / lo planes (row-major) first
     const size_t count = (size_t)batch * n;
     Planes xp;
