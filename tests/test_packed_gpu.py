@@ -196,6 +196,30 @@ def test_packed_gemm_tall(gpu_ctx, oracle_lib, t, batch, m, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [2304, 4096, 4352, 8192, 8448])
+@pytest.mark.parametrize("batch", [33, 35])
+def test_packed_gemm_row_split(gpu_ctx, oracle_lib, batch, n):
+    """Around the widths at which the chunk GEMM's plane split holds 1, 2 or 4
+    fragments per thread and reads the rest twice (above 8192), with 1 and 3
+    rows in its last workgroup of 4; rows scaled by 1e4 and 1e-4 in turn, so
+    that a row that took a neighbour's exponent shows."""
+    m = 68
+    w = oracle_lib.gen_quant(8, 78, n, m, n, std=0.02)
+    x = oracle_lib.normal(78, 901 + batch, batch * n).reshape(batch, n)
+    x *= np.where(np.arange(batch) % 2, np.float32(1e4), np.float32(1e-4))[:, None]
+    dw, dp, _ = _pack(gpu_ctx, 8, w, m, n)
+    dx, dy = gpu_ctx.to_device(x), gpu_ctx.alloc(batch * m * 4)
+    gpu_ctx.call("quant_gemm_packed", 8, dp, m, n, dx, batch, dy)
+    y = dy.download(np.float32, batch * m).reshape(batch, m)
+    ref = oracle_lib.gemm(8, w, m, n, x)
+    worst = max(max(rel_errs(y[b], ref[b])) for b in range(batch))
+    print(f"n={n} batch={batch}: worst row {worst:.2e}", flush=True)
+    assert worst <= TOL
+    for b in (dw, dp, dx, dy):
+        b.free()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("t", [8, 2])
 @pytest.mark.parametrize("m,n,batch", [(64, 256, 33), (260, 512, 64), (516, 768, 65), (256, 4096, 96), (2056, 2304, 129),
                                        (1028, 8448, 250)])
