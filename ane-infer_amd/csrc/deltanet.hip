@@ -459,6 +459,30 @@ __device__ __forceinline__ f32x4 mma16(f32x4 a, f32x4 b, f32x4 c) {
     for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
     return c;
 }
+// The same for a lower triangular a (rows and columns are the tokens of one
+// tile): an infinity or NaN in a token's row of b reaches that token's row of
+// the result and the rows after it, as in the token-by-token order, and not by
+// way of a's zeros the rows before it (their later layers' K / V rows are kept
+// when a sequence is rewound to before the token).  Finite b, which a few
+// integer instructions tell, takes the plain product.
+__device__ __forceinline__ f32x4 mma16_lower(f32x4 a, f32x4 b, f32x4 c) {
+    uint32_t top = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) top = max(top, __float_as_uint(b[e]) & 0x7fffffffu);
+    if (__ballot(top >= 0x7f800000u) == 0) return mma16(a, b, c);
+    const int r0 = 4 * ((threadIdx.x & 63) >> 4);  // the lane's rows of b and of the result
+    f32x4 out = c;
+#pragma unroll 1
+    for (int r = 0; r < 16; r++) {
+        f32x4 m;
+#pragma unroll
+        for (int e = 0; e < 4; e++) m[e] = r0 + e <= r ? b[e] : 0.0f;
+        m = mma16(a, m, c);
+#pragma unroll
+        for (int e = 0; e < 4; e++) out[e] = r0 + e == r ? m[e] : out[e];
+    }
+    return out;
+}
 
 // grid = (chunks of 64 tokens, n_heads), 512 threads.  Conv + SiLU over the
 // tokens' windows (conv_shift_and_append + conv_apply, deltanet_cache.rs:34-54),
@@ -670,7 +694,7 @@ __global__ __launch_bounds__(kChunkThreads) void dn_chunk_kernel(MixIn mix, MixI
                 for (int e = 0; e < 4; e++) xb[e] = X[(16 * k + 4 * lg + e) * kTriF + 16 * j + li];
                 p = mma16(row4(L, i, k), xb, p);
             }
-            const f32x4 v = mma16(row4(X, i, i), p, f32x4{});
+            const f32x4 v = mma16_lower(row4(X, i, i), p, f32x4{});
 #pragma unroll
             for (int e = 0; e < 4; e++) X[(16 * i + 4 * lg + e) * kTriF + 16 * j + li] = -v[e];
         }
@@ -698,7 +722,8 @@ __global__ __launch_bounds__(kChunkThreads) void dn_chunk_kernel(MixIn mix, MixI
             f32x4 s = {};
             if (i < nt) {
 #pragma unroll
-                for (int k = 0; k <= i; k++) s = mma16(row4(X, i, k), b[k], s);
+                for (int k = 0; k < i; k++) s = mma16(row4(X, i, k), b[k], s);
+                s = mma16_lower(row4(X, i, i), b[i], s);
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) dst[(16 * i + 4 * lg + e) * kDk + c] = s[e];
@@ -727,7 +752,7 @@ __global__ __launch_bounds__(kThreads) void dn_scan_kernel(const float *__restri
     for (int j = 0; j < 8; j++)
 #pragma unroll
         for (int e = 0; e < 4; e++) st[j][e] = Sh[(size_t)(16 * j + 4 * lg + e) * kDk];
-    f32x4 w4[8], q4[8], k4[2][4], a4[4], u;
+    f32x4 w4[8], q4[8], k4[2][4], a4[4], u;  // a4: A's tiles up to the diagonal one (a4[3])
     float g;
     auto base = [&](int c) { return scr + ((size_t)min(c, chunks - 1) * n_heads + h) * kDnChunkFloats; };
     auto load_w = [&](int c) {
@@ -755,7 +780,7 @@ __global__ __launch_bounds__(kThreads) void dn_scan_kernel(const float *__restri
     auto load_a = [&](int c) {
         const float *p = base(c) + kOffA + (16 * wave + li) * kCt + 4 * lg;
 #pragma unroll
-        for (int j = 0; j < 4; j++) a4[j] = *reinterpret_cast<const f32x4 *>(p + 16 * j);
+        for (int j = 0; j < 4; j++) a4[j] = *reinterpret_cast<const f32x4 *>(p + 16 * min(j, wave));
     };
     load_w(0);
     load_q(0);
@@ -768,7 +793,8 @@ __global__ __launch_bounds__(kThreads) void dn_scan_kernel(const float *__restri
             s0 = mma16(w4[j], st[j], s0);
             s1 = mma16(w4[j + 1], st[j + 1], s1);
         }
-        dl[wave][lane] = u - (s0 + s1);
+        const f32x4 own = u - (s0 + s1);
+        dl[wave][lane] = own;
         load_w(c + 1);
         f32x4 o = {}, o1 = {};
 #pragma unroll
@@ -800,13 +826,12 @@ __global__ __launch_bounds__(kThreads) void dn_scan_kernel(const float *__restri
         sl[2 * wave][lane] = n0;
         sl[2 * wave + 1][lane] = n1;
         load_k(c + 1);
-#pragma unroll
-        for (int j = 0; j < 4; j += 2) {
-            o = mma16(a4[j], dv[j], o);
-            o1 = mma16(a4[j + 1], dv[j + 1], o1);
-        }
+        // A Delta: the tiles left of the diagonal (wave-uniform), then the diagonal one
+        if (wave > 0) o = mma16(a4[0], dv[0], o);
+        if (wave > 1) o1 = mma16(a4[1], dv[1], o1);
+        if (wave > 2) o = mma16(a4[2], dv[2], o);
+        o += mma16_lower(a4[3], own, o1);
         load_a(c + 1);
-        o += o1;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int tok = c * kCt + 16 * wave + 4 * lg + e;

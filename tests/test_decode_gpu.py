@@ -588,6 +588,41 @@ def test_prefill_attention_groups(n_heads, n_kv, n):
     oseq.close()
 
 
+def _prefill_past_nan(spec, n, at):
+    """Prefills n tokens whose token `at` has NaN for its embedding.  Returns
+    the model and an oracle sequence run over the tokens before it."""
+    host = HostModel(spec, seed=12)
+    toks = oracle.randint(39, n, n, spec.vocab_size - 1)
+    toks[at] = spec.vocab_size - 1
+    gm = _model(host, 1, 256)
+    emb = host.tensors[(-1, anehip.T["EMBEDDING"])][0].reshape(spec.vocab_size, spec.dim).copy()
+    emb[-1] = np.nan
+    gm.upload_f32(-1, anehip.T["EMBEDDING"], emb)
+    oseq = host.seq(256)
+    for t in toks[:at]:
+        oseq.forward(int(t))
+    assert not np.isfinite(gm.prefill(0, toks)).any()
+    gm.set_pos(0, at)
+    return gm, oseq
+
+
+@pytest.mark.parametrize("at", [2, 70, 141])
+def test_prefill_nan_token_deltanet(at):
+    """A NaN in one token of a chunk of 150 leaves the tokens before it as they
+    are (the DeltaNet products run over 64 tokens, their triangular ones over
+    16-token tiles; token 141 in the ragged last tile): the KV rows before it
+    in the attention layer that follows."""
+    spec = anehip.Spec(**dict(SMALL, n_layers=2, layer_types=[anehip.LAYER_DELTANET, anehip.LAYER_ATTENTION]))
+    gm, oseq = _prefill_past_nan(spec, 150, at)
+    for which in (2, 3):
+        g = gm.get_state(1, which, 0).view(np.float16).reshape(spec.n_kv_heads, -1, spec.head_dim)[:, :at]
+        r = oseq.view(1, which, spec.n_kv_heads * 256 * spec.head_dim, np.uint16).view(np.float16)
+        r = r.reshape(spec.n_kv_heads, -1, spec.head_dim)[:, :at]
+        assert max(rel_errs(g.astype(np.float32), r.astype(np.float32))) <= TOL, which
+    gm.close()
+    oseq.close()
+
+
 def test_prefill_large_ffn():
     """A full chunk of 960 tokens of a model whose FFN rows pass 1 GiB (hidden
     140032, one kv head, random init): the last logits against the same prompt
