@@ -468,13 +468,15 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
 
 // Prefill: the k / v rows of T consecutive tokens of one sequence (row t at
 // position pos_arr[t]) -- RMSNorm + RoPE of k, both rounded to fp16 -- written
-// to the cache at cache_off, as the decode kernel appends one row.  grid =
-// (n_kv, T), one wave.
+// to the cache at cache_off, as the decode kernel appends one row.  odd (when
+// not null): [n_kv][T], 1 where the row's v holds an infinity or NaN (fp16
+// overflows from 65520), 0 else.  grid = (n_kv, T), one wave.
 __global__ __launch_bounds__(64) void attn_append_kernel(MixIn mix, const float *__restrict__ k_norm,
                                                          const float *__restrict__ inv_freq,
                                                          const uint32_t *__restrict__ pos_arr,
                                                          __half *__restrict__ k_cache, __half *__restrict__ v_cache,
-                                                         size_t cache_off, int max_seq, int n_heads, int n_kv) {
+                                                         size_t cache_off, int max_seq, int n_heads, int n_kv,
+                                                         uint32_t *__restrict__ odd) {
     const int lane = threadIdx.x, kvh = blockIdx.x, b = blockIdx.y;
     const uint32_t pos = pos_arr[b];
     const int kin = n_heads * 2 * kHd + kvh * kHd;
@@ -484,10 +486,17 @@ __global__ __launch_bounds__(64) void attn_append_kernel(MixIn mix, const float 
     const float4 v4 = mix.at4(b, vin + 4 * lane);
     const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
     const size_t o = cache_off + ((size_t)kvh * max_seq + pos) * kHd + 4 * lane;
+    bool bad = false;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
+        const __half v = __float2half_rn(vv[i]);
         k_cache[o + i] = __float2half_rn(k4[i]);
-        v_cache[o + i] = __float2half_rn(vv[i]);
+        v_cache[o + i] = v;
+        bad |= (__half_as_ushort(v) & 0x7c00) == 0x7c00;
+    }
+    if (odd) {
+        const bool any = __ballot(bad) != 0;
+        if (lane == 0) odd[(size_t)kvh * gridDim.y + b] = any;
     }
 }
 
@@ -652,30 +661,36 @@ __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const 
 // position 0 and 158 at 540 from 960 on, plus 17 for its merge; here 39 and 51,
 // 64 MFMAs of 32 cycles per wave and tile, the rest the softmax between the two
 // products, which one wave per SIMD doesn't hide.
-// A row's masked scores weigh 0, but the V rows of later tokens of its group
-// enter the product with that 0: an infinity there shows as a NaN in this row
-// too, and not only in the rows from that token on (whose results it ends
-// anyway, the prompt's logits with them).
+// A row's masked scores weigh 0, and the V rows of later tokens of its group
+// enter the product with that 0, so that an infinity or NaN among them would
+// make this row NaN, and not only the rows from that token on (the earlier
+// tokens' K / V rows in the layers after outlive it where the sequence is
+// rewound).  A group with such a row (odd, of attn_append_kernel) goes token by
+// token: no tile then holds a V row that its query rows don't see.
 constexpr int kQRows = 32;    // query rows per workgroup
 constexpr int kPTile = 32;    // positions per tile
 constexpr int kMergeF = 66;   // LDS row of the merge: reads along the dims hit all banks
 
+// Tokens t0 .. T - 1 (at most 32 / G) of kv head kvh; row t is at position p0 + t.
+// False, with nothing written, where a lane's bad is not 0 (looked at once the
+// first tiles' loads are on their way).
 template <int G>
-__global__ __launch_bounds__(kThreads, 1) void attn_prefill_kernel(
-    MixIn mix, const float *__restrict__ q_norm, const float *__restrict__ inv_freq,
-    const uint32_t *__restrict__ pos_arr, const __half *__restrict__ k_cache, const __half *__restrict__ v_cache,
-    size_t cache_off, int max_seq, int n_heads, int T, float *__restrict__ out) {
-    constexpr int QT = kQRows / G;  // tokens per workgroup
+__device__ __forceinline__ bool prefill_tokens(MixIn mix, const float *__restrict__ q_norm,
+                                               const float *__restrict__ inv_freq,
+                                               int p0, const __half *__restrict__ k_cache,
+                                               const __half *__restrict__ v_cache, size_t cache_off, int max_seq,
+                                               int n_heads, int kvh, int t0, int T, uint32_t bad,
+                                               float *__restrict__ out) {
     __shared__ __align__(16) h8v qs[16 * 2 * 64];             // q fragments [k-step][hi, lo][lane]
     __shared__ __align__(16) float lds[4 * 4 * 16 * kMergeF];  // the merge's [wave][c][element][lane]
     __shared__ int qexp[kQRows];
     __shared__ float wm[4][kQRows], wl[4][kQRows];
-    const int t = threadIdx.x, lane = t & 63, col = lane & 31, h = lane >> 5;
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));  // not invariant in the kernel's loop: what it gives would be held in registers and spill
+    const int lane = t & 63, col = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    // the last tokens see the most positions: they go first
-    const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * QT, kvh = blockIdx.y;
     const size_t base = cache_off + (size_t)kvh * max_seq * kHd;
-    const int last = (int)pos_arr[min(t0 + QT, T) - 1], plim = (int)pos_arr[min(t0 + col / G, T - 1)];
+    const int last = p0 + T - 1, plim = p0 + min(t0 + col / G, T - 1);
     const int tiles = last / kPTile + 1;
     const __amdgpu_buffer_rsrc_t krs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(k_cache) + base, 0, (last + 1) * kHd * 2, kWord3);
@@ -728,7 +743,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_prefill_kernel(
     for (int i = 0; i < QR; i++) {
         const int r = QR * wave + i;
         if (i % G == 0) {
-            const float fpos = (float)pos_arr[min(t0 + r / G, T - 1)];
+            const float fpos = (float)(p0 + min(t0 + r / G, T - 1));
             sincosf(fpos * fr.x, &sn0, &cs0);
             sincosf(fpos * fr.y, &sn1, &cs1);
         }
@@ -755,6 +770,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_prefill_kernel(
         reinterpret_cast<h4v *>(&qs[o + 64])[lane & 1] = lo;
     }
     lds_barrier();
+    if (__ballot(bad != 0)) return false;
     const int qe = qexp[col];
     float m_run = -INFINITY, l_run = 0.0f;
     f32x16 o[2][4] = {};  // [q][c]: dims 128 q + 4 i + c
@@ -877,6 +893,30 @@ __global__ __launch_bounds__(kThreads, 1) void attn_prefill_kernel(
                                 v[2] * (1.0f / (1.0f + expf(-g.z))), v[3] * (1.0f / (1.0f + expf(-g.w))));
         }
     }
+    return true;
+}
+
+template <int G>
+__global__ __launch_bounds__(kThreads, 1) void attn_prefill_kernel(
+    MixIn mix, const float *__restrict__ q_norm, const float *__restrict__ inv_freq,
+    const uint32_t *__restrict__ pos_arr, const __half *__restrict__ k_cache, const __half *__restrict__ v_cache,
+    size_t cache_off, int max_seq, int n_heads, int T, const uint32_t *__restrict__ odd, float *__restrict__ out) {
+    constexpr int QT = kQRows / G;  // tokens per workgroup
+    // the last tokens see the most positions: they go first
+    const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * QT, kvh = blockIdx.y, end = min(t0 + QT, T);
+    const int p0 = (int)pos_arr[0];
+    uint32_t bad = odd[(size_t)kvh * T + min(t0 + ((int)threadIdx.x & (QT - 1)), end - 1)];
+#pragma unroll 1
+    for (int a = t0, step = QT; a < end;) {
+        if (prefill_tokens<G>(mix, q_norm, inv_freq, p0, k_cache, v_cache, cache_off, max_seq, n_heads, kvh, a,
+                              min(a + step, end), bad, out)) {
+            a += step;
+            if (a < end) lds_barrier();  // the tokens before are done with the LDS
+        } else {
+            step = 1;
+            bad = 0;
+        }
+    }
 }
 
 // Chunks per (sequence, kv head): at most 128, at most one per 64-position
@@ -972,22 +1012,27 @@ int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int 
                              const MixIn &mix, const float *q_norm, const float *k_norm, const float *inv_freq,
                              const uint32_t *pos, __half *k_cache, __half *v_cache, size_t cache_off, float *part,
                              float *out, const Planes &xp) {
-    hipLaunchKernelGGL(attn_append_kernel, dim3(n_kv, rows), dim3(64), 0, stream, mix, k_norm, inv_freq, pos, k_cache,
-                       v_cache, cache_off, max_seq, n_heads, n_kv);
-    ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
     if ((size_t)max_seq * kHd * 2 >= (size_t)1 << 30)
         return set_error(ctx->err, ANEHIP_EUNSUPPORTED, "attention: max_seq %d too large", max_seq);
     // few rows: one workgroup of the decode kernel per row and kv head has less
     // to set up (16 rows from position 0: 8.8 + 4.1 us with its merge, against
     // 23.8 + 4.6 with the planes' launch); above, both sides' launches are those
     // of the uniform planes, and 33 rows of a 4-layer model take 535 us against 659
-    if (rows <= kPrefillFewRows && !xp.uniform)
+    const bool few = rows <= kPrefillFewRows && !xp.uniform;
+    uint32_t *odd = reinterpret_cast<uint32_t *>(part);  // [n_kv][rows]
+    if (!few && rows > kPrefillFewRows * (kHd + 2))
+        return set_error(ctx->err, ANEHIP_EINVAL, "attention: %d rows", rows);
+    hipLaunchKernelGGL(attn_append_kernel, dim3(n_kv, rows), dim3(64), 0, stream, mix, k_norm, inv_freq, pos, k_cache,
+                       v_cache, cache_off, max_seq, n_heads, n_kv, few ? nullptr : odd);
+    ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
+    if (few)
         return attention_impl(ctx, stream, rows, n_heads, n_kv, max_seq, mix, q_norm, k_norm, inv_freq, pos, k_cache,
                               v_cache, part, nullptr, xp, cache_off, 0, false);
     const int G = n_heads / n_kv;
 #define ANEHIP_ATTN_PREFILL(GG)                                                                                      \
     hipLaunchKernelGGL(attn_prefill_kernel<GG>, dim3((rows * GG + kQRows - 1) / kQRows, n_kv), dim3(kThreads), 0,     \
-                       stream, mix, q_norm, inv_freq, pos, k_cache, v_cache, cache_off, max_seq, n_heads, rows, out)
+                       stream, mix, q_norm, inv_freq, pos, k_cache, v_cache, cache_off, max_seq, n_heads, rows, odd, \
+                       out)
     if (G == 4) ANEHIP_ATTN_PREFILL(4);
     else if (G == 2) ANEHIP_ATTN_PREFILL(2);
     else if (G == 1) ANEHIP_ATTN_PREFILL(1);

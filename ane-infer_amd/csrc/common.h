@@ -561,7 +561,8 @@ int launch_attention(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads
 // attends row t over positions [0, pos[t]]: out [rows][n_heads * 256] fp32
 // (scratch), then its fragment-order planes.  Up to kPrefillFewRows rows into
 // planes that are not uniform run on the decode kernel instead, with part as
-// its scratch (attn_partial_floats of up to as many rows).
+// its scratch (attn_partial_floats of up to as many rows); more rows keep a
+// word per row and kv head there.
 constexpr int kPrefillFewRows = 32;
 int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, int n_kv, int max_seq,
                              const MixIn &mix, const float *q_norm, const float *k_norm, const float *inv_freq,

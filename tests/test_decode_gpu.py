@@ -623,6 +623,22 @@ def test_prefill_nan_token_deltanet(at):
     oseq.close()
 
 
+@pytest.mark.parametrize("n_heads,n_kv", [(2, 2), (4, 2), (4, 1)])
+@pytest.mark.parametrize("at", [1, 61])
+def test_prefill_nan_token_attention(n_heads, n_kv, at):
+    """The same for two attention layers, 1, 2 and 4 query heads per kv head
+    (32-, 16- and 8-token workgroups): the sequence rewound to the token goes
+    on as one that never met it."""
+    spec = anehip.Spec(**dict(SMALL, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv,
+                              layer_types=2 * [anehip.LAYER_ATTENTION]))
+    gm, oseq = _prefill_past_nan(spec, 65, at)
+    _check_state(gm, oseq, 0, spec, "rewound")
+    for t in (5, 6):
+        assert max(rel_errs(gm.step([t])[0], oseq.forward(t))) <= TOL
+    gm.close()
+    oseq.close()
+
+
 def test_prefill_large_ffn():
     """A full chunk of 960 tokens of a model whose FFN rows pass 1 GiB (hidden
     140032, one kv head, random init): the last logits against the same prompt
