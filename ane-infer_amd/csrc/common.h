@@ -530,7 +530,7 @@ int launch_deltanet_head(anehip_ctx *ctx, hipStream_t stream, int batch, int n_h
 // sequence's block S) carried over the chunks, raw head outputs to heads
 // [rows][dim] (scratch); row t's gated RMSNorm to the planes (uniform ones by
 // way of heads) and the conv windows (the sequence's block conv_state)
-// advanced by the rows.  Up to 32 rows are scanned token by token (scratch of
+// advanced by the rows.  Up to 128 rows are scanned token by token (scratch of
 // 386 floats per row and head).
 constexpr size_t kDnChunkFloats = 4 * 64 * 128 + 64 * 64 + 64;
 int launch_deltanet_scan(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, const MixIn &mix,

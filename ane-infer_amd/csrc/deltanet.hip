@@ -850,13 +850,16 @@ __global__ __launch_bounds__(kThreads) void dn_scan_kernel(const float *__restri
     }
 }
 
-// Up to kScanFewRows tokens are not a chunk's work: the products above are of
-// 64-token tiles and their chain (conv, Gram matrices, inverse, U and W, then
-// the scan) takes as long for one token as for 64.  They are scanned token by
-// token instead, after dn_prep_kernel has formed q, k, v, beta and decay of
-// all of them: 4.6 + 9.8 us for 16 tokens against 14.9 + 9.8, 4.6 + 12 for 32,
-// and 0.14 us more for each further one, so above 32 the gap closes.
-constexpr int kScanFewRows = 32;
+// Up to kScanFewRows tokens are scanned token by token instead, after
+// dn_prep_kernel has formed q, k, v, beta and decay of all of them: the chunk's
+// chain (conv, Gram matrices, inverse, U and W) takes as long for one token as
+// for 64 and for one chunk as for all, 15 us from whole sums and 32 from K-split
+// slices, the scan over it 1.5 us per 64 tokens, a token here 0.14 us.  Prompts of 4
+// layers (3 DeltaNet) in us, chunks / tokens: 1024 wide 64 tokens 504 / 445, 128
+// 533 / 513, 192 572 / 576; 2048 wide 64 594 / 535, 128 667 / 647, 160 722 / 730;
+// 2304 wide 128 879 / 886, 160 961 / 973.
+constexpr int kScanFewRows = 128;
+constexpr int kScanStage = 32;  // of them in LDS at a time
 
 // Token b's conv taps for channel ch: the last kKsize values of (the old
 // window, the inputs of tokens 0..b) (conv_shift_and_append + conv_apply,
@@ -937,8 +940,8 @@ __global__ __launch_bounds__(kWave) void dn_scan_few_kernel(const float *__restr
     constexpr int C = kScanCols, G = kWave / C, R = kDk / G;
     static_assert(G == 16, "a column's lanes are one DPP row");
     static_assert(C % 2 == 0 && C + 2 <= kWave, "lanes C, C + 1 carry beta and decay");
-    __shared__ __align__(16) float qks[kScanFewRows][2 * kDk];  // q then k of each token
-    __shared__ float exs[kScanFewRows][kWave];  // lanes 0..C-1: v of the columns, C, C+1: beta, decay
+    __shared__ __align__(16) float qks[kScanStage][2 * kDk];  // q then k of each token
+    __shared__ float exs[kScanStage][kWave];  // lanes 0..C-1: v of the columns, C, C+1: beta, decay
     const int l = threadIdx.x, h = blockIdx.y;
     const int chunk = n_heads * kDk;
     const int rgp = l % G, jl = l / G, j = blockIdx.x * C + jl;
@@ -947,58 +950,63 @@ __global__ __launch_bounds__(kWave) void dn_scan_few_kernel(const float *__restr
 #pragma unroll
     for (int r = 0; r < R; r++) st[r] = Sh[(size_t)(R * rgp + r) * kDk];
     const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, 4 * T * chunk, 0x00020000);
-    // all loads of half the tokens in flight at once (clamped to the last
-    // token; slots past T are never read): lane l copies float4 l of q | k,
-    // lanes 0..C-1 also v of column l, lanes >= C beta (even) / decay (odd)
+    // kScanStage tokens at a time, all loads of a half of them in flight at once
+    // (clamped to the last token; slots past T are never read): lane l copies
+    // float4 l of q | k, lanes 0..C-1 also v of column l, lanes >= C beta (even)
+    // / decay (odd)
+    for (int c0 = 0; c0 < T; c0 += kScanStage) {
+        if (c0) __syncthreads();  // the tokens before are done with the LDS
 #pragma unroll
-    for (int b0 = 0; b0 < kScanFewRows; b0 += kScanFewRows / 2) {
-        float4 qk[kScanFewRows / 2];
-        float ex[kScanFewRows / 2];
+        for (int b0 = 0; b0 < kScanStage; b0 += kScanStage / 2) {
+            float4 qk[kScanStage / 2];
+            float ex[kScanStage / 2];
 #pragma unroll
-        for (int i = 0; i < kScanFewRows / 2; i++) {
-            const int b = min(b0 + i, T - 1);
-            const float *src = prep + ((size_t)b * n_heads + h) * 3 * kDk;
-            qk[i] = reinterpret_cast<const float4 *>(src)[l];
-            ex[i] = l < C ? src[2 * kDk + blockIdx.x * C + l] : bd[((size_t)b * n_heads + h) * 2 + (l & 1)];
+            for (int i = 0; i < kScanStage / 2; i++) {
+                const int b = min(c0 + b0 + i, T - 1);
+                const float *src = prep + ((size_t)b * n_heads + h) * 3 * kDk;
+                qk[i] = reinterpret_cast<const float4 *>(src)[l];
+                ex[i] = l < C ? src[2 * kDk + blockIdx.x * C + l] : bd[((size_t)b * n_heads + h) * 2 + (l & 1)];
+            }
+#pragma unroll
+            for (int i = 0; i < kScanStage / 2; i++) {
+                reinterpret_cast<float4 *>(qks[b0 + i])[l] = qk[i];
+                exs[b0 + i][l] = ex[i];
+            }
         }
+        __syncthreads();
+        const int te = min(kScanStage, T - c0);
+        for (int b = 0; b < te; b++) {
+            const float beta = exs[b][C], decay = exs[b][C + 1], v = exs[b][jl];
+            float kr[R], qr[R];
 #pragma unroll
-        for (int i = 0; i < kScanFewRows / 2; i++) {
-            reinterpret_cast<float4 *>(qks[b0 + i])[l] = qk[i];
-            exs[b0 + i][l] = ex[i];
+            for (int r = 0; r < R; r += 4) {
+                const float4 k4 = *reinterpret_cast<const float4 *>(&qks[b][kDk + R * rgp + r]);
+                const float4 q4 = *reinterpret_cast<const float4 *>(&qks[b][R * rgp + r]);
+                kr[r] = k4.x, kr[r + 1] = k4.y, kr[r + 2] = k4.z, kr[r + 3] = k4.w;
+                qr[r] = q4.x, qr[r + 1] = q4.y, qr[r + 2] = q4.z, qr[r + 3] = q4.w;
+            }
+            // S' = decay S; sk_j = sum_i S'_ij k_i
+            float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                st[r] *= decay;
+                p[r & 3] += st[r] * kr[r];
+            }
+            const float sk = row_sum16((p[0] + p[1]) + (p[2] + p[3]));
+            const float delta = beta * (v - sk);
+            // S'' = S' + k delta^T; o_j = sum_i S''_ij q_i
+#pragma unroll
+            for (int r = 0; r < 4; r++) p[r] = 0.f;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                st[r] += kr[r] * delta;
+                p[r & 3] += st[r] * qr[r];
+            }
+            const float o = row_sum16((p[0] + p[1]) + (p[2] + p[3]));
+            // lanes of row group 0 store (the others' offset is past the buffer: dropped)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), orsrc,
+                                                  rgp == 0 ? 4 * ((c0 + b) * chunk + h * kDk + j) : kDropOffset, 0, 0);
         }
-    }
-    __syncthreads();
-    for (int b = 0; b < T; b++) {
-        const float beta = exs[b][C], decay = exs[b][C + 1], v = exs[b][jl];
-        float kr[R], qr[R];
-#pragma unroll
-        for (int r = 0; r < R; r += 4) {
-            const float4 k4 = *reinterpret_cast<const float4 *>(&qks[b][kDk + R * rgp + r]);
-            const float4 q4 = *reinterpret_cast<const float4 *>(&qks[b][R * rgp + r]);
-            kr[r] = k4.x, kr[r + 1] = k4.y, kr[r + 2] = k4.z, kr[r + 3] = k4.w;
-            qr[r] = q4.x, qr[r + 1] = q4.y, qr[r + 2] = q4.z, qr[r + 3] = q4.w;
-        }
-        // S' = decay S; sk_j = sum_i S'_ij k_i
-        float p[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            st[r] *= decay;
-            p[r & 3] += st[r] * kr[r];
-        }
-        const float sk = row_sum16((p[0] + p[1]) + (p[2] + p[3]));
-        const float delta = beta * (v - sk);
-        // S'' = S' + k delta^T; o_j = sum_i S''_ij q_i
-#pragma unroll
-        for (int r = 0; r < 4; r++) p[r] = 0.f;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            st[r] += kr[r] * delta;
-            p[r & 3] += st[r] * qr[r];
-        }
-        const float o = row_sum16((p[0] + p[1]) + (p[2] + p[3]));
-        // lanes of row group 0 store (the others' offset is past the buffer: dropped)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), orsrc,
-                                              rgp == 0 ? 4 * (b * chunk + h * kDk + j) : kDropOffset, 0, 0);
     }
 #pragma unroll
     for (int r = 0; r < R; r++) Sh[(size_t)(R * rgp + r) * kDk] = st[r];

@@ -535,13 +535,14 @@ def test_prefill_long_prompt_large_cache(mid_host, n):
     oseq.close()
 
 
-@pytest.mark.parametrize("n", [2, 32, 33, 48, 49, 63, 64, 65, 129])
+@pytest.mark.parametrize("n", [2, 32, 33, 48, 49, 63, 64, 65, 128, 129, 144, 145, 176, 177, 191, 192, 193])
 def test_prefill_scan_chunk_edges(mid_host, n):
-    """Prompts around the DeltaNet scan's 64-token chunks (two tokens, fewer
-    than the conv window; the last prompt scanned token by token and the first
-    that is not; a chunk of three and of four 16-token tiles; one short of a chunk, one chunk, one token over; two
-    and one), from a state that three decode steps left, vs the oracle run
-    token by token: logits, states, conv windows, then a decode step."""
+    """Prompts around the DeltaNet scans' edges: two tokens (fewer than the
+    conv window); up to 128 scanned token by token, 32 staged at a time; from
+    129 on in 64-token chunks, the last of one token, of one, two, three and
+    four 16-token tiles, one token short of a chunk and a whole one.  From a
+    state that three decode steps left, vs the oracle run token by token:
+    logits, states, conv windows, then a decode step."""
     spec = mid_host.spec
     gm = _model(mid_host, 1, 256)
     oseq = mid_host.seq(256)
