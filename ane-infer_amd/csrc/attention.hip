@@ -102,8 +102,8 @@ __device__ __forceinline__ int wave_scan(int v) {
 __device__ __forceinline__ uint32_t plan_pos(const uint32_t *__restrict__ pos_arr, int batch) {
     return pos_arr[min((int)threadIdx.x & 63, batch - 1)];
 }
-__device__ __forceinline__ AttnPlan attn_plan(uint32_t pos, int batch, int n_kv, int W, int max_tiles) {
-    const int lane = threadIdx.x & 63;
+__device__ __forceinline__ AttnPlan attn_plan(uint32_t pos, int batch, int n_kv, int nch, int max_tiles) {
+    const int lane = threadIdx.x & 63, W = batch * n_kv * nch;
     AttnPlan P;
     P.pos = (int)pos;
     P.tiles = min(P.pos / kCh + 1, max_tiles);
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(
     int tb = 0, te = 0;  // tiles [tb, te)
     bool shared_out = false;
     if constexpr (PLAN) {
-        const AttnPlan P = attn_plan(lane_pos, batch, n_kv, batch * n_kv * nch, (max_seq + kCh - 1) / kCh);
+        const AttnPlan P = attn_plan(lane_pos, batch, n_kv, nch, (max_seq + kCh - 1) / kCh);
         if (!P.even) {
             shared_out = true;
             b = 63 - __builtin_clzll(__ballot(P.start <= slot0 && lane < batch));
@@ -504,22 +504,26 @@ __global__ __launch_bounds__(64) void attn_append_kernel(MixIn mix, const float 
 // dims 4l..4l+3 of chunks g, g + GR, g + 2 GR, ...; merges them with a
 // log-sum-exp rescale against the maximum over all chunks, adds the GR groups
 // through LDS, normalises and multiplies by sigmoid(gate) (deltanet.rs:667-669).
-// GR = 16 where a head has more than kManyChunks chunks (up to 8 per group, all
-// loaded at once; with 4 groups of 32 chunks one after the other batch 1 at 32k
-// positions took 14.6 us; a step there 30.6 -> 22.5), 4 else: every 16 chunks
-// past the first 16 cost those ~1.5 us, the larger workgroup ~3 (20 chunks of 2
-// sequences 6.8 us traced, against 4.0).
-constexpr int kManyChunks = 48;
+// GR = 16 where a head has more than kManyChunks chunks, 8 above kSomeChunks (up
+// to 8 per group, all loaded at once; with 4 groups of 32 chunks one after the
+// other batch 1 at 32k positions took 14.6 us; a step there 30.6 -> 22.5), 4
+// else: every 16 chunks past the first 16 cost those ~1.5 us, a workgroup of 16
+// groups ~3 (20 chunks of 2 sequences 6.8 us traced, against 4.0).  Steps of 2
+// sequences, 4 heads on 2 kv heads, capacity 3300 (52 chunks), 4 / 8 / 16 groups:
+// 1.2k and 2.3k positions 11.1 / 11.2 / 11.8 us, 1.8k and 3.0k 11.7 / 11.4 / 11.9.
+constexpr int kSomeChunks = 32, kManyChunks = 64;
+constexpr int kMaxChunks = 128;  // the most chunk_count() gives; a plan may give a head more
 // out: [batch][n_heads * 256] fp32, or range-safe fragment-order planes xp
-// (Planes) when xp.hi is not null.  PLAN: the partials of a launch of plan_w
-// workgroups that attn_plan() may have shared out.
+// (Planes) when xp.hi is not null.  PLAN: the partials of a launch whose
+// workgroups attn_plan() may have shared out.
 template <int G, int GR, bool PLAN>
 __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const uint32_t *__restrict__ pos_arr,
                                                                const float *__restrict__ part_o,
                                                                const float *__restrict__ part_ml, int nch,
                                                                int n_heads, int n_kv, float *__restrict__ out,
-                                                               Planes xp, int plan_w, int max_seq) {
-    constexpr int PRE = GR == 16 ? 8 : 4;  // chunks of a group loaded before the maximum is known
+                                                               Planes xp, int max_seq) {
+    constexpr int PRE = GR >= 8 ? 8 : 4;  // chunks of a group loaded before the maximum is known
+    constexpr bool MORE = PLAN || GR * PRE < kMaxChunks;
     __shared__ float red[GR];
     __shared__ float4 accs[GR][64];
     __shared__ float dens[GR][64];
@@ -539,7 +543,7 @@ __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const 
         for (int q = 0; q < 8; q++) gq[q] = *reinterpret_cast<const float4 *>(g0 + (size_t)min(q, mix.kp - 1) * mix.split);
     }
     if constexpr (PLAN) {
-        const AttnPlan P = attn_plan(lane_pos, (int)gridDim.y, n_kv, plan_w, (max_seq + kCh - 1) / kCh);
+        const AttnPlan P = attn_plan(lane_pos, (int)gridDim.y, n_kv, nch, (max_seq + kCh - 1) / kCh);
         if (P.even) {
             nc = active_chunks(__builtin_amdgcn_readlane(P.pos, b) + 1, nch);
         } else {
@@ -570,14 +574,15 @@ __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const 
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < PRE; i++) mx = g + GR * i < nc ? fmaxf(mx, pm[i]) : mx;
-    for (int c2 = g + GR * PRE; c2 < nc; c2 += GR) mx = fmaxf(mx, part_ml[((base + c2) * G + hh) * 2]);
+    for (int c2 = g + GR * PRE; MORE && c2 < nc; c2 += GR) mx = fmaxf(mx, part_ml[((base + c2) * G + hh) * 2]);
     if (l == 0) red[g] = mx;
     __syncthreads();
     float M = red[0];
 #pragma unroll
     for (int k = 1; k < GR; k++) M = fmaxf(M, red[k]);
     // this group's chunks in order: those loaded above, then 4 per trip with
-    // their loads issued together
+    // their loads issued together (selects, not branches, on what is past the
+    // last chunk: the compiler moves a load into the branch that uses it)
     float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
     float den = 0.f;
 #pragma unroll
@@ -588,7 +593,7 @@ __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const 
             den += w * pl[i];
         }
     }
-    for (int cc = g + GR * PRE; cc < nc; cc += 4 * GR) {
+    for (int cc = g + GR * PRE; MORE && cc < nc; cc += 4 * GR) {
         float4 o4[4];
         float m4[4], l4[4];
 #pragma unroll
@@ -600,10 +605,11 @@ __global__ __launch_bounds__(64 * GR) void attn_combine_kernel(MixIn mix, const 
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            if (cc + GR * i >= nc) break;
+            const bool in = cc + GR * i < nc;
             const float w = expf(m4[i] - M);
-            num = make_float4(num.x + w * o4[i].x, num.y + w * o4[i].y, num.z + w * o4[i].z, num.w + w * o4[i].w);
-            den += w * l4[i];
+            num = make_float4(num.x + (in ? w * o4[i].x : 0.0f), num.y + (in ? w * o4[i].y : 0.0f),
+                              num.z + (in ? w * o4[i].z : 0.0f), num.w + (in ? w * o4[i].w : 0.0f));
+            den += in ? w * l4[i] : 0.0f;
         }
     }
     accs[g][l] = num;
@@ -931,7 +937,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_prefill_kernel(
 int chunk_count(int max_seq, int batch, int n_kv) {
     const int tiles = (max_seq + kCh - 1) / kCh;
     const int fill = std::max(1, kAttnWorkgroups / std::max(1, batch * n_kv));
-    return std::max(1, std::min(std::min(tiles, 128), fill));
+    return std::max(1, std::min(std::min(tiles, kMaxChunks), fill));
 }
 
 }  // namespace
@@ -962,15 +968,13 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
     // without a use for it (20.0 against 19.4 us at batch 32, 5 tiles a chunk)
     const bool plan = row_stride && batch >= 2 && batch <= kMaxPlanBatch && nch >= 2 &&
                       (max_seq + kCh - 1) / kCh >= kPlanTiles * nch;
-    const int W = batch * n_kv * nch;
-    const bool many = nch > kManyChunks;  // chunks per head, with a plan on average
 #define ANEHIP_ATTN_PART(GG, NT, PLAN)                                                                          \
     hipLaunchKernelGGL((attn_partial_kernel<GG, NT, PLAN>), g1, dim3(kThreads), 0, stream, mix, q_norm, k_norm, \
                        inv_freq, pos, k_cache, v_cache, max_seq, n_heads, n_kv, part_o, part_ml, cache_off,     \
                        row_stride, append, batch)
 #define ANEHIP_ATTN_COMBINE(GG, GR, PLAN)                                                                       \
     hipLaunchKernelGGL((attn_combine_kernel<GG, GR, PLAN>), g2, dim3(64 * GR), 0, stream, mix, pos, part_o,     \
-                       part_ml, nch, n_heads, n_kv, out, xp, W, max_seq)
+                       part_ml, nch, n_heads, n_kv, out, xp, max_seq)
 #define ANEHIP_ATTN_CASE(GG)                                                                                    \
     case GG:                                                                                                    \
         if (nt && plan) ANEHIP_ATTN_PART(GG, true, true);                                                       \
@@ -979,8 +983,10 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
         else ANEHIP_ATTN_PART(GG, false, false);                                                                \
         ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                            \
         if (!out && !xp.hi) return ANEHIP_OK; /* partials only */                                               \
-        if (many && plan) ANEHIP_ATTN_COMBINE(GG, 16, true);                                                    \
-        else if (many) ANEHIP_ATTN_COMBINE(GG, 16, false);                                                      \
+        if (nch > kManyChunks && plan) ANEHIP_ATTN_COMBINE(GG, 16, true);                                       \
+        else if (nch > kManyChunks) ANEHIP_ATTN_COMBINE(GG, 16, false);                                         \
+        else if (nch > kSomeChunks && plan) ANEHIP_ATTN_COMBINE(GG, 8, true);                                   \
+        else if (nch > kSomeChunks) ANEHIP_ATTN_COMBINE(GG, 8, false);                                          \
         else if (plan) ANEHIP_ATTN_COMBINE(GG, 4, true);                                                        \
         else ANEHIP_ATTN_COMBINE(GG, 4, false);                                                                 \
         ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                            \
