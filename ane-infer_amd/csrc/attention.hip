@@ -78,9 +78,10 @@ constexpr size_t kNtKvBytes = (size_t)32 << 20;
 // sequence fixed by the batch alone, the longest sequence's set the time:
 // batch 32, 2 kv heads, lengths spread over 2k-8k: 77 us a step against 65.)
 // Lane b of each wave holds sequence b's chunks per kv head (n) and its first
-// workgroup (start): kv head k's chunk c is workgroup start + k n + c.  With as
-// many tiles in every sequence the fixed split stands (even), and costs the
-// kernels no more than the positions' load.
+// workgroup (start): kv head k's chunk c is workgroup start + k n + c.  Where
+// that takes no tile off the longest chunk the fixed split stands (even): two
+// sequences of 24.5k and 24.2k positions, 4 kv heads, 41.1 us a step with the
+// plan all the same, 39.7 without, 39.0 by kernels that have none.
 struct AttnPlan {
     int pos, tiles, n, start;
     bool even;
@@ -112,8 +113,11 @@ __device__ __forceinline__ AttnPlan attn_plan(uint32_t pos, int batch, int n_kv,
     if (P.even) return P;
     if (lane >= batch) P.tiles = 0;
     const int total = __builtin_amdgcn_readlane(wave_scan(P.tiles), 63) * n_kv;
+    int s = (total + W - 1) / W;
+    P.even = __ballot(P.tiles > s * nch) == 0;
+    if (P.even) return P;
     // ends at s = max_tiles at the latest: one chunk each, and batch x n_kv <= W
-    for (int s = (total + W - 1) / W;; s += 1 + s / 32) {
+    for (;; s += 1 + s / 32) {
         P.n = (P.tiles + s - 1) / s;
         const int end = wave_scan(P.n * n_kv);
         P.start = end - P.n * n_kv;
@@ -965,7 +969,8 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
     const bool nt = (size_t)(row_stride ? batch : 1) * n_kv * max_seq * 2 * kHd * sizeof(__half) >= kNtKvBytes;
     // sequences of their own, at least two workgroups each to share out, and
     // chunks that can grow to kPlanTiles tiles: equal lengths pay the plan
-    // without a use for it (20.0 against 19.4 us at batch 32, 5 tiles a chunk)
+    // without a use for it (20.0 against 19.4 us at batch 32, 5 tiles a chunk).
+    // Their caches hold 80 MiB and more, so that plans come with nt.
     const bool plan = row_stride && batch >= 2 && batch <= kMaxPlanBatch && nch >= 2 &&
                       (max_seq + kCh - 1) / kCh >= kPlanTiles * nch;
 #define ANEHIP_ATTN_PART(GG, NT, PLAN)                                                                          \
@@ -977,9 +982,8 @@ int attention_impl(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads, 
                        part_ml, nch, n_heads, n_kv, out, xp, max_seq)
 #define ANEHIP_ATTN_CASE(GG)                                                                                    \
     case GG:                                                                                                    \
-        if (nt && plan) ANEHIP_ATTN_PART(GG, true, true);                                                       \
+        if (plan) ANEHIP_ATTN_PART(GG, true, true);                                                             \
         else if (nt) ANEHIP_ATTN_PART(GG, true, false);                                                         \
-        else if (plan) ANEHIP_ATTN_PART(GG, false, true);                                                       \
         else ANEHIP_ATTN_PART(GG, false, false);                                                                \
         ANEHIP_HIP_TRY(ctx->err, hipGetLastError());                                                            \
         if (!out && !xp.hi) return ANEHIP_OK; /* partials only */                                               \

@@ -190,15 +190,44 @@ def test_attention_live_length_split(gpu_ctx, oracle_lib):
     _attn_case(gpu_ctx, oracle_lib, 8, 8, 2, 8192, [0, 63, 64, 700, 4095, 5000, 8000, 8191], seed=77, tol=5e-4)
 
 
+def _attn_split(n_kv, max_seq, positions):
+    """How attention_step splits a launch: (chunks per head, whether the plan
+    kernels run, whether the plan shares the workgroups out by length)."""
+    batch, cap = len(positions), -(-max_seq // 64)
+    nch = max(1, min(cap, 128, max(1, 256 // (batch * n_kv))))
+    plan = 2 <= batch <= 64 and nch >= 2 and cap >= 8 * nch
+    tiles = [p // 64 + 1 for p in positions]
+    s = -(-sum(tiles) * n_kv // (batch * n_kv * nch))
+    return nch, plan, plan and max(tiles) > s * nch
+
+
 @pytest.mark.parametrize("n_heads,n_kv,max_seq,positions", [
     (8, 2, 4096, [4095, 0]), (4, 4, 2048, [5, 2047, 64]), (2, 1, 640, [639] + 5 * [0]),
     (4, 1, 1000, [17 * i % 1000 for i in range(33)]), (2, 2, 700, [(37 * i) % 700 for i in range(64)]),
     (2, 2, 130, [i for i in range(65)]), (4, 2, 300, 3 * [255])])
-def test_attention_shared_out_workgroups(gpu_ctx, oracle_lib, n_heads, n_kv, max_seq, positions):
-    """Launches whose workgroups are shared out by length (batch 2 to 64, at
-    least two per sequence and kv head): one long sequence beside empty ones,
-    more chunks for one head than the combine loads at once, batches that do
-    not divide the workgroups, equal lengths; batch 65 keeps the fixed split."""
+def test_attention_fixed_split(gpu_ctx, oracle_lib, n_heads, n_kv, max_seq, positions):
+    """Ragged batches whose capacity is below 8 tiles a chunk (or of 65
+    sequences), so every sequence has the same number of chunks: one long
+    sequence beside empty ones, more chunks for one head than the combine's 4
+    groups load at once (and 8 groups at 33 and more), equal lengths."""
+    assert not _attn_split(n_kv, max_seq, positions)[1]
+    _attn_case(gpu_ctx, oracle_lib, len(positions), n_heads, n_kv, max_seq, positions, seed=max_seq + len(positions), tol=5e-4)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,max_seq,positions,shared", [
+    (2, 2, 1024, [(37 * i) % 1024 for i in range(64)], True), (4, 1, 3584, [(1117 * i) % 3584 for i in range(33)], True),
+    (4, 2, 2048, [(613 * i + 77) % 2048 for i in range(32)], True), (4, 2, 2048, 32 * [1300], False),
+    (2, 1, 21504, [21503] + 5 * [0], True), (8, 2, 32768, [32767, 0], True), (2, 1, 65536, [60000, 9000], True),
+    (4, 4, 16384, [12100, 12000], False), (8, 2, 8192, [0, 63, 64, 700, 4095, 5000, 8000, 8191], True)])
+def test_attention_shared_out_workgroups(gpu_ctx, oracle_lib, n_heads, n_kv, max_seq, positions, shared):
+    """Launches that may share their workgroups out by length (2 to 64
+    sequences, at least two chunks each, a capacity of 8 tiles a chunk), at 1, 2
+    and 4 query heads per kv head and with 4, 8 and 16 merge groups: a sequence
+    in every lane, batches that do not divide the workgroups, one long sequence
+    beside empty ones, more chunks for one head than the merge loads at once;
+    and lengths that gain nothing, which keep the fixed split."""
+    nch, plan, out = _attn_split(n_kv, max_seq, positions)
+    assert plan and out == shared
     _attn_case(gpu_ctx, oracle_lib, len(positions), n_heads, n_kv, max_seq, positions, seed=max_seq + len(positions), tol=5e-4)
 
 
