@@ -374,11 +374,15 @@ int launch_chunk(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const 
 // rounds of workgroups (one per CU) at 3.5 us + 3.5 us per panel (measured:
 // 31.4 us for 8 panels, 45-47 for 12), the traffic of the extra partial
 // slices (written here, read by the consumer: 2 x 4 bytes per row and output
-// at ~5 TB/s), and a launch that adds them.
+// at ~2 TB/s), and a launch that adds them.  Over 190 products of 1024..16384
+// x 1024..8192 at 33-960 rows, every split timed, the one chosen costs 0.1 % more
+// than the best on average and 5 % at most (5 TB/s and 3 us for the launch: 1.2 %
+// and 16 %; 4096 x 2048 at 128 rows 8 splits 26.9 us, 4 24.2; 6144 x 1024 at 256
+// 2 splits 26.9, 1 23.2).
 int gemm_chunk_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t rows) {
     const int nsb = (int)(n / 256), cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const int wgs = (int)((m + kTileRows - 1) / kTileRows) * (int)((rows + kRowBlock - 1) / kRowBlock);
-    const double fixed_us = 3.5, panel_us = 3.5, sum_us = 3.0, part_us = 8.0 / 5.0e6 * (double)rows * m;
+    const double fixed_us = 3.5, panel_us = 3.5, sum_us = 4.0, part_us = 8.0 / 2.0e6 * (double)rows * m;
     int best = 1;
     double best_cost = -1.0;
     for (int k = 1; k <= nsb && k <= 16; k++) {
