@@ -49,8 +49,22 @@ __device__ __forceinline__ void rmsnorm_row(const float *x, const float *__restr
         for (int i = threadIdx.x; i < n; i += kThreads) out[i] = (x[i] * inv_rms) * w[i];
         return;
     }
-    for (int i = threadIdx.x; i < n; i += kThreads)
-        atomicMax(&gmax[xp.uniform ? 0 : i / kXeGroup], __float_as_int(fabsf((x[i] * inv_rms) * w[i])));
+    if (xp.uniform) {
+        // one exponent for the row: each wave's maximum, then one update per wave
+        // (embedding norm of 256 / 960 rows of 2304: 12.4 / 18.0 us, with the one word
+        // updated per element 13.9 / 23.0; a word per group 12.3 at 256)
+        float top = 0.0f;
+#pragma unroll 4
+        for (int i = threadIdx.x; i < n; i += kThreads) {
+            const float a = fabsf((x[i] * inv_rms) * w[i]);
+            top = a <= 3.402823466e38f ? fmaxf(top, a) : INFINITY;  // a NaN stays: no exponent
+        }
+        top = wave_max64(top);
+        if ((threadIdx.x & 63) == 0) atomicMax(&gmax[0], __float_as_int(top));
+    } else {
+        for (int i = threadIdx.x; i < n; i += kThreads)
+            atomicMax(&gmax[i / kXeGroup], __float_as_int(fabsf((x[i] * inv_rms) * w[i])));
+    }
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += kThreads) {
         const float v = (x[i] * inv_rms) * w[i];

@@ -589,6 +589,23 @@ def test_prefill_attention_groups(n_heads, n_kv, n):
     oseq.close()
 
 
+def test_prefill_wide_model():
+    """A 40-token prompt of a model 2304 wide: residual norms past 2048 columns
+    into planes of one exponent per row.  Vs the oracle run token by token."""
+    host = HostModel(anehip.Spec(**WIDE), seed=9)
+    gm = _model(host, 1, 64)
+    oseq = host.seq(64)
+    toks = oracle.randint(40, 1, 41, host.spec.vocab_size)
+    g = gm.prefill(0, toks[:40])
+    for t in toks[:40]:
+        r = oseq.forward(int(t))
+    assert max(rel_errs(g, r)) <= TOL
+    _check_state(gm, oseq, 0, host.spec, "after prefill")
+    assert max(rel_errs(gm.step([int(toks[40])])[0], oseq.forward(int(toks[40])))) <= TOL
+    gm.close()
+    oseq.close()
+
+
 def _prefill_past_nan(spec, n, at):
     """Prefills n tokens whose token `at` has NaN for its embedding.  Returns
     the model and an oracle sequence run over the tokens before it."""
