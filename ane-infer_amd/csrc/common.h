@@ -191,13 +191,13 @@ struct MixIn {
 
 // gemv.hip.  y[b][r] = W[r] . x[b].  launch_quant_gemm writes final values;
 // launch_gemm_raw writes part[ks][batch][m] for ks < ksplit (final values when
-// ksplit == 1), with ksplit from gemm_ksplit().
+// ksplit == 1), with ksplit from gemm_raw_ksplit().
 int launch_quant_gemm(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w,
                       uint32_t m, uint32_t n, const float *x, uint32_t batch, float *y);
-// Number of K splits for an [m x n] product: split ks covers super-blocks
-// [ks * per, min(nsb, (ks + 1) * per)) with per = split_len(nsb, ksplit);
-// max_k bounds the splits a consumer has to add (fused consumers take 8).
-int gemm_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, int max_k = 8);
+// Number of K splits of launch_gemm_raw's [m x n] product: split ks covers
+// super-blocks [ks * per, min(nsb, (ks + 1) * per)) with per = split_len(nsb,
+// ksplit) at batch 1; above, where no other number of splits is taken, per = 8.
+int gemm_raw_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t batch);
 inline int split_len(int nsb, int ksplit) { return (nsb + ksplit - 1) / ksplit; }
 // xsplit: device scratch of batch * n floats (x split into fp16 hi / lo
 // planes for the MFMA path); may be null up to batch 16.

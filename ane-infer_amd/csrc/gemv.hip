@@ -2946,9 +2946,12 @@ static int packed_ksplit(int tiles, int nsb, int want) {
     return best;
 }
 
-int gemm_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, int max_k) {
+int gemm_raw_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t batch) {
+    if (batch > 1) return (int)((n / 256 + 7) / 8);
     const int tiles = (int)((m + kWave - 1) / kWave);
-    return choose_ksplit(tiles, (int)(n / 256), ctx->cu_count > 0 ? ctx->cu_count : 256, max_k);
+    // launch_sum_partials takes any number of splits, so the batch-1 kernel
+    // never needs more than kMaxSliceSb super-blocks per split
+    return choose_ksplit(tiles, (int)(n / 256), ctx->cu_count > 0 ? ctx->cu_count : 256, 1 << 20);
 }
 
 int gemv_packed_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, int mode) {
@@ -3445,6 +3448,8 @@ int launch_gemm_raw(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, con
                     const float *x, uint32_t batch, float *out, int ksplit, void *xsplit) {
     _Float16 *xs = static_cast<_Float16 *>(xsplit);
     if (batch > 16 && !xs) return set_error(ctx->err, ANEHIP_EINVAL, "gemm: batch > 16 needs an x split buffer");
+    if (batch > 1 && ksplit != gemm_raw_ksplit(ctx, m, n, batch))
+        return set_error(ctx->err, ANEHIP_EINVAL, "gemm: %d K splits of %u columns at batch %u", ksplit, n, batch);
     if (ggml_type == ANEHIP_GGML_Q8_0)
         return dispatch_raw<ANEHIP_GGML_Q8_0>(ctx, stream, w, m, n, x, batch, out, ksplit, xs);
     return dispatch_raw<ANEHIP_GGML_Q4_0>(ctx, stream, w, m, n, x, batch, out, ksplit, xs);
@@ -3473,9 +3478,7 @@ int launch_sum_partials(anehip_ctx *ctx, hipStream_t stream, const float *part, 
 
 int launch_quant_gemm(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w, uint32_t m,
                       uint32_t n, const float *x, uint32_t batch, float *y) {
-    // the sum_partials consumer takes any number of splits, so the batch-1
-    // kernel never needs more than kMaxSliceSb super-blocks per split
-    const int ksplit = batch == 1 ? gemm_ksplit(ctx, m, n, 1 << 20) : (int)((n / 256 + 7) / 8);
+    const int ksplit = gemm_raw_ksplit(ctx, m, n, batch);
     const size_t count = (size_t)batch * m;
     // workspace: [ksplit partials][x hi/lo planes (2 * batch * n halves)][group exponents]
     const size_t part = ksplit > 1 ? ((size_t)ksplit * count + 3) & ~(size_t)3 : 0;
