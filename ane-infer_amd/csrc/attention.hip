@@ -1028,10 +1028,10 @@ int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int 
     // to set up (16 rows from position 0: 8.8 + 4.1 us with its merge, against
     // 23.8 + 4.6 with the planes' launch); above, both sides' launches are those
     // of the uniform planes, and 33 rows of a 4-layer model take 535 us against 659
-    const bool few = rows <= kPrefillFewRows && !xp.uniform;
+    const bool few = !xp.uniform;
     uint32_t *odd = reinterpret_cast<uint32_t *>(part);  // [n_kv][rows]
-    if (!few && rows > kPrefillFewRows * (kHd + 2))
-        return set_error(ctx->err, ANEHIP_EINVAL, "attention: %d rows", rows);
+    if (rows > (few ? kPrefillFewRows : kPrefillFewRows * (kHd + 2)))
+        return set_error(ctx->err, ANEHIP_EINVAL, "attention: %d rows into %s planes", rows, few ? "grouped" : "uniform");
     hipLaunchKernelGGL(attn_append_kernel, dim3(n_kv, rows), dim3(64), 0, stream, mix, k_norm, inv_freq, pos, k_cache,
                        v_cache, cache_off, max_seq, n_heads, n_kv, few ? nullptr : odd);
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
@@ -1049,8 +1049,7 @@ int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int 
     else return set_error(ctx->err, ANEHIP_EUNSUPPORTED, "attention: %d query heads per kv head (1, 2 or 4)", G);
 #undef ANEHIP_ATTN_PREFILL
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-    return xp.uniform ? launch_split_rows(ctx, stream, out, (uint32_t)rows, (uint32_t)(n_heads * kHd), xp)
-                      : launch_split_x(ctx, stream, out, (uint32_t)rows, (uint32_t)(n_heads * kHd), xp);
+    return launch_split_rows(ctx, stream, out, (uint32_t)rows, (uint32_t)(n_heads * kHd), xp);
 }
 
 }  // namespace anehip

@@ -271,18 +271,6 @@ struct Planes {
     // value, and to 2^-39 of that below -- what a GEMM that brings the
     // groups of a row to one exponent is left with.)
     bool uniform = false;
-    // the planes of rows 32 g .. 32 g + 31 for an n-column input
-    __host__ __device__ Planes group(int g, int n) const {
-        Planes p;
-        p.hi = hi ? hi + (size_t)g * xf_plane_len((size_t)n) : nullptr;
-        p.lo = lo ? lo + (size_t)g * xf_plane_len((size_t)n) : nullptr;
-        p.xe = xe ? xe + (size_t)g * 32 * xe_stride(n) : nullptr;
-        p.rs = rs ? rs + (size_t)g * 32 * rs_parts : nullptr;
-        p.rs_parts = rs_parts;
-        p.rs_eps = rs_eps;
-        p.uniform = uniform;
-        return p;
-    }
     Planes without_scale() const {
         Planes p = *this;
         p.rs = nullptr;
@@ -339,8 +327,6 @@ __device__ __forceinline__ float dpp_add(float v) {
     return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf,
                                                                      false));
 }
-// sum over each group of 8 lanes: quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror
-__device__ __forceinline__ float sum8(float v) { return dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v))); }
 // sum over each 16-lane row: row_ror 8, 4, 2, 1
 __device__ __forceinline__ float row_sum16(float v) {
     return dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(v))));
@@ -431,8 +417,8 @@ int gemm_packed_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t b
 int launch_gemm_packed(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *wp, uint32_t m,
                        uint32_t n, const Planes &xp, uint32_t batch, float *out, int ksplit, size_t split_stride = 0);
 // The same for any number of rows (gemm_chunk.hip): above 32 one gemm_chunk
-// launch over the 32-row groups of the planes (Planes::group, which must be
-// uniform), writing out[ks][row][r] with a split stride of rows * m; ksplit
+// launch over the planes' 32-row groups (one after the other; the planes must
+// be uniform), writing out[ks][row][r] with a split stride of rows * m; ksplit
 // from gemm_rows_ksplit.
 int gemm_rows_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t rows);
 int launch_gemm_rows(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *wp, uint32_t m, uint32_t n,
@@ -559,10 +545,10 @@ int launch_attention(anehip_ctx *ctx, hipStream_t stream, int batch, int n_heads
 // pos[t], q / k / v in mix row t): appends every row's k / v to the cache at
 // cache_off (halves; the sequence's [kv_head][max_seq][256] block), then
 // attends row t over positions [0, pos[t]]: out [rows][n_heads * 256] fp32
-// (scratch), then its fragment-order planes.  Up to kPrefillFewRows rows into
-// planes that are not uniform run on the decode kernel instead, with part as
-// its scratch (attn_partial_floats of up to as many rows); more rows keep a
-// word per row and kv head there.
+// (scratch), then its uniform fragment-order planes; part holds a word per row
+// and kv head.  Planes that are not uniform take up to kPrefillFewRows rows, on
+// the decode kernel, with part as its scratch (attn_partial_floats of up to as
+// many rows).
 constexpr int kPrefillFewRows = 32;
 int launch_attention_prefill(anehip_ctx *ctx, hipStream_t stream, int rows, int n_heads, int n_kv, int max_seq,
                              const MixIn &mix, const float *q_norm, const float *k_norm, const float *inv_freq,
