@@ -228,7 +228,7 @@ __host__ __device__ __forceinline__ int gu_index(int f) { return 64 * (f >> 5) +
 // one step's operand with one fully contiguous 1 KiB load.  Rows past the
 // batch are never read.  More than 32 rows (the prefill's chunks) are stored
 // as consecutive 32-row planes, each xf_plane_len(n) halves: row b lies in
-// plane b / 32 at row b % 32, and each 32-row group is one GEMM's input.
+// plane b / 32 at row b % 32.
 __host__ __device__ inline size_t xf_index(int b, int c, int n) {
     return (size_t)(b >> 5) * 32 * (size_t)n +
            ((size_t)(c >> 4) * 64 + (size_t)((b & 31) + 32 * ((c >> 3) & 1))) * 8 + (size_t)(c & 7);

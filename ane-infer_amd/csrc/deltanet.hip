@@ -437,9 +437,11 @@ __global__ __launch_bounds__(kThreads) void deltanet_head_kernel(
 // token-by-token order keeps.  dn_scan_finish_kernel applies the gated RMSNorm
 // and commits the conv windows.
 //
-// What bounds it: the scan is serial in the chunks, 112 MFMAs of 32 cycles
-// per wave and chunk (1.5 us) plus two barriers; a token-by-token scan pays a
-// chain of LDS reads, FMAs and lane sums of 0.14 us per token (9 us per 64).
+// What bounds it: the scan is serial in the chunks, up to 112 MFMAs of 32 cycles
+// per wave and chunk (1.5 us) plus two barriers, and reads 144 KiB of a chunk and
+// head in every XCD that one of the head's 8 workgroups runs on (59 us for 15
+// chunks of 16 heads); a token-by-token scan pays a chain of LDS reads, FMAs and
+// lane sums of 0.14 us per token (9 us per 64).
 constexpr int kCt = 64;               // tokens per chunk
 constexpr int kRowF = kDk + 4;        // LDS row of a [64][128] matrix: 16-byte reads of 16 rows hit all banks
 constexpr int kTriF = kCt + 4;        // LDS row of a [64][64] matrix

@@ -782,10 +782,10 @@ __device__ __forceinline__ bool overlapped_ok(const GemvInput &in, int n, int le
 }
 
 // GEMV_IN_ATTN_COMBINE: head c0 / 256 of batch row 0, the decode attention's
-// merge of its chunk partials (attn_combine_kernel's arithmetic and order:
-// the maximum over the active chunks, then 4 groups of 64 lanes sum chunks
-// g, g + 4, ... with weights exp(m - M), the groups added in order, num / den
-// times sigmoid(gate)) into xs[0..256).  The gate and the first 16 chunks are
+// merge of its chunk partials (attn_combine_kernel's arithmetic, in the order
+// it has with 4 groups, up to 32 chunks: the maximum over the active chunks,
+// then 4 groups of 64 lanes sum chunks g, g + 4, ... with weights exp(m - M), the
+// groups added in order, num / den times sigmoid(gate)) into xs[0..256).  The gate and the first 16 chunks are
 // loaded before `issue` starts the weight loads; groups 4.. (threads >= 256)
 // mirror groups 0..3 for those loads, so every address stays in bounds.
 template <int KP, int NT, class Issue, class Store>

@@ -258,7 +258,7 @@ def bench_decode(anehip, steps, warmup, points=DECODE_POINTS, prefill_tokens=0, 
     lengths = [prefill_tokens] if isinstance(prefill_tokens, int) else list(prefill_tokens)
     lengths = [n for n in lengths if n]
     if lengths:
-        # anehip_prefill of one sequence from position 0 (chunks of 256 tokens),
+        # anehip_prefill of one sequence from position 0 (chunks of 960 tokens),
         # synchronous, timed on the host clock; one untimed run first
         gm.alloc_state(1, max([1024] + lengths))
         for n_tok in lengths:

@@ -199,10 +199,11 @@ def test_packed_gemm_tall(gpu_ctx, oracle_lib, t, batch, m, n):
 @pytest.mark.parametrize("n", [2304, 4096, 4352, 8192, 8448])
 @pytest.mark.parametrize("batch", [33, 35])
 def test_packed_gemm_row_split(gpu_ctx, oracle_lib, batch, n):
-    """Around the widths at which the chunk GEMM's plane split holds 1, 2 or 4
-    fragments per thread and reads the rest twice (above 8192), with 1 and 3
-    rows in its last workgroup of 4; rows scaled by 1e4 and 1e-4 in turn, so
-    that a row that took a neighbour's exponent shows."""
+    """Rows scaled by 1e4 and 1e-4 in turn, so that a row that took a
+    neighbour's exponent shows, in the plane split (a workgroup per row, 8
+    consecutive rows on one XCD: 1 and 3 rows in the last of them) and in the
+    chunk GEMM's output scale; at widths that the split holds in registers (8192
+    the widest, thread by thread full, half full or empty) and past them."""
     m = 68
     w = oracle_lib.gen_quant(8, 78, n, m, n, std=0.02)
     x = oracle_lib.normal(78, 901 + batch, batch * n).reshape(batch, n)
