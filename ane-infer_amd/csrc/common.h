@@ -189,20 +189,11 @@ struct MixIn {
 // ---- kernel launchers (all pointers are device pointers; work is queued on
 // `stream`; they return ANEHIP_OK or set ctx->err) ---------------------------
 
-// gemv.hip.  y[b][r] = W[r] . x[b].  launch_quant_gemm writes final values;
-// launch_gemm_raw writes part[ks][batch][m] for ks < ksplit (final values when
-// ksplit == 1), with ksplit from gemm_raw_ksplit().
+// gemv.hip.  y[b][r] = W[r] . x[b] over GGUF blocks, batch 1..32.
 int launch_quant_gemm(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w,
                       uint32_t m, uint32_t n, const float *x, uint32_t batch, float *y);
-// Number of K splits of launch_gemm_raw's [m x n] product: split ks covers
-// super-blocks [ks * per, min(nsb, (ks + 1) * per)) with per = split_len(nsb,
-// ksplit) at batch 1; above, where no other number of splits is taken, per = 8.
-int gemm_raw_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t batch);
+// Super-blocks of a K split: split ks covers [ks * per, min(nsb, (ks + 1) * per)).
 inline int split_len(int nsb, int ksplit) { return (nsb + ksplit - 1) / ksplit; }
-// xsplit: device scratch of batch * n floats (x split into fp16 hi / lo
-// planes for the MFMA path); may be null up to batch 16.
-int launch_gemm_raw(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w, uint32_t m,
-                    uint32_t n, const float *x, uint32_t batch, float *out, int ksplit, void *xsplit);
 int launch_sum_partials(anehip_ctx *ctx, hipStream_t stream, const float *part, float *y, size_t count,
                         int ksplit);
 // Panel layout (see gemv.hip): bytes of an [m x n] matrix, repack from GGUF

@@ -2465,33 +2465,6 @@ __global__ __launch_bounds__(256) void split_x_frag_kernel(const float *__restri
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-// fp32 x[batch][n] -> range-safe fp16 planes hi[batch][n], lo[batch][n]
-// (row-major; hi + lo = x * 2^-e per 128-column group, exponents to xe), one
-// thread per 8 consecutive columns, 16 threads per group (n % 128 == 0).
-__global__ __launch_bounds__(256) void split_x_kernel(const float *__restrict__ x, Planes xp, int batch, int n) {
-    const int g = blockIdx.x * 256 + threadIdx.x, per_row = n >> 3;
-    if (g >= batch * per_row) return;  // whole 16-thread groups leave together
-    const int b = g / per_row, c = 8 * (g % per_row);
-    const size_t o = (size_t)b * n + c;
-    const float4 v0 = *reinterpret_cast<const float4 *>(x + o), v1 = *reinterpret_cast<const float4 *>(x + o + 4);
-    const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-    float amax = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
-    const int ex = group_exp(row_max16(amax));  // a group is a 16-lane row
-    f16x8 h, l;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        _Float16 hh, ll;
-        split_scaled(v[e], ex, hh, ll);
-        h[e] = hh;
-        l[e] = ll;
-    }
-    *reinterpret_cast<f16x8 *>(xp.hi + o) = h;
-    *reinterpret_cast<f16x8 *>(xp.lo + o) = l;
-    if ((g & 15) == 0) xp.xe[xe_index(b, c, n)] = (int8_t)ex;
-}
-
 // 8 weights of one row of one block, as fp16, from the LDS tile row `wl`
 // (u32 words of the row's super-block segment): quant bytes 8g..8g+7 of block
 // `blk` (Q8_0: int8; Q4_0: element k < 16 is the low nibble of byte k, k >= 16
@@ -2528,33 +2501,34 @@ __device__ __forceinline__ float blk_scale(const uint32_t *wl, int blk) {
     return half_at(wl, blk * QTraits<T>::kBlockBytes);
 }
 
-// GEMM over GGUF blocks at batch 2..16, x-stationary: 8 waves per workgroup,
-// wave w holds the x fragments (hi + lo) of super-block ks * 8 + w in
-// registers, split from the fp32 rows by the wave itself (one exponent per
-// batch row over its super-block; the wave's sums are multiplied by 2^E, exact,
-// before the waves' are added), and the workgroup walks the row tiles (16 RS
-// rows) t = blockIdx.x, + gridDim.x, ...  Per tile each wave stages its rows x
-// 1 super-block of GGUF blocks through its own LDS slice and issues the next
-// tile's loads at once (in flight while this tile is multiplied), then the 8
-// waves' sums are added through LDS (the staging area, after a barrier).
-// grid = (workgroups per split, K splits of 8 super-blocks, the last possibly
+// GEMM over GGUF blocks at batch 2..32, x-stationary: 8 waves per workgroup, KW
+// of them along K and 8 / KW side by side.  Wave w holds the x fragments (hi + lo)
+// of super-block ks * KW + w % KW in registers, split from the fp32 rows by the
+// wave itself (one exponent per batch row over its super-block; the wave's sums
+// are multiplied by 2^E, exact, before the waves' are added), and the workgroup
+// walks the row tiles (16 RS rows for each w / KW) t = blockIdx.x, + gridDim.x,
+// ...  Per tile each wave stages its rows x 1 super-block of GGUF blocks through
+// its own LDS slice and issues the next tile's loads at once (in flight while
+// this tile is multiplied), then a tile's KW waves' sums are added through LDS (the
+// staging area, after a barrier).
+// grid = (workgroups per split, K splits of KW super-blocks, the last possibly
 // fewer, groups of 16 batch rows); out[ks * split_stride + b * m + r].
 //
 // What bounds it on few tiles: the chain x -> weights -> LDS -> fragments
 // (about 20 VALU operations per 16 x 8 weights: 4 us for a 64-row tile, two
-// waves per SIMD).  So the tile is the smallest of 64, 32, 16 rows that still
-// gives one workgroup per CU at most.  Measured (graphs of back-to-back calls,
+// waves per SIMD).  So tiles of 32 or 16 rows, rarely of 64 (xs_plan).  Measured (graphs of back-to-back calls,
 // weights rotated past the caches; before: x split into planes, 4-wave
 // workgroups over 2 K splits, their sum), Q8_0 at batch 8 / 32:
-//   2048 x 2048 6.3 / 7.7 us (12.8 / 21.8), 6144 x 2048 7.9 / 12.2 (13.4 /
-//   22.9), 12288 x 2048 11.4 / 22.9 (16.9 / 31.3), 2048 x 6144 10.0 / 14.3
+//   2048 x 2048 6.3 / 7.7 us (12.8 / 21.8), 6144 x 2048 7.9 / 11.3 (13.4 /
+//   22.9), 12288 x 2048 10.3 / 15.5 (16.9 / 31.3), 2048 x 6144 10.0 / 14.3
 //   (13.8 / 24.0); with 64-row tiles only: 10.5, 10.8, 11.3, 13.0 at batch 8.
-template <uint32_t T, int RS>
+template <uint32_t T, int RS, int KW>
 __global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__ W, const float *__restrict__ x,
                                                      float *__restrict__ out, int m, int n, int batch,
                                                      size_t split_stride) {
     constexpr int V = QTraits<T>::kSbVec;
-    constexpr int NW = 8, R = 16 * RS;          // rows per tile
+    constexpr int NW = 8, SUB = NW / KW;
+    constexpr int R = 16 * RS;  // rows of a wave's tile, R SUB of the workgroup's
     constexpr int C = V * R, VJ = (C + kWave - 1) / kWave;  // a wave's 16-byte chunks of a tile, per lane
     constexpr int kSegWords = QTraits<T>::kSbBytes / 4;
     constexpr int RED = 4 * RS;  // sums per lane: [row group rs][element r]
@@ -2563,13 +2537,14 @@ __global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int G = gridDim.x, ks = blockIdx.y;
-    const int nsb = n >> 8, tiles = (m + R - 1) / R;
+    const int nsb = n >> 8, tiles = (m + R * SUB - 1) / (R * SUB);
+    const int kw = wave % KW, sub = wave / KW;
     x += (size_t)16 * blockIdx.z * n;
     out += (size_t)16 * blockIdx.z * m;
     batch = min(batch - 16 * (int)blockIdx.z, 16);
     const uint32_t row_bytes = (uint32_t)nsb * QTraits<T>::kSbBytes;
-    const bool on = ks * NW + wave < nsb;  // waves past the last super-block add zeros
-    const int sb = on ? ks * NW + wave : nsb - 1;
+    const bool on = ks * KW + kw < nsb;  // waves past the last super-block add zeros
+    const int sb = on ? ks * KW + kw : nsb - 1;
     const int li = lane & 15, g = lane >> 4;
     int t = blockIdx.x;
     if (t >= tiles) return;  // uniform
@@ -2591,8 +2566,8 @@ __global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__
     u32x4 regs[VJ];
     auto chunk = [&](int j) { return C % kWave ? min(j * kWave + lane, C - 1) : j * kWave + lane; };
     auto issue = [&](int tt) {
-        const int rows_left = m - tt * R;
-        const uint8_t *base = W + (size_t)tt * R * row_bytes + (size_t)sb * QTraits<T>::kSbBytes;
+        const int row0 = min((tt * SUB + sub) * R, m - 1), rows_left = m - row0;
+        const uint8_t *base = W + (size_t)row0 * row_bytes + (size_t)sb * QTraits<T>::kSbBytes;
 #pragma unroll
         for (int j = 0; j < VJ; j++) {
             const int c = chunk(j);
@@ -2661,133 +2636,18 @@ __global__ __launch_bounds__(512) void quant_gemm_xs(const uint8_t *__restrict__
             for (int r = 0; r < 4; r++) red[(wave * RED + rs * 4 + r) * kWave + lane] = ldexpf(acc[rs][r], Er[r]);
         __syncthreads();
         // outputs (tile row rs * 16 + l % 16, batch row 4 (l / 16) + r), the
-        // 8 waves added in wave order
+        // a tile's KW waves added in wave order
 #pragma unroll
-        for (int k = 0; k < (RED * kWave + 511) / 512; k++) {
+        for (int k = 0; k < (SUB * RED * kWave + 511) / 512; k++) {
             const int o = (int)threadIdx.x + 512 * k;
-            if (o >= RED * kWave) break;
-            const int idx = o >> 6, l = o & 63;
-            float s = red[idx * kWave + l];
+            if (o >= SUB * RED * kWave) break;
+            const int u = (o >> 6) / RED, idx = (o >> 6) % RED, l = o & 63;
+            const float *p = red + ((u * KW * RED) + idx) * kWave + l;
+            float s = p[0];
 #pragma unroll
-            for (int w = 1; w < NW; w++) s += red[(w * RED + idx) * kWave + l];
-            const int row = t * R + (idx >> 2) * 16 + (l & 15), b = 4 * (l >> 4) + (idx & 3);
+            for (int w = 1; w < KW; w++) s += p[w * RED * kWave];
+            const int row = (t * SUB + u) * R + (idx >> 2) * 16 + (l & 15), b = 4 * (l >> 4) + (idx & 3);
             if (row < m && b < batch) dst[(size_t)b * m + row] = s;
-        }
-        __syncthreads();  // the staging area is free again
-    }
-}
-
-// The same for batch 17..32: wave w = 4 h + q holds the x fragments of batch
-// rows 16 h .. + 15 for the two super-blocks ks * 8 + 2 q, + 1 (128
-// registers: 32 rows of one super-block would not fit beside the weights in
-// flight at two waves per SIMD) and loads segment 2 q + h of each tile; the
-// pair's two segments are shared through LDS by waves q and q + 4, and each
-// batch half's 4 waves are added per tile.  The lane's load offsets are
-// recomputed per tile (held across the loop they cost 34 registers and the
-// kernel spilled); x comes as planes (Planes, row-major), brought to one
-// exponent per batch row over the split.  lm_head 151936 x 2048 at batch 32
-// 133-134 us, against 160-166 with the x fragments reloaded for every tile.
-template <uint32_t T>
-__global__ __launch_bounds__(512) void quant_gemm_xs32(const uint8_t *__restrict__ W, Planes xp,
-                                                       float *__restrict__ out, int m, int n, int batch,
-                                                       size_t split_stride) {
-    constexpr int V = QTraits<T>::kSbVec;
-    constexpr int kSegWords = QTraits<T>::kSbBytes / 4;
-    constexpr int RED = 16;  // sums per lane: [row group rs][element r]
-    static_assert(8 * RED * kWave * 4 <= 8 * V * kWave * 16, "the reduction fits the staging area");
-    __shared__ u32x4 lds[4][2][V * kWave];
-    __shared__ int xeE[32];
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int hh = wave >> 2, q = wave & 3;
-    const int G = gridDim.x, ks = blockIdx.y;
-    const int nsb = n >> 8, tiles = (m + kWave - 1) / kWave;
-    const uint32_t row_bytes = (uint32_t)nsb * QTraits<T>::kSbBytes;
-    const int sb0 = ks * 8 + 2 * q;  // past the last super-block: its copy, multiplied by zeros
-    const int li = lane & 15, g = lane >> 4;
-    int t = blockIdx.x;
-    if (t >= tiles) return;  // uniform
-    u32x4 regs[V];
-    auto issue = [&](int tt) {
-        int ln = lane;
-        asm volatile("" : "+v"(ln));  // not loop-invariant: the offsets are not kept in registers
-        const int rows_left = m - tt * kWave;
-        const uint8_t *base = W + (size_t)tt * kWave * row_bytes + (size_t)min(sb0 + hh, nsb - 1) * QTraits<T>::kSbBytes;
-#pragma unroll
-        for (int j = 0; j < V; j++) {
-            const int c = j * kWave + ln;
-            const uint32_t o = (uint32_t)min(c / V, rows_left - 1) * row_bytes + (uint32_t)(c % V) * 16u;
-            regs[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + o));
-        }
-    };
-    issue(t);
-    h8v ah[2][8], al[2][8];
-    {
-        const int b = min(li + 16 * hh, batch - 1);
-        const int En = xe_max(xp.xe, b, 2 * ks * 8, min(16, 2 * (nsb - ks * 8)), n);
-        if (q == 0 && g == 0) xeE[li + 16 * hh] = En;
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const int sb = min(sb0 + s, nsb - 1);
-            const int8_t *e = xp.xe + (size_t)b * xe_stride(n) + 2 * sb;
-            const bool on = sb0 + s < nsb;
-            const _Float16 f0 = xe_factor(e[0], En), f1 = xe_factor(e[1], En);
-            const h8v zero = {};
-#pragma unroll
-            for (int blk = 0; blk < 8; blk++) {
-                const size_t xo = (size_t)b * n + (size_t)sb * 256 + 32 * blk + 8 * g;
-                const _Float16 f = blk < 4 ? f0 : f1;
-                ah[s][blk] = on ? *reinterpret_cast<const h8v *>(xp.hi + xo) * f : zero;
-                al[s][blk] = on ? *reinterpret_cast<const h8v *>(xp.lo + xo) * f : zero;
-            }
-        }
-    }
-    float *red = reinterpret_cast<float *>(&lds[0][0][0]);  // [wave][RED][lane], after the tile's barrier
-    float *dst = out + (size_t)ks * split_stride;
-    for (; t < tiles; t += G) {
-#pragma unroll
-        for (int j = 0; j < V; j++) lds[q][hh][j * kWave + lane] = regs[j];
-        __syncthreads();  // both segments of every pair staged
-        if (t + G < tiles) issue(t + G);
-        f32x4 acc[4];
-#pragma unroll
-        for (int rs = 0; rs < 4; rs++) acc[rs] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const uint32_t *lw = reinterpret_cast<const uint32_t *>(lds[q][s]);
-#pragma unroll
-            for (int blk = 0; blk < 8; blk++) {
-#pragma unroll
-                for (int rs = 0; rs < 4; rs++) {
-                    const uint32_t *wl = lw + (rs * 16 + li) * kSegWords;
-                    const h8v bw = (blk & 1) ? w_frag<T, 1>(wl, blk, g) : w_frag<T, 0>(wl, blk, g);
-                    const float d = blk_scale<T>(wl, blk);
-                    f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s][blk], bw, f32x4{0.f, 0.f, 0.f, 0.f}, 0,
-                                                                     0, 0);
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s][blk], bw, c, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[rs][r] = fmaf(c[r], d, acc[rs][r]);
-                    __builtin_amdgcn_sched_barrier(0);  // one weight fragment live at a time
-                }
-            }
-        }
-        __syncthreads();  // every wave is done with the staged segments
-#pragma unroll
-        for (int rs = 0; rs < 4; rs++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) red[(wave * RED + rs * 4 + r) * kWave + lane] = acc[rs][r];
-        __syncthreads();
-        // output o: batch half h = o / 1024, then (rs, r, lane); the half's 4
-        // waves added in wave order
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int o = (int)threadIdx.x + 512 * k;
-            const int h = o >> 10, idx = (o >> 6) & 15, l = o & 63;
-            float sum = red[((4 * h) * RED + idx) * kWave + l];
-#pragma unroll
-            for (int w = 1; w < 4; w++) sum += red[((4 * h + w) * RED + idx) * kWave + l];
-            const int row = t * kWave + (idx >> 2) * 16 + (l & 15), b = 16 * h + 4 * (l >> 4) + (idx & 3);
-            if (row < m && b < batch) dst[(size_t)b * m + row] = ldexpf(sum, xeE[b]);
         }
         __syncthreads();  // the staging area is free again
     }
@@ -2870,14 +2730,63 @@ int dispatch_fused(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t 
     }
 }
 
+// How the GGUF-layout GEMM of 2..32 rows runs: kw waves of a workgroup along K
+// (one super-block each), rs 16-row groups in a wave's tile, ksplit splits of kw
+// super-blocks, wgs workgroups per split and group of 16 batch rows.
+struct XsPlan {
+    int kw, rs, ksplit, wgs, groups;
+};
+// 17..32 rows are two groups of 16 side by side (the second group's weights come
+// from the L2 or the MALL: 151936 x 2048 at 32 rows 128 us, 137 on a kernel of 32
+// rows); each split and group has its share of the CUs, whose workgroups walk
+// the tiles, so that x is staged once per workgroup and the next tile's weights
+// are in flight (16384 x 8192 (4 splits) at batch 9 / 17 / 32 (Q4_0) 38 / 64 / 63
+// us, with a workgroup per tile and split 45 / 84 / 90).  rs and kw by an
+// estimate: rounds of tiles at 1.5 or 2.9 us for 16 or 32 rows (both weight
+// types), and with K splits 1.7 us and the partial slices' round trip at 2.4 TB/s.
+// 4 waves along K take twice the rows at once, which fills the waves that a K of
+// few super-blocks, or of a few more than 8 or 16, leaves idle; small tiles in
+// more rounds leave fewer CUs without one in the last.  Tiles of 64 rows (5.7 us,
+// 6 in further rounds) only where they take one round of both groups and 32 rows
+// two: 2048 x 6144 at 32 rows 14.1 us against 15.1.  Measured against 8 waves along
+// K always and tiles of 16, 32 or 64 rows by what one round covers, over 1528
+// products of 1024..150000 x 256..8192 (3, 12, 20 and 32 rows, both types):
+// 0.22-1.05 of the time.  Q8_0 at 3 rows 12288 x 2048 10.5 -> 9.2 us, 8448 x 2304 18
+// -> 12, 150000 x 1024 68 -> 35.
+XsPlan xs_plan(uint32_t m, uint32_t n, uint32_t batch, int cus) {
+    const int nsb = (int)(n / 256);
+    XsPlan best{};
+    double best_cost = -1.0;
+    for (int kw = 8; kw >= 1; kw /= 2) {
+        XsPlan P{kw, 4, (nsb + kw - 1) / kw, 1, batch <= 16 ? 1 : 2};
+        // below 4 waves only without a K split; at most the 16 slices that one
+        // pass adds, but for 8 waves
+        if ((kw < 4 && P.ksplit > 1) || (kw < 8 && P.ksplit > 16)) continue;
+        const int share = std::max(1, cus / (P.ksplit * P.groups));
+        const auto tiles = [&](int rs) { return (int)((m + 16 * rs * (8 / kw) - 1) / (16 * rs * (8 / kw))); };
+        const double slices = P.ksplit > 1 ? 1.7 + 8.0 / 2.4e6 * P.ksplit * batch * (double)m : 0.0;
+        for (P.rs = 1; P.rs <= 4; P.rs *= 2) {
+            P.wgs = std::min(tiles(P.rs), share);
+            const int rounds = (tiles(P.rs) + P.wgs - 1) / P.wgs;
+            if (P.rs == 4 && (P.groups == 1 || rounds > 1 || kw < 4)) continue;
+            const double cost = rounds * (P.rs == 1 ? 1.5 : P.rs == 2 ? 2.9 : 5.7) + slices;
+            if (best_cost < 0.0 || cost < best_cost) {
+                best_cost = cost;
+                best = P;
+            }
+        }
+    }
+    return best;
+}
+
 template <uint32_t T>
 int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m, uint32_t n, const float *x,
-                 uint32_t batch, float *out, int ksplit, _Float16 *xsplit) {
+                 uint32_t batch, float *out, int ksplit, const XsPlan &P) {
     const size_t split_stride = (size_t)batch * m;
     const int tiles = (int)((m + kWave - 1) / kWave), cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     // the x-stationary kernels: one workgroup per CU walks the row tiles with
-    // the x of its K split of 8 super-blocks staged once (batch 1, where there
-    // are at least 4 tiles per CU: as digits in LDS; batch 2..32: as MFMA
+    // the x of its K split staged once (batch 1, where there are at least 4 tiles
+    // per CU and splits of 8 super-blocks: as digits in LDS; batch 2..32: as MFMA
     // fragments in registers)
     if (batch == 1) {
         if ((int)(n / 256) == 8 * ksplit && tiles >= 4 * cus) {
@@ -2891,42 +2800,23 @@ int dispatch_raw(anehip_ctx *ctx, hipStream_t stream, const void *w, uint32_t m,
         return dispatch_fused<T>(ctx, stream, w, m, n, in, out, ksplit);
     }
     const uint8_t *wb = static_cast<const uint8_t *>(w);
-    // With several K splits (or groups) each has its share of the CUs and its
-    // workgroups walk the tiles, so that x is staged once per workgroup and
-    // the next tile's weights are in flight: 16384 x 8192 (4 splits) at batch
-    // 9 / 17 / 32 (Q4_0) 38 / 64 / 63 us, with a workgroup per tile and split 45 /
-    // 84 / 90.
-    // 17..32 rows as two groups of 16 side by side where each workgroup has
-    // one tile to do, or two (the second group's weights come from the L2 or
-    // the MALL)
-    const int groups = batch <= 16 ? 1 : 2;
-    if (batch <= 16 || tiles * ksplit <= cus) {
-        const int work = ksplit * groups;
-        auto rows_tiles = [&](int r) { return (int)((m + r - 1) / r); };
-        const int per_work = max(1, cus / work);
-#define ANEHIP_XS(RS)                                                                                       \
-    hipLaunchKernelGGL((quant_gemm_xs<T, RS>), dim3(min(rows_tiles(16 * RS), per_work), ksplit, groups), dim3(512), \
-                       0, stream, wb, x, out, (int)m, (int)n, (int)batch, split_stride)
-        if (rows_tiles(16) * work <= cus) ANEHIP_XS(1);
-        else if (rows_tiles(32) * work <= cus) ANEHIP_XS(2);
-        else ANEHIP_XS(4);
+    const dim3 grid(P.wgs, P.ksplit, P.groups);
+#define ANEHIP_XS(RS, KW)                                                                                          \
+    hipLaunchKernelGGL((quant_gemm_xs<T, RS, KW>), grid, dim3(512), 0, stream, wb, x, out, (int)m, (int)n, (int)batch, \
+                       split_stride)
+#define ANEHIP_XS_KW(KW)                 \
+    do {                                 \
+        if (P.rs == 1) ANEHIP_XS(1, KW); \
+        else ANEHIP_XS(2, KW);           \
+    } while (0)
+    if (P.rs == 4 && P.kw == 8) ANEHIP_XS(4, 8);
+    else if (P.rs == 4) ANEHIP_XS(4, 4);
+    else if (P.kw == 8) ANEHIP_XS_KW(8);
+    else if (P.kw == 4) ANEHIP_XS_KW(4);
+    else if (P.kw == 2) ANEHIP_XS_KW(2);
+    else ANEHIP_XS_KW(1);
+#undef ANEHIP_XS_KW
 #undef ANEHIP_XS
-        ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-        return ANEHIP_OK;
-    }
-    const dim3 grid(min(tiles, max(1, cus / ksplit)), ksplit);
-    // 17..32: x split into range-safe fp16 hi / lo planes (row-major) first
-    const size_t count = (size_t)batch * n;
-    Planes xp;
-    xp.hi = xsplit;
-    xp.lo = xsplit + count;
-    xp.xe = reinterpret_cast<int8_t *>(xsplit + 2 * count);
-    const size_t vecs = count / 8;
-    hipLaunchKernelGGL(split_x_kernel, dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, stream, x, xp, (int)batch,
-                       (int)n);
-    ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
-    hipLaunchKernelGGL((quant_gemm_xs32<T>), grid, dim3(512), 0, stream, wb, xp, out, (int)m, (int)n, (int)batch,
-                       split_stride);
     ANEHIP_HIP_TRY(ctx->err, hipGetLastError());
     return ANEHIP_OK;
 }
@@ -2944,14 +2834,6 @@ static int packed_ksplit(int tiles, int nsb, int want) {
         if (tiles * k >= want && per <= kMaxSliceSb) return k;
     }
     return best;
-}
-
-int gemm_raw_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, uint32_t batch) {
-    if (batch > 1) return (int)((n / 256 + 7) / 8);
-    const int tiles = (int)((m + kWave - 1) / kWave);
-    // launch_sum_partials takes any number of splits, so the batch-1 kernel
-    // never needs more than kMaxSliceSb super-blocks per split
-    return choose_ksplit(tiles, (int)(n / 256), ctx->cu_count > 0 ? ctx->cu_count : 256, 1 << 20);
 }
 
 int gemv_packed_ksplit(const anehip_ctx *ctx, uint32_t m, uint32_t n, int mode) {
@@ -3444,17 +3326,6 @@ int launch_gemv_fused(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, c
     return dispatch_fused<ANEHIP_GGML_Q4_0>(ctx, stream, w, m, n, in, out, ksplit);
 }
 
-int launch_gemm_raw(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w, uint32_t m, uint32_t n,
-                    const float *x, uint32_t batch, float *out, int ksplit, void *xsplit) {
-    _Float16 *xs = static_cast<_Float16 *>(xsplit);
-    if (batch > 16 && !xs) return set_error(ctx->err, ANEHIP_EINVAL, "gemm: batch > 16 needs an x split buffer");
-    if (batch > 1 && ksplit != gemm_raw_ksplit(ctx, m, n, batch))
-        return set_error(ctx->err, ANEHIP_EINVAL, "gemm: %d K splits of %u columns at batch %u", ksplit, n, batch);
-    if (ggml_type == ANEHIP_GGML_Q8_0)
-        return dispatch_raw<ANEHIP_GGML_Q8_0>(ctx, stream, w, m, n, x, batch, out, ksplit, xs);
-    return dispatch_raw<ANEHIP_GGML_Q4_0>(ctx, stream, w, m, n, x, batch, out, ksplit, xs);
-}
-
 int launch_sum_partials(anehip_ctx *ctx, hipStream_t stream, const float *part, float *y, size_t count, int ksplit) {
     const bool v4 = count % 4 == 0 && ksplit >= 1 && ksplit <= 16 && reinterpret_cast<uintptr_t>(part) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(y) % 16 == 0;
@@ -3478,17 +3349,23 @@ int launch_sum_partials(anehip_ctx *ctx, hipStream_t stream, const float *part, 
 
 int launch_quant_gemm(anehip_ctx *ctx, hipStream_t stream, uint32_t ggml_type, const void *w, uint32_t m,
                       uint32_t n, const float *x, uint32_t batch, float *y) {
-    const int ksplit = gemm_raw_ksplit(ctx, m, n, batch);
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const XsPlan P = batch > 1 ? xs_plan(m, n, batch, cus) : XsPlan{};
+    // (launch_sum_partials takes any number of splits, so the batch-1 kernel never
+    // needs more than kMaxSliceSb super-blocks per split)
+    const int ksplit =
+        batch > 1 ? P.ksplit : choose_ksplit((int)((m + kWave - 1) / kWave), (int)(n / 256), cus, 1 << 20);
     const size_t count = (size_t)batch * m;
-    // workspace: [ksplit partials][x hi/lo planes (2 * batch * n halves)][group exponents]
-    const size_t part = ksplit > 1 ? ((size_t)ksplit * count + 3) & ~(size_t)3 : 0;
-    const size_t xs_floats = batch > 16 ? (size_t)batch * n + (xe_bytes(n) + 3) / 4 : 0;
-    int rc = ensure_workspace(ctx, part + xs_floats);
-    if (rc) return rc;
-    void *xs = batch > 16 ? static_cast<void *>(ctx->ws.partial + part) : nullptr;
-    if (ksplit == 1) return launch_gemm_raw(ctx, stream, ggml_type, w, m, n, x, batch, y, 1, xs);
-    rc = launch_gemm_raw(ctx, stream, ggml_type, w, m, n, x, batch, ctx->ws.partial, ksplit, xs);
-    if (rc) return rc;
+    float *out = y;
+    if (ksplit > 1) {
+        const int rc = ensure_workspace(ctx, (size_t)ksplit * count);  // the splits' partial sums
+        if (rc) return rc;
+        out = ctx->ws.partial;
+    }
+    const int rc = ggml_type == ANEHIP_GGML_Q8_0
+                       ? dispatch_raw<ANEHIP_GGML_Q8_0>(ctx, stream, w, m, n, x, batch, out, ksplit, P)
+                       : dispatch_raw<ANEHIP_GGML_Q4_0>(ctx, stream, w, m, n, x, batch, out, ksplit, P);
+    if (rc || ksplit == 1) return rc;
     return launch_sum_partials(ctx, stream, ctx->ws.partial, y, count, ksplit);
 }
 

@@ -85,17 +85,7 @@ def test_small_batch_gemm_parity(gpu_ctx, oracle_lib, t, batch, m, n):
     assert l2 <= TOL and mx <= TOL
 
 
-@pytest.mark.parametrize("t", [8, 2])
-@pytest.mark.parametrize("m,n,batch", [(1, 256, 2), (17, 2304, 16), (33, 4352, 17), (4100, 2048, 9), (4113, 512, 31),
-                                       (8200, 1792, 5), (8255, 2048, 32), (16400, 256, 3), (17000, 2304, 20)])
-def test_gguf_gemm_tile_edges(gpu_ctx, oracle_lib, t, m, n, batch):
-    """The GGUF-layout GEMM's tile heights and batch groups: 16-row tiles (one
-    row; one past a tile), 32-row tiles (4100 and 4113 rows: a last tile of 4
-    and 17), 64-row tiles (8200, 8255: 8 and 63), more tiles than CUs (16400:
-    a second tile for one workgroup), super-block counts that leave waves
-    without one (1, 2, 7 of 8; 9 and 17 over 2 and 3 K splits), and 17..32
-    rows as two groups side by side or on the 32-row kernel with a short last
-    K split."""
+def _gguf_gemm_case(gpu_ctx, oracle_lib, t, m, n, batch):
     w = oracle_lib.gen_quant(t, 41, m + n + batch, m, n, std=0.02)
     x = oracle_lib.normal(41, batch, batch * n).reshape(batch, n)
     dw, dx, dy = gpu_ctx.to_device(w), gpu_ctx.to_device(x), gpu_ctx.alloc(batch * m * 4)
@@ -106,6 +96,49 @@ def test_gguf_gemm_tile_edges(gpu_ctx, oracle_lib, t, m, n, batch):
     assert l2 <= TOL and mx <= TOL
     for b in (dw, dx, dy):
         b.free()
+
+
+@pytest.mark.parametrize("t", [8, 2])
+@pytest.mark.parametrize("m,n,batch", [(1, 256, 2), (17, 2304, 16), (33, 4352, 17), (4100, 2048, 9), (4113, 512, 31),
+                                       (8200, 1792, 5), (8255, 2048, 32), (16400, 256, 3), (17000, 2304, 20)])
+def test_gguf_gemm_tile_edges(gpu_ctx, oracle_lib, t, m, n, batch):
+    """The GGUF-layout GEMM at one row, one row past a tile, ragged last tiles,
+    more tiles than CUs, super-block counts that leave waves without one (1, 2, 7
+    of 8; 9 and 17 over several K splits) and 17..32 rows as two groups."""
+    _gguf_gemm_case(gpu_ctx, oracle_lib, t, m, n, batch)
+
+
+def _gguf_tiles(m, n, batch, cus=256):
+    """(waves along K, 16-row groups per wave's tile) of the GGUF-layout GEMM."""
+    nsb, groups, best = n // 256, 1 if batch <= 16 else 2, None
+    for kw in (8, 4, 2, 1):
+        ks = -(-nsb // kw)
+        if (kw < 4 and ks > 1) or (kw < 8 and ks > 16):
+            continue
+        share = max(1, cus // (ks * groups))
+        for rs, us in ((1, 1.5), (2, 2.9), (4, 5.7)):
+            tiles = -(-m // (16 * rs * (8 // kw)))
+            rounds = -(-tiles // min(tiles, share))
+            if rs == 4 and (groups == 1 or rounds > 1 or kw < 4):
+                continue
+            cost = rounds * us + (1.7 + 8.0 / 2.4e6 * ks * batch * m if ks > 1 else 0.0)
+            if best is None or cost < best[0]:
+                best = cost, (kw, rs)
+    return best[1]
+
+
+@pytest.mark.parametrize("t", [8, 2])
+@pytest.mark.parametrize("m,n,batch,tiles", [
+    (8278, 256, 31, (1, 1)), (16441, 256, 17, (1, 2)), (4106, 256, 31, (2, 1)), (8196, 512, 31, (2, 2)), (2051, 768, 17, (4, 1)),
+    (4100, 768, 31, (4, 2)), (8449, 2304, 5, (4, 2)), (2053, 1280, 17, (8, 2)), (33000, 1280, 16, (8, 1)),
+    (20001, 4352, 2, (4, 1)), (2033, 6144, 19, (8, 4)),
+    (4108, 2304, 17, (4, 4))])
+def test_gguf_gemm_waves_along_k(gpu_ctx, oracle_lib, t, m, n, batch, tiles):
+    """1, 2, 4 and 8 waves along K with 16-, 32- and 64-row tiles: a last workgroup
+    tile in which whole waves lie past the matrix or all but one of their rows
+    do, waves without a super-block, several rounds of tiles, K splits."""
+    assert _gguf_tiles(m, n, batch) == tiles
+    _gguf_gemm_case(gpu_ctx, oracle_lib, t, m, n, batch)
 
 
 @pytest.mark.parametrize("t", [8, 2])
