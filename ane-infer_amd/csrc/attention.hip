@@ -514,7 +514,7 @@ __global__ __launch_bounds__(64) void attn_append_kernel(MixIn mix, const float 
 // else: every 16 chunks past the first 16 cost those ~1.5 us, a workgroup of 16
 // groups ~3 (20 chunks of 2 sequences 6.8 us traced, against 4.0).  Steps of 2
 // sequences, 4 heads on 2 kv heads, capacity 3300 (52 chunks), 4 / 8 / 16 groups:
-// 1.2k and 2.3k positions 11.1 / 11.2 / 11.8 us, 1.8k and 3.0k 11.7 / 11.4 / 11.9.
+// 1.2k and 2.3k positions 11.1 / 10.8 / 11.9 us, 1.8k and 3.0k 11.7 / 10.7 / 12.0.
 constexpr int kSomeChunks = 32, kManyChunks = 64;
 constexpr int kMaxChunks = 128;  // the most chunk_count() gives; a plan may give a head more
 // out: [batch][n_heads * 256] fp32, or range-safe fragment-order planes xp
